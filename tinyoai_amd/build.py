@@ -23,7 +23,7 @@ ARCH = os.environ.get("TINYOAI_OFFLOAD_ARCH", "gfx950")
 # (matvec_<format>.hip), so they compile in parallel.
 MATVEC_FORMATS = ["q8_0", "bf16", "f32", "f16", "q5_1", "q4_k", "q5_k", "q6_k"]
 SOURCES = ["decode.hip", "api.cpp", "llama.cpp", "prefill.hip", "weights.hip", "gemm.hip", "gemm_q8.hip",
-           "flash.hip", "logprobs.hip", "kq_rows.hip", "llama_tiny.hip"] + [f"matvec_{f}.hip" for f in MATVEC_FORMATS]
+           "flash.hip", "logprobs.hip", "kq_rows.hip", "few_rows.hip", "gemm_exact.hip", "llama_tiny.hip"] + [f"matvec_{f}.hip" for f in MATVEC_FORMATS]
 FLAGS = ["-O3", "-std=c++17", "-fPIC", "-x", "hip", f"--offload-arch={ARCH}", "-ffp-contract=off",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-Wall", "-Wno-unused-function", "-Wno-unused-variable", "-Wno-unused-value", "-Wno-unused-result",
@@ -37,11 +37,12 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
-# Per-source additions: the Q8_0 wide-tile kernel keeps its matrix-core
-# results in ordinary vector registers (each quant block's products are
-# rescaled on the vector unit, which cannot read the accumulation
-# registers); the BF16 kernels keep theirs in the accumulation registers.
-EXTRA = {"gemm_q8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+# Per-source additions: the Q8_0 wide-tile and the fp32-accurate kernels keep
+# their matrix-core results in ordinary vector registers (each K step's
+# products are rescaled or added on the vector unit, which cannot read the
+# accumulation registers); the BF16 kernels keep theirs in the accumulation registers.
+EXTRA = {"gemm_q8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+         "gemm_exact.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _compile(src: str) -> str:

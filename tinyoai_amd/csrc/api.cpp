@@ -136,7 +136,10 @@ int DevMatrix::create(int32_t dtype, int64_t rows, int64_t cols, hipStream_t st)
   auto round256 = [](size_t v) { return (v + 255) / 256 * 256; };
   const size_t vbytes = round256((size_t)(m.vstride * rows)), mbytes = round256((size_t)(m.mstride * rows));
   const size_t hbytes = round256((size_t)(m.hstride * rows));
-  const size_t total = vbytes + mbytes + hbytes + 256;
+  // the row scales, where the format takes them, and 256 spare bytes (the
+  // first word: finish()'s flag)
+  const size_t sbytes = dtype == FMT_F32 || is_kquant(dtype) ? round256((size_t)rows * 4) : 0;
+  const size_t total = vbytes + mbytes + hbytes + sbytes + 256;
   hipError_t e = hipMalloc(&mem, total);
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc(%zu): %s", total, hipGetErrorString(e));
   bytes = total;
@@ -217,13 +220,28 @@ int DevMatrix::place(int32_t dtype, int64_t rows, int64_t cols, const void *data
   return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "weight repack");
 }
 
+int DevMatrix::finish(hipStream_t st) {
+  MatDesc &m = desc;
+  if (m.fmt == FMT_Q8_0 || m.fmt == FMT_BF16) return TINYOAI_OK;
+  unsigned special = 0, *flag = reinterpret_cast<unsigned *>((uint8_t *)mem + bytes - 256);
+  float *scales = m.fmt == FMT_F16 ? nullptr : reinterpret_cast<float *>((uint8_t *)flag - ((size_t)m.rows * 4 + 255) / 256 * 256);
+  hipError_t e = launch_row_scales(m, scales, flag, st);
+  if (e == hipSuccess) e = hipMemcpyAsync(&special, flag, 4, hipMemcpyDeviceToHost, st);
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  if (e != hipSuccess) return hip_fail(e, "row scales");
+  m.special = special != 0;
+  m.rscale = scales;
+  return TINYOAI_OK;
+}
+
 int DevMatrix::upload(int32_t dtype, int64_t rows, int64_t cols, const void *data, uint64_t nbytes, hipStream_t st) {
   const int64_t want = gguf_bytes(dtype, rows, cols);
   if (want >= 0 && (int64_t)nbytes != want)
     return fail(TINYOAI_EINVAL, "tensor [%lld, %lld] of type %d needs %lld bytes, got %llu", (long long)rows,
                 (long long)cols, dtype, (long long)want, (unsigned long long)nbytes);
   int rc = create(dtype, rows, cols, st);
-  return rc ? rc : place(dtype, rows, cols, data, nbytes, RowMap{ROWMAP_IDENTITY, 0, 0, 0, 0}, 0, st);
+  if (!rc) rc = place(dtype, rows, cols, data, nbytes, RowMap{ROWMAP_IDENTITY, 0, 0, 0, 0}, 0, st);
+  return rc ? rc : finish(st);
 }
 
 MatDesc column_view(const MatDesc &m, int64_t col0, int64_t cols) {
@@ -460,6 +478,8 @@ int StableModel::init(const tinyoai_stablelm_config &c, const tinyoai_tensor *te
     if ((rc = place(wout, p + names[3], t[3], RowMap{ROWMAP_IDENTITY, 0, 0, 0, 0}, 0)) ||
         (rc = place(down, p + names[6], t[6], RowMap{ROWMAP_IDENTITY, 0, 0, 0, 0}, down0)))
       return rc;
+    for (DevMatrix *m : {&win, &wout, &win2, &wout2})
+      if (m->mem && (rc = m->finish(stream))) return rc;
     LayerDev &L = layers[l];
     L.win = win.desc;
     L.wout = wout.desc;
@@ -500,16 +520,17 @@ int StableModel::init(const tinyoai_stablelm_config &c, const tinyoai_tensor *te
   e = hipMemsetAsync(counters, 0, att_queries * dims.heads * 4, stream);
   if (e != hipSuccess) return hip_fail(e, "counter init");
   if ((rc = alloc((void **)&partials, att_queries * dims.heads * partial_region(max_splits, hd) * 4))) return rc;
-  const size_t B = chunk, wide = std::max(d, I);
+  const size_t B = chunk, wide = (std::max(d, I) + 31) / 32 * 32;
   if ((rc = alloc((void **)&X, B * d * 4)) || (rc = alloc((void **)&H, B * d * 4)) ||
       (rc = alloc((void **)&Y, B * win_rows * 4)) || (rc = alloc((void **)&Q, B * w_att * 4)) ||
       (rc = alloc((void **)&M, B * I * 4)) || (rc = alloc((void **)&A, B * w_att * 4)) ||
       (rc = alloc((void **)&P, kPrefillSplits * B * d * 4)) || (rc = alloc((void **)&D, kPrefillSplits * B * d * 4)) ||
-      (rc = alloc((void **)&XH, 2 * B * wide * 2)) || (rc = alloc((void **)&MH, 2 * B * I * 2)))
+      (rc = alloc((void **)&XH, 2 * B * wide * 2)) || (rc = alloc((void **)&XU, 2 * B * 4)) ||
+      (rc = alloc((void **)&MH, 2 * B * ((I + 31) / 32 * 32) * 2)))
     return rc;
   // One allocation per operand: the hi plane, then the lo plane.
   XL = XH + B * wide;
-  ML = MH + B * I;
+  ML = MH + B * ((I + 31) / 32 * 32);
   // The error word after the logits: set by a decode step whose bounded
   // in-kernel wait timed out.
   perr = (unsigned *)(logits_dev + c.vocab_size);
@@ -751,6 +772,34 @@ int StableModel::decode_step(int token, int pos, bool want_logits) {
   return TINYOAI_OK;
 }
 
+// The wide-tile shape (rows per block 128 * mf, columns 32 * nf) for an
+// n-row product with N outputs: the fewest rounds of 256 blocks weighted
+// by the tile area, the 64-row-per-wave tiles counted at their measured
+// advantage (2048 x 21504 x 2560 with two planes: 472 us at 256 x 224
+// against 551 at 128 x 256).
+static void wide_shape(int n, int N, int *mf, int *nf) {
+  double best = 1e30;
+  for (int f = 2; f >= 1; f--)
+    for (int c = 7; c <= 8; c++) {
+      const int64_t tiles = (int64_t)((n + 128 * f - 1) / (128 * f)) * ((N + 32 * c - 1) / (32 * c));
+      const double cost = (double)((tiles + 255) / 256) * (128 * f) * (32 * c) / (f == 2 ? 1.0 : 0.85);
+      if (cost < best) {
+        best = cost;
+        *mf = f;
+        *nf = c;
+      }
+    }
+}
+
+// K splits of n-row fp32-accurate products that run in one launch: one round
+// of blocks, each product at least four K steps a split.
+static int exact_splits(int n, int max_splits, const MatDesc &w, const MatDesc *other = nullptr) {
+  const int bm = gemm_exact_tall(n) ? 256 : 128;
+  const int64_t tiles = (int64_t)((n + bm - 1) / bm) * ((w.rows + 255) / 256 + (other ? (other->rows + 255) / 256 : 0));
+  const int cols = other ? std::min(w.cols, other->cols) : w.cols;
+  return (int)std::max<int64_t>(1, std::min<int64_t>({256 / tiles, max_splits, cols / 128}));
+}
+
 // y[n][ldy] = x[n][ldx] * W^T: on the matrix cores when the format allows
 // (activations split into bf16 hi/lo planes first), else the vector-unit
 // GEMM. Without rowstream every output row depends only on its own input
@@ -761,7 +810,19 @@ int StableModel::project(const MatDesc &w, const float *x, int ldx, int n, float
   if (splits) *splits = 1;
   const bool reuse = staged && *staged;
   if (staged) *staged = false;
-  if (gemm_mfma_supported(w)) {
+  if (use_few(w, n) && few_rows_supported(w, n, ldx)) {
+    const int ks = splits ? few_rows_splits(w, n, std::max(1, max_splits)) : 1;
+    if (splits) *splits = ks;
+    const FewProduct p{w, x, ldx, y, ldy, ks, (int64_t)n * ldy};
+    STAGE(ST_PREFILL_GEMM, launch_few_rows(&p, 1, n, stream), "projection");
+  } else if (use_exact(w, n) || (!rowstream && w.fmt == FMT_F32 && use_wide && gemm_exact_supported(w, n))) {
+    const int ks = splits ? exact_splits(n, std::max(1, max_splits), w) : 1;
+    if (splits) *splits = ks;
+    const int ld = gemm_exact_ld(w);
+    STAGE(ST_PREFILL_GEMM, launch_split_f16(x, ldx, w.cols, n, XH, XL, ld, XU, stream), "fp16 split");
+    const ExactProduct p{w, XH, XL, ld, XU, y, ldy, ks, (int64_t)n * ldy};
+    STAGE(ST_PREFILL_GEMM, launch_gemm_exact(&p, 1, n, stream), "projection");
+  } else if (gemm_mfma_supported(w)) {
     const bool two = gemm_planes(w, bf16_acts) == 2;
     // K-split partial products (summed by the caller) where the output
     // tiles alone would leave most of the device idle.
@@ -814,25 +875,6 @@ int StableModel::project(const MatDesc &w, const float *x, int ldx, int n, float
   return TINYOAI_OK;
 }
 
-
-// The wide-tile shape (rows per block 128 * mf, columns 32 * nf) for an
-// n-row product with N outputs: the fewest rounds of 256 blocks weighted
-// by the tile area, the 64-row-per-wave tiles counted at their measured
-// advantage (2048 x 21504 x 2560 with two planes: 472 us at 256 x 224
-// against 551 at 128 x 256).
-static void wide_shape(int n, int N, int *mf, int *nf) {
-  double best = 1e30;
-  for (int f = 2; f >= 1; f--)
-    for (int c = 7; c <= 8; c++) {
-      const int64_t tiles = (int64_t)((n + 128 * f - 1) / (128 * f)) * ((N + 32 * c - 1) / (32 * c));
-      const double cost = (double)((tiles + 255) / 256) * (128 * f) * (32 * c) / (f == 2 ? 1.0 : 0.85);
-      if (cost < best) {
-        best = cost;
-        *mf = f;
-        *nf = c;
-      }
-    }
-}
 
 // The same for a Q8_0 product on the wide tiles, 128 * mf rows x 32 * nf
 // columns (nf 8 or 6), the 256-row tiles counted at their measured
@@ -898,6 +940,42 @@ bool StableModel::wide_layer(int l) const {
          dims.inter % 32 == 0;
 }
 
+// Whether an n-row product with w may take the few-row kernel: the format's
+// wide tiles switched on (launch stages 7 and 10 select the 128 x 256 tiles
+// at every size) and, for BF16, two activation planes.
+bool StableModel::use_few(const MatDesc &w, int n) const {
+  return n >= 2 && n <= kFewRowsMax && use_wide &&
+         (w.fmt == FMT_F16 || (w.fmt == FMT_Q8_0 && q8_wide) || (w.fmt == FMT_BF16 && !bf16_acts));
+}
+
+// Whether an n-row product takes the fp32-accurate matrix-core kernel: more
+// rows than the few-row kernels (F16: 64, 5/6-bit formats: 32).
+bool StableModel::use_exact(const MatDesc &w, int n) const {
+  return use_wide && n > 32 && !use_few(w, n) && gemm_exact_supported(w, n);
+}
+
+// The o and down products of n rows (inputs A and M, fp32) as one launch of
+// fp32-accurate products, in *sp and *sd K splits into P and D. The splits
+// are shared in proportion to the K lengths, about one block per CU in all.
+int StableModel::exact_out_products(const MatDesc &wo, const MatDesc &wd, int n, int max_splits, int *sp, int *sd) {
+  const int d = dims.d, I = dims.inter, bm = gemm_exact_tall(n) ? 256 : 128, lo = gemm_exact_ld(wo), ld = gemm_exact_ld(wd);
+  wide_out_splits(n, d, d, I, max_splits, sp, sd, bm);
+  STAGE(ST_PREFILL_GEMM, launch_split_f16(A, d, d, n, XH, XL, lo, XU, stream), "fp16 split");
+  STAGE(ST_PREFILL_GEMM, launch_split_f16(M, I, I, n, MH, ML, ld, XU + chunk, stream), "fp16 split");
+  const ExactProduct out[2] = {{wo, XH, XL, lo, XU, P, d, *sp, (int64_t)n * d},
+                               {wd, MH, ML, ld, XU + chunk, D, d, *sd, (int64_t)n * d}};
+  STAGE(ST_PREFILL_GEMM, launch_gemm_exact(out, 2, n, stream), "projection");
+  return TINYOAI_OK;
+}
+
+// Whether layer l takes an n-token chunk through the few-row kernel: fused
+// win and wout of one of its formats.
+bool StableModel::few_layer(int l, int n) const {
+  const LayerDev &w = layers[l];
+  return !w.win2.rows && !w.wout2.rows && dims.heads * dims.hd == dims.d && use_few(w.win, n) && use_few(w.wout, n) &&
+         few_rows_supported(w.win, n, dims.d) && few_rows_supported(w.wout, n, std::max(dims.d, dims.inter));
+}
+
 // n tokens at positions start.. (StableLM.prefill, prefill.go:33-115): per
 // layer LayerNorm, one product with win and its fused epilogue, causal
 // attention over the cache, the o and down products over the two column
@@ -912,7 +990,7 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
   // matrix-core in-projection, else fp32 H.
   auto ln_out = [&](int l, float *&out, uint16_t *&oh, uint16_t *&ol) {
     const LayerDev &w = layers[l];
-    const bool planes = wide_layer(l) || (!w.win2.rows && gemm_mfma_supported(w.win));
+    const bool planes = !few_layer(l, n) && (wide_layer(l) || (!w.win2.rows && gemm_mfma_supported(w.win)));
     out = planes ? nullptr : H;
     oh = planes ? XH : nullptr;
     ol = planes ? XL : nullptr;
@@ -925,6 +1003,14 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       uint16_t *oh, *ol;
       ln_out(l + 1, out, oh, ol);
       const LayerDev &nw = layers[l + 1];
+      if (n <= kFewRowsMax) {
+        // Few rows: a block per row would leave most of the chip idle while
+        // it sums the partials (19 rows of 25 partials: 26 us).
+        STAGE(ST_PREFILL_ELEMENTWISE, launch_residual(X, P, sp, D, sd, (int64_t)n * d, stream), "residual");
+        STAGE(ST_PREFILL_NORM,
+              launch_layer_norm_rows(X, nw.ln_w, nw.ln_b, dims.eps, n, d, out, stream, oh, ol), "layer_norm");
+        return TINYOAI_OK;
+      }
       STAGE(ST_PREFILL_ELEMENTWISE,
             launch_residual_norm_rows(X, P, sp, D, sd, n, d, nw.ln_w, nw.ln_b, dims.eps, out, oh, ol, stream),
             "residual + layer_norm");
@@ -948,7 +1034,32 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
     // the matrix cores) -> MH, ML -> down; attention -> XH, XL -> o.
     const bool pin = !split_in && gemm_mfma_supported(w.win), pd = gemm_mfma_supported(wd);
     const bool flash = flash_prefill_supported(dims.hd), po = flash && gemm_mfma_supported(wo);
-    if (wide_layer(l)) {
+    if (few_layer(l, n)) {
+      // Up to 64 rows: the few-row products from the fp32 rows, as K splits
+      // that the epilogue and the residual sum; o and down in one launch.
+      if (!normed)
+        STAGE(ST_PREFILL_NORM, launch_layer_norm_rows(X, w.ln_w, w.ln_b, dims.eps, n, d, H, stream), "layer_norm");
+      const int pd_splits = (int)std::min<int64_t>(64, (int64_t)kPrefillSplits * chunk / n);
+      const int si = few_rows_splits(w.win, n, std::min(pd_splits, chunk / n));
+      const FewProduct in{w.win, H, d, Y, win_rows, si, (int64_t)n * win_rows};
+      STAGE(ST_PREFILL_GEMM, launch_few_rows(&in, 1, n, stream), "projection");
+      STAGE(ST_PREFILL_EPILOGUE,
+            launch_in_epilogue(dims, kv[l], Y, win_rows, rope, d_pos0, n, Q, M, stream, nullptr, nullptr, nullptr, si),
+            "in_epilogue");
+      if (flash)
+        STAGE(ST_PREFILL_ATTENTION,
+              launch_flash_prefill(dims, kv[l], Q, d_pos0, n, A, stream, nullptr, nullptr, nullptr, 0, 0, 0, nullptr, 0,
+                                   flash_ksplit ? Y : nullptr, (int64_t)chunk * win_rows, start + n - 1),
+              "attention");
+      else
+        STAGE(ST_PREFILL_ATTENTION,
+              launch_attention(dims, kv[l], Q, d_pos0, n, start + n - 1, partials, counters, A, stream), "attention");
+      int so, sd;
+      few_rows_pair_splits(wo, wd, n, pd_splits, &so, &sd);
+      const FewProduct out[2] = {{wo, A, d, P, d, so, (int64_t)n * d}, {wd, M, I, D, d, sd, (int64_t)n * d}};
+      STAGE(ST_PREFILL_GEMM, launch_few_rows(out, 2, n, stream), "projection");
+      if ((rc = residual(l, so, sd))) return rc;
+    } else if (wide_layer(l)) {
       // BF16 layers on wide tiles: LayerNorm -> planes; win, then its
       // epilogue (q, K/V, SiLU-gate planes); attention -> planes; the o and
       // down products as one launch of K splits; the parallel residual sums
@@ -1007,13 +1118,28 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
         da.inter = 0;
         dm.win_q = dm.win_kv = 0;
         const int ra = w.win.rows, rm = w.win2.rows;
-        float *Ya = Y, *Ym = Y + (size_t)n * ra;
-        if ((rc = project(w.win, H, d, n, Ya, ra)) || (rc = project(w.win2, H, d, n, Ym, rm))) return rc;
+        int sy = 1;
+        const int max_sy = chunk / n;
+        float *Ya = Y, *Ym = Y;
+        if (use_exact(w.win, n) && use_exact(w.win2, n) && gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)) {
+          // one split of H serves both products, which share a launch
+          sy = exact_splits(n, std::max(1, max_sy), w.win, &w.win2);
+          Ym = Y + (size_t)sy * n * ra;
+          const int ld = gemm_exact_ld(w.win);
+          STAGE(ST_PREFILL_GEMM, launch_split_f16(H, d, d, n, XH, XL, ld, XU, stream), "fp16 split");
+          const ExactProduct in[2] = {{w.win, XH, XL, ld, XU, Ya, ra, sy, (int64_t)n * ra},
+                                      {w.win2, XH, XL, ld, XU, Ym, rm, sy, (int64_t)n * rm}};
+          STAGE(ST_PREFILL_GEMM, launch_gemm_exact(in, 2, n, stream), "projection");
+        } else {
+          Ym = Y + (size_t)n * ra;
+          if ((rc = project(w.win, H, d, n, Ya, ra)) || (rc = project(w.win2, H, d, n, Ym, rm))) return rc;
+        }
         STAGE(ST_PREFILL_EPILOGUE,
-              launch_in_epilogue(da, kv[l], Ya, ra, rope, d_pos0, n, Q, M, stream, nullptr, nullptr), "in_epilogue");
+              launch_in_epilogue(da, kv[l], Ya, ra, rope, d_pos0, n, Q, M, stream, nullptr, nullptr, nullptr, sy),
+              "in_epilogue");
         STAGE(ST_PREFILL_EPILOGUE,
               launch_in_epilogue(dm, kv[l], Ym, rm, rope, d_pos0, n, Q, m32, stream, pd ? MH : nullptr,
-                                 pd ? ML : nullptr),
+                                 pd ? ML : nullptr, nullptr, sy),
               "in_epilogue");
       } else if (pin && pd && w.win.fmt == FMT_Q8_0 && n <= 1024 && 2 * n <= chunk) {
         // Up to 1024 rows the Q8_0 in-projection runs as two K halves (twice
@@ -1030,16 +1156,21 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
         STAGE(ST_PREFILL_GEMM, launch_gemm_in_epilogue(w.win, XH, lo_plane(w.win), n, e, stream),
               "projection + epilogue");
       } else {
+        int sy = 1;  // (5/6-bit and F16 products alone come in K splits here)
         if ((rc = pin ? project_planes(w.win, XH, lo_plane(w.win), n, Y, win_rows)
-                      : project(w.win, H, d, n, Y, win_rows)))
+                      : project(w.win, H, d, n, Y, win_rows, use_exact(w.win, n) ? &sy : nullptr, false,
+                                std::max(1, chunk / n))))
           return rc;
         STAGE(ST_PREFILL_EPILOGUE,
               launch_in_epilogue(dims, kv[l], Y, win_rows, rope, d_pos0, n, Q, m32, stream, pd ? MH : nullptr,
-                                 pd ? ML : nullptr),
+                                 pd ? ML : nullptr, nullptr, sy),
               "in_epilogue");
       }
       int sp = 1, sd = 1;
-      if ((rc = pd ? project_planes(wd, MH, gemm_planes(wd, bf16_acts) == 2 ? ML : nullptr, n, D, d, &sd) : project(wd, M, I, n, D, d, &sd)))
+      const bool exact_out = use_exact(wo, n) && use_exact(wd, n) && gemm_exact_pair_supported(wo.fmt, wd.fmt);
+      if (exact_out) {
+        // with the o product, after the attention
+      } else if ((rc = pd ? project_planes(wd, MH, gemm_planes(wd, bf16_acts) == 2 ? ML : nullptr, n, D, d, &sd) : project(wd, M, I, n, D, d, &sd)))
         return rc;
       if (flash)
         STAGE(ST_PREFILL_ATTENTION,
@@ -1051,8 +1182,11 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       else
         STAGE(ST_PREFILL_ATTENTION,
               launch_attention(dims, kv[l], Q, d_pos0, n, start + n - 1, partials, counters, A, stream), "attention");
-      if ((rc = po ? project_planes(wo, XH, lo_plane(wo), n, P, d, &sp) : project(wo, A, d, n, P, d, &sp)))
+      if (exact_out) {
+        if ((rc = exact_out_products(wo, wd, n, kPrefillSplits, &sp, &sd))) return rc;
+      } else if ((rc = po ? project_planes(wo, XH, lo_plane(wo), n, P, d, &sp) : project(wo, A, d, n, P, d, &sp))) {
         return rc;
+      }
       if ((rc = residual(l, sp, sd))) return rc;
     }
     if (tracing) {
@@ -1566,10 +1700,24 @@ struct tinyoai_weight {
   DevMatrix m;
   int device = 0;  // the device the weight lives on
   hipStream_t stream = nullptr;
-  uint16_t *planes = nullptr;  // bf16 hi/lo planes of the last batched product's input
-  size_t planes_bytes = 0;
+  // Operand planes and K-split partials of tinyoai_weight_mul_device, one
+  // buffer per stream it is called on (calls on one stream run in order;
+  // `mu` keeps one call's launches together). At most kStreams of them: with
+  // more, those no captured graph uses are given back. A buffer used under
+  // capture is kept until the weight is closed.
+  struct Scratch {
+    void *ptr = nullptr;
+    size_t bytes = 0;
+    bool captured = false;
+  };
+  static constexpr size_t kStreams = 8;
+  std::mutex mu;
+  std::map<hipStream_t, Scratch> scratch;
+  std::vector<void *> kept;
   ~tinyoai_weight() {
-    if (planes) hipFree(planes);
+    for (auto &s : scratch)
+      if (s.second.ptr) hipFree(s.second.ptr);
+    for (void *p : kept) hipFree(p);
     if (stream) hipStreamDestroy(stream);
   }
 };
@@ -1987,76 +2135,142 @@ int tinyoai_weight_read_values(tinyoai_weight *w, int64_t offset, int64_t n, flo
 
 }  // extern "C"
 
-// Bytes of operand scratch a product of n rows needs: bf16 planes of the
-// matrix-core GEMM, the staged X of the few-row 5/6-bit product, or none
-// (one row: the row-streaming matvec; other formats: the vector-unit GEMM).
-// K splits of a matrix-core product (the output tiles alone leave most of
-// the CUs idle below a few hundred rows: 27 tiles for 128 x 6912), their
-// partials within kProductPartialBytes. A rule of the shape alone, so the
-// allocating and the no-allocation entry points sum alike.
-constexpr size_t kProductPartialBytes = (size_t)32 << 20;
-static int product_splits(const MatDesc &m, int n) {
-  if (n == 1 || !gemm_mfma_supported(m)) return 1;
-  int ks = gemm_splits(m, n, StableModel::kPrefillSplits);
-  while (ks > 1 && (size_t)ks * n * m.rows * 4 > kProductPartialBytes) ks--;
-  return ks;
-}
-static size_t product_planes_bytes(const MatDesc &m, int n) {
-  return ((size_t)n * m.cols * 2 * gemm_planes(m) + 255) / 256 * 256;
-}
-
-static size_t product_scratch(const MatDesc &m, const float *x_dev, int n) {
-  if (n == 1) return 0;
-  if (gemm_mfma_supported(m)) {
-    const int ks = product_splits(m, n);
-    return product_planes_bytes(m, n) + (ks > 1 ? (size_t)ks * n * m.rows * 4 : 0);
+// How a product of n rows runs, and the scratch it needs: partial outputs of
+// `ks` K splits (summed in order), then operand planes. A rule of the shape
+// alone (the partials within kProductPartialBytes), so the allocating and the
+// no-allocation entry points sum alike.
+//   one row: the row-streaming matvec;
+//   F16, BF16, Q8_0 up to 64 rows: the few-row kernel;
+//   Q8_0, BF16: the large tiles (bf16 planes);
+//   5/6-bit formats up to 32 rows: the few-row product (staged X);
+//   F16, F32, 5/6-bit formats: the fp32-accurate tiles (fp16 planes and the
+//   rows' factors);
+//   else (values that are not finite, very few columns) the vector-unit GEMM.
+// Under capture an F16 product of few rows runs in one range, and a product
+// of the fp32-accurate tiles on the vector-unit GEMM, both of which need no
+// scratch: a graph holds no buffer of theirs that other calls use.
+constexpr size_t kProductPartialBytes = (size_t)32 << 20, kProductScratchBytes = (size_t)48 << 20;
+enum class Route { row, few, mfma, exact, kq, simt };
+struct Product {
+  Route route = Route::simt;
+  int ks = 1;
+  size_t planes = 0, partials = 0;  // bytes
+  size_t bytes() const { return planes + partials; }
+};
+static Product plan_product(const MatDesc &m, const float *x_dev, int n, bool capturing) {
+  Product p;
+  auto round256 = [](size_t v) { return (v + 255) / 256 * 256; };
+  auto split = [&](int ks, size_t limit = kProductPartialBytes) {
+    while (ks > 1 && (size_t)ks * n * m.rows * 4 > limit) ks--;
+    p.ks = ks;
+    p.partials = ks > 1 ? round256((size_t)ks * n * m.rows * 4) : 0;
+  };
+  if (n == 1) {
+    p.route = Route::row;
+  } else if (few_rows_supported(m, n, m.cols)) {
+    p.route = Route::few;
+    split(capturing && m.fmt == FMT_F16 ? 1 : few_rows_splits(m, n, 64));
+  } else if (gemm_mfma_supported(m)) {
+    p.route = Route::mfma;
+    p.planes = round256((size_t)n * m.cols * 2 * gemm_planes(m));
+    split(gemm_splits(m, n, StableModel::kPrefillSplits));
+  } else if (kq_rows_supported(m, n) && (reinterpret_cast<uintptr_t>(x_dev) & 15) == 0 && m.cols % 4 == 0) {
+    p.route = Route::kq;
+    p.planes = kq_rows_stage_bytes(m.cols, n);
+  } else if (!capturing && gemm_exact_supported(m, n)) {
+    p.route = Route::exact;
+    p.planes = round256((size_t)n * gemm_exact_ld(m) * 4) + round256((size_t)n * 4);
+    // planes and partials together within the no-allocation array
+    split(exact_splits(n, 32, m), kProductScratchBytes - std::min(p.planes + 256, kProductScratchBytes));
   }
-  if (kq_rows_supported(m, n) && (reinterpret_cast<uintptr_t>(x_dev) & 15) == 0 && m.cols % 4 == 0)
-    return kq_rows_stage_bytes(m.cols, n);
-  return 0;
+  return p;
 }
 
-// out = x * W^T with `scratch` of product_scratch bytes.
-static hipError_t product_launch(const MatDesc &m, const float *x_dev, int n, float *out_dev, void *scratch,
+// out = x * W^T as planned, with `scratch` of p.bytes() bytes.
+static hipError_t product_launch(const Product &p, const MatDesc &m, const float *x, int n, float *out, void *scratch,
                                  hipStream_t st) {
-  // One row: the row-streaming matvec, two blocks per CU (6912 x 2560 Q8_0:
-  // 7.2 us against 9.4 with four and 8.1 with one).
-  if (n == 1) return launch_ln_matvec(m, nullptr, nullptr, 0.0, 0, x_dev, out_dev, device_cu_count() * 2, 256, st);
-  if (gemm_mfma_supported(m)) {
-    uint16_t *hi = (uint16_t *)scratch, *lo = gemm_planes(m) == 2 ? hi + (size_t)n * m.cols : nullptr;
-    const int ks = product_splits(m, n);
-    float *part = reinterpret_cast<float *>((char *)scratch + product_planes_bytes(m, n));
-    hipError_t e = launch_split_bf16(x_dev, m.cols, m.cols, n, hi, lo, st);
-    if (e == hipSuccess) e = launch_gemm_mfma(m, hi, lo, n, ks > 1 ? part : out_dev, m.rows, st, ks);
-    if (e == hipSuccess && ks > 1) e = launch_sum_splits(out_dev, part, ks, (int64_t)n * m.rows, st);
-    return e;
+  uint8_t *planes = (uint8_t *)scratch;
+  float *y = p.ks > 1 ? reinterpret_cast<float *>(planes + p.planes) : out;
+  hipError_t e = hipSuccess;
+  switch (p.route) {
+    case Route::row:
+      // One row: the row-streaming matvec, two blocks per CU (6912 x 2560 Q8_0:
+      // 7.2 us against 9.4 with four and 8.1 with one).
+      return launch_ln_matvec(m, nullptr, nullptr, 0.0, 0, x, out, device_cu_count() * 2, 256, st);
+    case Route::few: {
+      const FewProduct f{m, x, m.cols, y, m.rows, p.ks, (int64_t)n * m.rows};
+      e = launch_few_rows(&f, 1, n, st);
+      break;
+    }
+    case Route::mfma: {
+      uint16_t *hi = (uint16_t *)planes, *lo = gemm_planes(m) == 2 ? hi + (size_t)n * m.cols : nullptr;
+      e = launch_split_bf16(x, m.cols, m.cols, n, hi, lo, st);
+      if (e == hipSuccess) e = launch_gemm_mfma(m, hi, lo, n, y, m.rows, st, p.ks);
+      break;
+    }
+    case Route::exact: {
+      const int ld = gemm_exact_ld(m);
+      uint16_t *hi = (uint16_t *)planes, *lo = hi + (size_t)n * ld;
+      float *unscale = reinterpret_cast<float *>(planes + ((size_t)n * ld * 4 + 255) / 256 * 256);
+      e = launch_split_f16(x, m.cols, m.cols, n, hi, lo, ld, unscale, st);
+      const ExactProduct q{m, hi, lo, ld, unscale, y, m.rows, p.ks, (int64_t)n * m.rows};
+      if (e == hipSuccess) e = launch_gemm_exact(&q, 1, n, st);
+      break;
+    }
+    case Route::kq: return launch_kq_rows(m, x, m.cols, n, out, m.rows, 1, scratch, st);
+    case Route::simt: return launch_gemm(m, x, n, out, st);
   }
-  if (product_scratch(m, x_dev, n)) return launch_kq_rows(m, x_dev, m.cols, n, out_dev, m.rows, 1, scratch, st);
-  return launch_gemm(m, x_dev, n, out_dev, st);
+  if (e == hipSuccess && p.ks > 1) e = launch_sum_splits(out, y, p.ks, (int64_t)n * m.rows, st);
+  return e;
 }
 
 extern "C" {
 
-int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, float *out_dev, void *stream) {
+int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, float *out_dev, void *stream) try {
   if (!w || !x_dev || !out_dev || n <= 0) return fail(TINYOAI_EINVAL, "invalid product arguments");
   hipStream_t st = stream ? (hipStream_t)stream : w->stream;
   const MatDesc &m = w->m.desc;
-  // The operand scratch grows on demand (the stream is drained before an
-  // old buffer is released).
-  const size_t need = product_scratch(m, x_dev, n);
-  if (need > w->planes_bytes) {
-    if (w->planes) {
-      hipStreamSynchronize(st);
-      hipFree(w->planes);
-      w->planes = nullptr;
-      w->planes_bytes = 0;
-    }
-    hipError_t e = hipMalloc(&w->planes, need);
-    if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc(%zu): %s", need, hipGetErrorString(e));
-    w->planes_bytes = need;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(st, &cap);
+  if (e != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
+  const bool capturing = cap != hipStreamCaptureStatusNone;
+  const Product p = plan_product(m, x_dev, n, capturing);
+  if (!p.bytes()) {
+    e = product_launch(p, m, x_dev, n, out_dev, nullptr, st);
+    return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
   }
-  const hipError_t e = product_launch(m, x_dev, n, out_dev, w->planes, st);
+  std::lock_guard<std::mutex> lock(w->mu);
+  if (!capturing && w->scratch.size() >= tinyoai_weight::kStreams && !w->scratch.count(st)) {
+    if ((e = hipDeviceSynchronize()) != hipSuccess) return hip_fail(e, "product scratch");
+    for (auto it = w->scratch.begin(); it != w->scratch.end();) {
+      if (it->second.captured) w->kept.push_back(it->second.ptr);
+      else hipFree(it->second.ptr);
+      it = w->scratch.erase(it);
+    }
+  }
+  // A stream's scratch grows on demand (the stream is drained before an old
+  // buffer is released).
+  tinyoai_weight::Scratch &s = w->scratch[st];
+  if (p.bytes() > s.bytes) {
+    if (s.ptr && s.captured) {
+      w->kept.push_back(s.ptr);
+    } else if (s.ptr) {
+      hipStreamSynchronize(st);
+      hipFree(s.ptr);
+    }
+    s = {};
+    e = hipMalloc(&s.ptr, p.bytes());
+    if (e != hipSuccess) {
+      s.ptr = nullptr;
+      return fail(TINYOAI_ENOMEM, "hipMalloc(%zu): %s", p.bytes(), hipGetErrorString(e));
+    }
+    s.bytes = p.bytes();
+  }
+  s.captured |= capturing;
+  e = product_launch(p, m, x_dev, n, out_dev, s.ptr, st);
   return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
+} catch (const std::exception &e) {
+  return fail(TINYOAI_ENOMEM, "product: %s", e.what());
 }
 
 }  // extern "C"
@@ -2069,7 +2283,8 @@ int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, 
 // per device, with that device current) and only that address is used.
 constexpr size_t kScratchValues = (size_t)4 << 20;  // activation values per call (n * cols)
 // bf16 hi and lo planes (16 MiB), then the K-split partials (32 MiB)
-static __device__ __align__(256) uint16_t scratch[2 * kScratchValues + kProductPartialBytes / 2];
+static __device__ __align__(256) uint16_t scratch[kProductScratchBytes / 2];
+static_assert(2 * kScratchValues * 2 + kProductPartialBytes <= kProductScratchBytes, "planes, then partials");
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -2115,9 +2330,6 @@ int tinyoai_weight_mul_device_noalloc(tinyoai_weight *w, const float *x_dev, int
   if ((size_t)n * m.cols > kScratchValues)
     return fail(TINYOAI_EINVAL, "product of %d x %d activation values exceeds the no-allocation limit of %zu", n, m.cols,
                 kScratchValues);
-  if (product_scratch(m, x_dev, n) > sizeof(scratch))
-    return fail(TINYOAI_EINVAL, "product of %d x %d needs more than the no-allocation limit of %zu bytes", n, m.cols,
-                sizeof(scratch));
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
@@ -2133,8 +2345,12 @@ int tinyoai_weight_mul_device_noalloc(tinyoai_weight *w, const float *x_dev, int
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if ((e = hipStreamIsCapturing(st, &cap)) != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
   const bool order = cap == hipStreamCaptureStatusNone;
+  const Product p = plan_product(m, x_dev, n, !order);
+  if (p.bytes() > sizeof(scratch))
+    return fail(TINYOAI_EINVAL, "product of %d x %d needs more than the no-allocation limit of %zu bytes", n, m.cols,
+                sizeof(scratch));
   if (order && (e = hipStreamWaitEvent(st, d->done, 0)) != hipSuccess) return hip_fail(e, "no-allocation ordering");
-  e = product_launch(m, x_dev, n, out_dev, product_scratch(m, x_dev, n) ? d->ptr : nullptr, st);
+  e = product_launch(p, m, x_dev, n, out_dev, d->ptr, st);
   if (e == hipSuccess && order) e = hipEventRecord(d->done, st);
   return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
 }

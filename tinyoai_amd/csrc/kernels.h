@@ -250,6 +250,25 @@ hipError_t launch_kq_rows_pair(const KqProduct &a, const KqProduct &b, int M, hi
 // with the LayerNorm (weights lw, bias lb, eps) applied on the way.
 hipError_t launch_kq_stage_norm(const float *x, int ldx, int M, int K, const float *lw, const float *lb, double eps,
                                 void *stage, hipStream_t st);
+// Products of 2 to kFewRowsMax rows with an F16 (finite), BF16 or Q8_0
+// matrix: y[M][N] (row stride ldy) = X * W^T, X fp32 with rows ldx apart
+// (converted by the kernel). Product i of a launch (one format) cuts its K
+// range in ks parts whose results go to y + s * split_stride.
+// few_rows_splits, few_rows_pair_splits: the split counts that fill the
+// device for one product or two in a launch (at most max_splits each).
+constexpr int kFewRowsMax = 64;
+struct FewProduct {
+  MatDesc w;
+  const float *x;
+  int64_t ldx;
+  float *y;
+  int ldy, ks;
+  int64_t split_stride;
+};
+bool few_rows_supported(const MatDesc &w, int M, int64_t ldx);
+int few_rows_splits(const MatDesc &w, int M, int max_splits);
+void few_rows_pair_splits(const MatDesc &a, const MatDesc &b, int M, int max_splits, int *sa, int *sb);
+hipError_t launch_few_rows(const FewProduct *p, int nprod, int M, hipStream_t st);
 // The fused in-projection epilogue of a matrix-core win product for M
 // tokens at positions *pos0 + j: RoPE'd q [M][heads*hd], K/V into the
 // cache, and the SiLU-gate outputs as bf16 planes mh, ml [M][inter] (and
@@ -297,6 +316,31 @@ hipError_t launch_gemm_wide(const WideGemm *p, int nprod, int M, int mf, int nf,
 // matrix), on wide tiles.
 hipError_t launch_gemm_wide_in_epilogue(const MatDesc &w, const uint16_t *xh, const uint16_t *xl, int lda, int M,
                                         const InEpilogue &e, int mf, int nf, hipStream_t st);
+// Products of many rows (M >= 2, K >= 64) with F16, F32 or 5/6-bit weights
+// (finite values, row scales formed) on the matrix cores, at fp32 accuracy:
+// y = X * W^T with X as the two fp16 planes of launch_split_f16, rows lda >=
+// gemm_exact_ld apart (zeros past K), and the factor of each row. A launch
+// carries one product, or two of gemm_exact_pair_supported formats; product
+// i cuts its K range in ksplit parts whose results go to
+// y + s * split_stride.
+struct ExactProduct {
+  MatDesc w;
+  const uint16_t *xh, *xl;
+  int lda;
+  const float *unscale;
+  float *y;
+  int ldy, ksplit;
+  int64_t split_stride;
+};
+bool gemm_exact_supported(const MatDesc &w, int M);
+bool gemm_exact_pair_supported(int a, int b);
+inline int gemm_exact_ld(const MatDesc &w) { return (w.cols + 31) / 32 * 32; }
+// Tiles of 256 rows (else 128): where they hold less padding than half of
+// a 128-row tile per 256.
+inline bool gemm_exact_tall(int M) { return (M + 255) / 256 * 2 == (M + 127) / 128; }
+hipError_t launch_gemm_exact(const ExactProduct *p, int nprod, int M, hipStream_t st);
+hipError_t launch_split_f16(const float *x, int64_t ldx, int k, int rows, uint16_t *hi, uint16_t *lo, int ldo,
+                            float *unscale, hipStream_t st);
 // x fp32 [rows][k] (row stride ldx) -> bf16 hi [rows][k] and lo = x - hi.
 hipError_t launch_split_bf16(const float *x, int ldx, int k, int64_t rows, uint16_t *hi, uint16_t *lo,
                              hipStream_t st);
@@ -384,6 +428,9 @@ hipError_t launch_repack(int fmt, const uint8_t *raw, int64_t rows, int64_t cols
 // dst_stride) at byte col0b of the mapped row: placement of one plane.
 hipError_t launch_place_bytes(const uint8_t *src, int64_t rows, int64_t row_bytes, uint8_t *dst, int64_t dst_stride,
                               int64_t col0b, const RowMap &map, hipStream_t st);
+// The row scales of m (see MatDesc::rscale; not for F16) into rscale, and
+// *flag (device memory) nonzero if m holds an infinity or NaN.
+hipError_t launch_row_scales(const MatDesc &m, float *rscale, unsigned *flag, hipStream_t st);
 hipError_t launch_read_values(const MatDesc &m, int64_t offset, int64_t n, float *out, hipStream_t st);
 
 int device_cu_count();

@@ -33,6 +33,12 @@ struct DevMatrix {
   // col0 (a value index) under a row map; waits for the copy to finish.
   int place(int32_t dtype, int64_t rows, int64_t cols, const void *data, uint64_t nbytes, const RowMap &map,
             int64_t col0, hipStream_t st);
+  // Once every tensor is placed: the row scales of F32 and 5/6-bit matrices,
+  // and whether an F16, F32 or 5/6-bit matrix holds an infinity or NaN (the
+  // matrix-core products multiply every weight by both planes of a value,
+  // where an infinite result would become NaN: such a matrix is marked and
+  // keeps to the vector-unit products).
+  int finish(hipStream_t st);
   // create + place of a whole matrix.
   int upload(int32_t dtype, int64_t rows, int64_t cols, const void *data, uint64_t nbytes, hipStream_t st);
 };
@@ -114,6 +120,7 @@ struct StableModel {
   float *X = nullptr, *H = nullptr, *Y = nullptr, *Q = nullptr, *M = nullptr, *A = nullptr, *P = nullptr,
         *D = nullptr;
   uint16_t *XH = nullptr, *XL = nullptr;
+  float *XU = nullptr;  // each row's factor of the fp16 planes in XH, XL, then of those in MH, ML
   uint16_t *MH = nullptr, *ML = nullptr;  // the SiLU-gate outputs as bf16 planes (down projection operand)
   void *h_pinned = nullptr;
   hipEvent_t params_copied = nullptr;  // last H2D copy out of h_pinned's parameter slot
@@ -185,6 +192,10 @@ struct StableModel {
   // layer's whole prefill takes the wide-tile path.
   bool use_wide = true;
   bool wide_layer(int l) const;
+  bool use_few(const MatDesc &w, int n) const;
+  bool use_exact(const MatDesc &w, int n) const;
+  int exact_out_products(const MatDesc &wo, const MatDesc &wd, int n, int max_splits, int *sp, int *sd);
+  bool few_layer(int l, int n) const;
   // The wide-tile in-projection forms its epilogue as a kernel of its own
   // from the product's output (the default), or in the product's own
   // launch (set_launch stage 8 on: one wave per SIMD then runs the float64

@@ -60,7 +60,34 @@ __global__ void read_values_kernel(MatDesc m, int64_t offset, int64_t n, float *
   }
 }
 
+// One block per row.
+__global__ __launch_bounds__(256) void row_scales_kernel(MatDesc m, float *rscale, unsigned *flag) {
+  const int64_t row = blockIdx.x;
+  int most = 0;
+  if (m.fmt == FMT_F16) {  // only whether every value is finite
+    const uint16_t *v = reinterpret_cast<const uint16_t *>(m.vals + row * m.vstride);
+    for (int c = threadIdx.x; c < m.cols; c += 256) most = max(most, (v[c] & 0x7c00) == 0x7c00 ? 0x7f800000 : 0);
+  } else {
+    for (int c = threadIdx.x; c < m.cols; c += 256) most = max(most, __float_as_int(mat_value(m, row, c)) & 0x7fffffff);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o));
+  __shared__ int waves[4];
+  if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = most;
+  __syncthreads();
+  if (threadIdx.x) return;
+  most = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
+  if (most >= 0x7f800000) atomicOr(flag, 1u);
+  const int e = min(max((most >> 23) - 127, -112), 127);
+  if (rscale) rscale[row] = __int_as_float((127 + 14 - e) << 23);
+}
+
 }  // namespace
+
+hipError_t launch_row_scales(const MatDesc &m, float *rscale, unsigned *flag, hipStream_t st) {
+  hipLaunchKernelGGL(row_scales_kernel, dim3(m.rows), dim3(256), 0, st, m, rscale, flag);
+  return hipGetLastError();
+}
 
 hipError_t launch_repack(int fmt, const uint8_t *raw, int64_t rows, int64_t cols, const MatDesc &dst,
                          const RowMap &map, int64_t col0, hipStream_t st) {
