@@ -791,15 +791,6 @@ static void wide_shape(int n, int N, int *mf, int *nf) {
     }
 }
 
-// K splits of n-row fp32-accurate products that run in one launch: one round
-// of blocks, each product at least four K steps a split.
-static int exact_splits(int n, int max_splits, const MatDesc &w, const MatDesc *other = nullptr) {
-  const int bm = gemm_exact_tall(n) ? 256 : 128;
-  const int64_t tiles = (int64_t)((n + bm - 1) / bm) * ((w.rows + 255) / 256 + (other ? (other->rows + 255) / 256 : 0));
-  const int cols = other ? std::min(w.cols, other->cols) : w.cols;
-  return (int)std::max<int64_t>(1, std::min<int64_t>({256 / tiles, max_splits, cols / 128}));
-}
-
 // y[n][ldy] = x[n][ldx] * W^T: on the matrix cores when the format allows
 // (activations split into bf16 hi/lo planes first), else the vector-unit
 // GEMM. Without rowstream every output row depends only on its own input
@@ -816,12 +807,12 @@ int StableModel::project(const MatDesc &w, const float *x, int ldx, int n, float
     const FewProduct p{w, x, ldx, y, ldy, ks, (int64_t)n * ldy};
     STAGE(ST_PREFILL_GEMM, launch_few_rows(&p, 1, n, stream), "projection");
   } else if (use_exact(w, n) || (!rowstream && w.fmt == FMT_F32 && use_wide && gemm_exact_supported(w, n))) {
-    const int ks = splits ? exact_splits(n, std::max(1, max_splits), w) : 1;
-    if (splits) *splits = ks;
+    const ExactPlan plan = gemm_exact_plan(n, w, nullptr, splits ? std::max(1, max_splits) : 1);
+    if (splits) *splits = plan.ks;
     const int ld = gemm_exact_ld(w);
     STAGE(ST_PREFILL_GEMM, launch_split_f16(x, ldx, w.cols, n, XH, XL, ld, XU, stream), "fp16 split");
-    const ExactProduct p{w, XH, XL, ld, XU, y, ldy, ks, (int64_t)n * ldy};
-    STAGE(ST_PREFILL_GEMM, launch_gemm_exact(&p, 1, n, stream), "projection");
+    const ExactProduct p{w, XH, XL, ld, XU, y, ldy, plan.ks, (int64_t)n * ldy};
+    STAGE(ST_PREFILL_GEMM, launch_gemm_exact(&p, 1, n, plan.tall, stream), "projection");
   } else if (gemm_mfma_supported(w)) {
     const bool two = gemm_planes(w, bf16_acts) == 2;
     // K-split partial products (summed by the caller) where the output
@@ -954,17 +945,35 @@ bool StableModel::use_exact(const MatDesc &w, int n) const {
   return use_wide && n > 32 && !use_few(w, n) && gemm_exact_supported(w, n);
 }
 
+// The q/k/v and gate/up products of n rows (LayerNorm output H, split once)
+// as one launch of fp32-accurate products: *sa and *sm K splits at *ya and
+// *ym in Y.
+int StableModel::exact_in_products(const LayerDev &w, int n, float **ya, float **ym, int *sa, int *sm) {
+  const int d = dims.d, ra = w.win.rows, rm = w.win2.rows, ld = gemm_exact_ld(w.win);
+  const ExactPlan plan = gemm_exact_plan(n, w.win, &w.win2, std::max(1, chunk / n));
+  *sa = plan.ks;
+  *sm = plan.ks2;
+  *ya = Y;
+  *ym = Y + (size_t)*sa * n * ra;
+  STAGE(ST_PREFILL_GEMM, launch_split_f16(H, d, d, n, XH, XL, ld, XU, stream), "fp16 split");
+  const ExactProduct in[2] = {{w.win, XH, XL, ld, XU, *ya, ra, *sa, (int64_t)n * ra},
+                              {w.win2, XH, XL, ld, XU, *ym, rm, *sm, (int64_t)n * rm}};
+  STAGE(ST_PREFILL_GEMM, launch_gemm_exact(in, 2, n, plan.tall, stream), "projection");
+  return TINYOAI_OK;
+}
+
 // The o and down products of n rows (inputs A and M, fp32) as one launch of
-// fp32-accurate products, in *sp and *sd K splits into P and D. The splits
-// are shared in proportion to the K lengths, about one block per CU in all.
+// fp32-accurate products, in *sp and *sd K splits into P and D.
 int StableModel::exact_out_products(const MatDesc &wo, const MatDesc &wd, int n, int max_splits, int *sp, int *sd) {
-  const int d = dims.d, I = dims.inter, bm = gemm_exact_tall(n) ? 256 : 128, lo = gemm_exact_ld(wo), ld = gemm_exact_ld(wd);
-  wide_out_splits(n, d, d, I, max_splits, sp, sd, bm);
+  const int d = dims.d, I = dims.inter, lo = gemm_exact_ld(wo), ld = gemm_exact_ld(wd);
+  const ExactPlan plan = gemm_exact_plan(n, wo, &wd, max_splits);
+  *sp = plan.ks;
+  *sd = plan.ks2;
   STAGE(ST_PREFILL_GEMM, launch_split_f16(A, d, d, n, XH, XL, lo, XU, stream), "fp16 split");
   STAGE(ST_PREFILL_GEMM, launch_split_f16(M, I, I, n, MH, ML, ld, XU + chunk, stream), "fp16 split");
   const ExactProduct out[2] = {{wo, XH, XL, lo, XU, P, d, *sp, (int64_t)n * d},
                                {wd, MH, ML, ld, XU + chunk, D, d, *sd, (int64_t)n * d}};
-  STAGE(ST_PREFILL_GEMM, launch_gemm_exact(out, 2, n, stream), "projection");
+  STAGE(ST_PREFILL_GEMM, launch_gemm_exact(out, 2, n, plan.tall, stream), "projection");
   return TINYOAI_OK;
 }
 
@@ -1118,28 +1127,20 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
         da.inter = 0;
         dm.win_q = dm.win_kv = 0;
         const int ra = w.win.rows, rm = w.win2.rows;
-        int sy = 1;
-        const int max_sy = chunk / n;
+        int sa = 1, sm = 1;
         float *Ya = Y, *Ym = Y;
         if (use_exact(w.win, n) && use_exact(w.win2, n) && gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)) {
-          // one split of H serves both products, which share a launch
-          sy = exact_splits(n, std::max(1, max_sy), w.win, &w.win2);
-          Ym = Y + (size_t)sy * n * ra;
-          const int ld = gemm_exact_ld(w.win);
-          STAGE(ST_PREFILL_GEMM, launch_split_f16(H, d, d, n, XH, XL, ld, XU, stream), "fp16 split");
-          const ExactProduct in[2] = {{w.win, XH, XL, ld, XU, Ya, ra, sy, (int64_t)n * ra},
-                                      {w.win2, XH, XL, ld, XU, Ym, rm, sy, (int64_t)n * rm}};
-          STAGE(ST_PREFILL_GEMM, launch_gemm_exact(in, 2, n, stream), "projection");
+          if ((rc = exact_in_products(w, n, &Ya, &Ym, &sa, &sm))) return rc;
         } else {
           Ym = Y + (size_t)n * ra;
           if ((rc = project(w.win, H, d, n, Ya, ra)) || (rc = project(w.win2, H, d, n, Ym, rm))) return rc;
         }
         STAGE(ST_PREFILL_EPILOGUE,
-              launch_in_epilogue(da, kv[l], Ya, ra, rope, d_pos0, n, Q, M, stream, nullptr, nullptr, nullptr, sy),
+              launch_in_epilogue(da, kv[l], Ya, ra, rope, d_pos0, n, Q, M, stream, nullptr, nullptr, nullptr, sa),
               "in_epilogue");
         STAGE(ST_PREFILL_EPILOGUE,
               launch_in_epilogue(dm, kv[l], Ym, rm, rope, d_pos0, n, Q, m32, stream, pd ? MH : nullptr,
-                                 pd ? ML : nullptr, nullptr, sy),
+                                 pd ? ML : nullptr, nullptr, sm),
               "in_epilogue");
       } else if (pin && pd && w.win.fmt == FMT_Q8_0 && n <= 1024 && 2 * n <= chunk) {
         // Up to 1024 rows the Q8_0 in-projection runs as two K halves (twice
@@ -1358,9 +1359,17 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
   }
   const int hq = dims.heads * dims.hd;
   // Final LayerNorm of every branch's newest row, then the classifier.
+  // In K splits, summed into P, while Y and P hold them: one range leaves half
+  // of the CUs idle for 16 rows of a 16384-word vocabulary (49 us).
+  const int64_t head_rows = (int64_t)b.count * V;
+  const int head_room = head_rows <= (int64_t)kPrefillSplits * chunk * d
+                            ? (int)std::min<int64_t>(8, (int64_t)chunk * win_rows / head_rows) : 1;
   auto enqueue_head = [&]() -> int {
     TRY_HIP(launch_layer_norm_rows(b.last, norm_w, norm_b, dims.eps, b.count, d, H, stream), "final norm");
-    return project(head.desc, H, d, b.count, Y, V, nullptr, true);
+    int ks = 1;
+    if (int rc = project(head.desc, H, d, b.count, Y, V, head_room > 1 ? &ks : nullptr, true, head_room)) return rc;
+    if (head_room > 1) TRY_HIP(launch_sum_splits(P, Y, ks, head_rows, stream), "classifier");
+    return TINYOAI_OK;
   };
   const bool lockstep = use_graphs && !prof.on && n == b.count && run == 1 && n <= per;
   for (int r0 = 0; r0 < n; r0 += per) {
@@ -1446,6 +1455,9 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
             sm = kq_rows_splits(w.win2, (int)(ycap / 2 / ((size_t)nc * rm)));
             const KqProduct pa{w.win, XH, Ya, ra, sa, 0}, pm{w.win2, XH, Ym, rm, sm, 0};
             STAGE(ST_PREFILL_GEMM, launch_kq_rows_pair(pa, pm, nc, stream), "projection");
+          } else if (use_exact(w.win, nc) && use_exact(w.win2, nc) &&
+                     gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)) {
+            if ((rc = exact_in_products(w, nc, &Ya, &Ym, &sa, &sm))) return rc;
           } else if ((rc = project(w.win, H, d, nc, Ya, ra, few ? &sa : nullptr, true,
                                    (int)(ycap / 2 / ((size_t)nc * ra)), &staged)) ||
                      (rc = project(w.win2, H, d, nc, Ym, rm, few ? &sm : nullptr, true,
@@ -1485,7 +1497,9 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
                               kq_rows_supported(wd, nc) && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
                               (reinterpret_cast<uintptr_t>(M) & 15) == 0 && d % 4 == 0 && I % 4 == 0 &&
                               st_a + kq_rows_stage_bytes(I, nc) <= cap;
-        if (!out_pair && (rc = project(wd, M, I, nc, D, d, &sd, true, pd_splits))) return rc;
+        const bool exact_out = !out_pair && use_exact(wo, nc) && use_exact(wd, nc) &&
+                               gemm_exact_pair_supported(wo.fmt, wd.fmt);
+        if (!out_pair && !exact_out && (rc = project(wd, M, I, nc, D, d, &sd, true, pd_splits))) return rc;
         if (use_flash) {
           TRY_HIP(launch_flash_prefill(dims, kv[l], Q, d_rows, longest, A, stream, nullptr, nullptr, &b.kv[l], pfx, 0, 0,
                                        b.segs, (int)seg.size() - 1),
@@ -1502,16 +1516,20 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
           STAGE(ST_PREFILL_GEMM, launch_kq_stage_pair(A, d, d, sa, M, I, I, sm, nc, stream), "staging");
           const KqProduct po{wo, sa, P, d, sp, 0}, pm{wd, sm, D, d, sd, 0};
           STAGE(ST_PREFILL_GEMM, launch_kq_rows_pair(po, pm, nc, stream), "projection");
-        } else if ((rc = project(wo, A, d, nc, P, d, &sp, true, pd_splits))) {
+        } else if ((rc = exact_out ? exact_out_products(wo, wd, nc, pd_splits, &sp, &sd)
+                                   : project(wo, A, d, nc, P, d, &sp, true, pd_splits))) {
           return rc;
         }
         TRY_HIP(launch_residual(X, P, sp, D, sd, (int64_t)nc * d, stream), "residual");
       }
-      // each branch's newest row of this chunk
+      // each branch's newest row of this chunk, in one launch (a launch a row
+      // took 4.6 us each, 73 us of a 16-branch step)
+      std::vector<int> src, dst;
       for (size_t k = 0; k + 1 < seg.size(); k++) {
-        const int last_row = seg[k + 1] - 1, j = br[r0 + last_row];
-        TRY_HIP(launch_copy_row(X + (size_t)last_row * d, b.last + (size_t)j * d, d, stream), "branch row");
+        src.push_back(seg[k + 1] - 1);
+        dst.push_back(br[r0 + seg[k + 1] - 1]);
       }
+      TRY_HIP(launch_gather_rows(X, b.last, d, src.data(), dst.data(), (int)src.size(), stream), "branch rows");
       return TINYOAI_OK;
     };
     if (lockstep) {
@@ -1560,7 +1578,7 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
       return fail(TINYOAI_ENOMEM, "pinned logits buffer");
     b.logits_bytes = lbytes;
   }
-  TRY_HIP(hipMemcpyAsync(b.logits_host, Y, lbytes, hipMemcpyDeviceToHost, stream), "logits");
+  TRY_HIP(hipMemcpyAsync(b.logits_host, head_room > 1 ? P : Y, lbytes, hipMemcpyDeviceToHost, stream), "logits");
   TRY_HIP(hipStreamSynchronize(stream), "branch step");
   memcpy(logits, b.logits_host, lbytes);
   for (int j = 0; j < b.count; j++) b.len[j] += add[j];
@@ -2154,6 +2172,7 @@ enum class Route { row, few, mfma, exact, kq, simt };
 struct Product {
   Route route = Route::simt;
   int ks = 1;
+  bool tall = false;                // the fp32-accurate tiles' height
   size_t planes = 0, partials = 0;  // bytes
   size_t bytes() const { return planes + partials; }
 };
@@ -2181,7 +2200,9 @@ static Product plan_product(const MatDesc &m, const float *x_dev, int n, bool ca
     p.route = Route::exact;
     p.planes = round256((size_t)n * gemm_exact_ld(m) * 4) + round256((size_t)n * 4);
     // planes and partials together within the no-allocation array
-    split(exact_splits(n, 32, m), kProductScratchBytes - std::min(p.planes + 256, kProductScratchBytes));
+    const ExactPlan plan = gemm_exact_plan(n, m, nullptr, 32);
+    p.tall = plan.tall;
+    split(plan.ks, kProductScratchBytes - std::min(p.planes + 256, kProductScratchBytes));
   }
   return p;
 }
@@ -2214,7 +2235,7 @@ static hipError_t product_launch(const Product &p, const MatDesc &m, const float
       float *unscale = reinterpret_cast<float *>(planes + ((size_t)n * ld * 4 + 255) / 256 * 256);
       e = launch_split_f16(x, m.cols, m.cols, n, hi, lo, ld, unscale, st);
       const ExactProduct q{m, hi, lo, ld, unscale, y, m.rows, p.ks, (int64_t)n * m.rows};
-      if (e == hipSuccess) e = launch_gemm_exact(&q, 1, n, st);
+      if (e == hipSuccess) e = launch_gemm_exact(&q, 1, n, p.tall, st);
       break;
     }
     case Route::kq: return launch_kq_rows(m, x, m.cols, n, out, m.rows, 1, scratch, st);

@@ -119,16 +119,13 @@ constexpr int loads_of() {
 }
 
 template <int WF, int WM>
-__device__ __forceinline__ void exact_body(const ExactArgs &g, const ExactProduct &P, int b, uint8_t *lds8) {
+__device__ __forceinline__ void exact_body(const ExactArgs &g, const ExactProduct &P, int t, uint8_t *lds8) {
   constexpr int BM = 128 * WM, NW = 4, WP = planes_of<WF>();
   constexpr int kAPlane = BM * 64, kSlot = 2 * kAPlane, kB0 = 2 * kSlot;
   uint16_t *lds16 = reinterpret_cast<uint16_t *>(lds8);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wm = wave & 3, wn = wave >> 2;
   const int K = P.w.cols, N = P.w.rows, nk = (K + kWK - 1) / kWK;
   const int MT = (g.M + BM - 1) / BM, NT = (N + kBN - 1) / kBN, tiles = MT * NT;
-  const int total = tiles * P.ksplit, per = (total + 7) / 8;
-  const int t = (b & 7) * per + (b >> 3);  // blocks go round-robin to the XCDs: one XCD's share a weight tile
-  if (t >= total) return;
   const int split = t / tiles, tt = t - split * tiles, nt = tt / MT, mt = tt - nt * MT;
   const int m0 = mt * BM, n0 = nt * kBN;
   const int k_lo = (int)((int64_t)nk * split / P.ksplit), k_hi = (int)((int64_t)nk * (split + 1) / P.ksplit);
@@ -374,25 +371,33 @@ __device__ __forceinline__ void exact_body(const ExactArgs &g, const ExactProduc
 }
 
 template <int WM>
-int blocks_of(const MatDesc &w, int M, int ks) {
-  const int tiles = ((M + 128 * WM - 1) / (128 * WM)) * ((w.rows + kBN - 1) / kBN);
-  return (tiles * ks + 7) / 8 * 8;
+int tiles_of(const ExactArgs &g, int i) {
+  const ExactProduct &p = g.p[i];
+  return ((g.M + 128 * WM - 1) / (128 * WM)) * ((p.w.rows + kBN - 1) / kBN) * p.ksplit;
 }
+// The launch's tiles in runs over the 8 XCDs (blocks go to them round-robin):
+// XCD x takes tiles [x * per, (x + 1) * per) of both products together, so one
+// XCD's blocks share weight tiles and none holds more than its share. (A run
+// per product gave seven XCDs 33 blocks for 32 CUs where the whole launch had
+// 252: 472 us instead of 258 for 700 rows of 21504 x 2560.)
+__device__ __forceinline__ int tile_of(int per) { return ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3); }
 
 template <int WF, int WM>
-__global__ __launch_bounds__(kThreads) void gemm_exact_kernel(ExactArgs g) {
+__global__ __launch_bounds__(kThreads) void gemm_exact_kernel(ExactArgs g, int tiles, int per) {
   extern __shared__ __align__(16) uint8_t exact_lds[];
-  exact_body<WF, WM>(g, g.p[0], blockIdx.x, exact_lds);
+  const int t = tile_of(per);
+  if (t < tiles) exact_body<WF, WM>(g, g.p[0], t, exact_lds);
 }
 // Two products of the same rows (their own planes, formats and splits), the
-// second's blocks after the first's.
+// second's tiles after the first's.
 template <int WFA, int WFB, int WM>
-__global__ __launch_bounds__(kThreads) void gemm_exact_pair_kernel(ExactArgs g, int blocks0) {
+__global__ __launch_bounds__(kThreads) void gemm_exact_pair_kernel(ExactArgs g, int tiles0, int tiles, int per) {
   extern __shared__ __align__(16) uint8_t exact_lds[];
-  if ((int)blockIdx.x < blocks0)
-    exact_body<WFA, WM>(g, g.p[0], blockIdx.x, exact_lds);
-  else
-    exact_body<WFB, WM>(g, g.p[1], (int)blockIdx.x - blocks0, exact_lds);
+  const int t = tile_of(per);
+  if (t < tiles0)
+    exact_body<WFA, WM>(g, g.p[0], t, exact_lds);
+  else if (t < tiles)
+    exact_body<WFB, WM>(g, g.p[1], t - tiles0, exact_lds);
 }
 
 template <int WF, int WM>
@@ -401,8 +406,8 @@ hipError_t exact_launch(const ExactArgs &g, hipStream_t st) {
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_exact_kernel<WF, WM>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((gemm_exact_kernel<WF, WM>), dim3(blocks_of<WM>(g.p[0].w, g.M, g.p[0].ksplit)), dim3(kThreads),
-                     lds, st, g);
+  const int tiles = tiles_of<WM>(g, 0), per = (tiles + 7) / 8;
+  hipLaunchKernelGGL((gemm_exact_kernel<WF, WM>), dim3(8 * per), dim3(kThreads), lds, st, g, tiles, per);
   return hipGetLastError();
 }
 template <int WFA, int WFB, int WM>
@@ -411,8 +416,8 @@ hipError_t exact_pair_launch(const ExactArgs &g, hipStream_t st) {
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_exact_pair_kernel<WFA, WFB, WM>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return attr;
-  const int b0 = blocks_of<WM>(g.p[0].w, g.M, g.p[0].ksplit), b1 = blocks_of<WM>(g.p[1].w, g.M, g.p[1].ksplit);
-  hipLaunchKernelGGL((gemm_exact_pair_kernel<WFA, WFB, WM>), dim3(b0 + b1), dim3(kThreads), lds, st, g, b0);
+  const int t0 = tiles_of<WM>(g, 0), tiles = t0 + tiles_of<WM>(g, 1), per = (tiles + 7) / 8;
+  hipLaunchKernelGGL((gemm_exact_pair_kernel<WFA, WFB, WM>), dim3(8 * per), dim3(kThreads), lds, st, g, t0, tiles, per);
   return hipGetLastError();
 }
 
@@ -458,7 +463,30 @@ bool gemm_exact_pair_supported(int a, int b) {
   return (a == FMT_Q6_K && b == FMT_Q4_K) || (a == FMT_Q4_K && b == FMT_Q6_K) || (a == b && (a == FMT_Q5_K || a == FMT_F16));
 }
 
-hipError_t launch_gemm_exact(const ExactProduct *p, int nprod, int M, hipStream_t st) {
+ExactPlan gemm_exact_plan(int M, const MatDesc &a, const MatDesc *b, int max_splits) {
+  ExactPlan best;
+  double cost = 1e30;
+  for (int f = 2; f >= 1; f--) {
+    const int64_t mt = (M + 128 * f - 1) / (128 * f), ta = mt * ((a.rows + kBN - 1) / kBN),
+                  tb = b ? mt * ((b->rows + kBN - 1) / kBN) : 0;
+    const int ka = (a.cols + kWK - 1) / kWK, kb = b ? (b->cols + kWK - 1) / kWK : 0;
+    // blocks of at most `steps` K steps each, whichever product they work for
+    for (int steps = 8; steps <= std::max({ka, kb, 8}); steps++) {
+      const int sa = std::min((ka + steps - 1) / steps, max_splits);
+      const int sb = b ? std::min((kb + steps - 1) / steps, max_splits) : 0;
+      const int longest = std::max((ka + sa - 1) / sa, b ? (kb + sb - 1) / sb : 0);
+      const double rounds = (double)((ta * sa + tb * sb + 255) / 256);
+      // a step's time, a block's start and end in steps, and the partial
+      // outputs (written and read) over the steps of the chip
+      const double step = f == 2 ? 3.4 : 2.3;
+      const double c = rounds * (longest + 6) * step + 8e-6 / 5 * M * ((sa - 1.0) * a.rows + (b ? (sb - 1.0) * b->rows : 0));
+      if (c < cost) cost = c, best = ExactPlan{f == 2, sa, sb};
+    }
+  }
+  return best;
+}
+
+hipError_t launch_gemm_exact(const ExactProduct *p, int nprod, int M, bool tall, hipStream_t st) {
   if (nprod < 1 || nprod > 2) return hipErrorInvalidValue;
   ExactArgs g{};
   g.nprod = nprod;
@@ -471,5 +499,5 @@ hipError_t launch_gemm_exact(const ExactProduct *p, int nprod, int M, hipStream_
       return hipErrorInvalidValue;
     g.p[i] = q;
   }
-  return gemm_exact_tall(M) ? exact_dispatch<2>(g, st) : exact_dispatch<1>(g, st);
+  return tall ? exact_dispatch<2>(g, st) : exact_dispatch<1>(g, st);
 }

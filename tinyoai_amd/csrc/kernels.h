@@ -335,10 +335,16 @@ struct ExactProduct {
 bool gemm_exact_supported(const MatDesc &w, int M);
 bool gemm_exact_pair_supported(int a, int b);
 inline int gemm_exact_ld(const MatDesc &w) { return (w.cols + 31) / 32 * 32; }
-// Tiles of 256 rows (else 128): where they hold less padding than half of
-// a 128-row tile per 256.
-inline bool gemm_exact_tall(int M) { return (M + 255) / 256 * 2 == (M + 127) / 128; }
-hipError_t launch_gemm_exact(const ExactProduct *p, int nprod, int M, hipStream_t st);
+// The tiles of 256 rows (tall) or 128 and the K splits of one product or of
+// two in a launch that take the least time by a model of rounds of 256
+// blocks: a K step of a 256-row tile takes 3.4 us on a full chip, of a
+// 128-row one 2.3.
+struct ExactPlan {
+  bool tall = false;
+  int ks = 1, ks2 = 1;
+};
+ExactPlan gemm_exact_plan(int M, const MatDesc &a, const MatDesc *b, int max_splits);
+hipError_t launch_gemm_exact(const ExactProduct *p, int nprod, int M, bool tall, hipStream_t st);
 hipError_t launch_split_f16(const float *x, int64_t ldx, int k, int rows, uint16_t *hi, uint16_t *lo, int ldo,
                             float *unscale, hipStream_t st);
 // x fp32 [rows][k] (row stride ldx) -> bf16 hi [rows][k] and lo = x - hi.
@@ -374,6 +380,10 @@ hipError_t launch_residual_norm_rows(float *x, const float *p, int sp, const flo
                                      uint16_t *ol, hipStream_t st);
 // out[i] = sum over s < sp of p[s * n + i], in order of s.
 hipError_t launch_sum_splits(float *out, const float *p, int sp, int64_t n, hipStream_t st);
+// Rows src[i] of x -> rows dst[i] of out, i < n (host arrays; d values a row),
+// kRowPairs rows a launch.
+constexpr int kRowPairs = 64;
+hipError_t launch_gather_rows(const float *x, float *out, int d, const int *src, const int *dst, int n, hipStream_t st);
 hipError_t launch_copy_row(const float *src, float *dst, int n, hipStream_t st);
 // n 32-bit words from src to dst (both 16-byte aligned; either may be
 // host-mapped memory), with 16-byte accesses.

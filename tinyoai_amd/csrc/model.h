@@ -194,6 +194,7 @@ struct StableModel {
   bool wide_layer(int l) const;
   bool use_few(const MatDesc &w, int n) const;
   bool use_exact(const MatDesc &w, int n) const;
+  int exact_in_products(const LayerDev &w, int n, float **ya, float **ym, int *sa, int *sm);
   int exact_out_products(const MatDesc &wo, const MatDesc &wd, int n, int max_splits, int *sp, int *sd);
   bool few_layer(int l, int n) const;
   // The wide-tile in-projection forms its epilogue as a kernel of its own

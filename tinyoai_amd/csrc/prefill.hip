@@ -247,6 +247,16 @@ __global__ void copy_kernel(const float *src, float *dst, int n) {
   for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
 }
 
+struct RowPairs {
+  int src[kRowPairs], dst[kRowPairs];
+};
+// Row src[i] of x -> row dst[i] of out (d values each), one block per row.
+__global__ void gather_rows_kernel(const float *x, float *out, int d, RowPairs p) {
+  const float *s = x + (int64_t)p.src[blockIdx.x] * d;
+  float *o = out + (int64_t)p.dst[blockIdx.x] * d;
+  for (int i = threadIdx.x; i < d; i += blockDim.x) o[i] = s[i];
+}
+
 // n 32-bit words, 16 bytes per store where both ends allow it: a wide copy
 // (a host-mapped destination then takes full PCIe writes).
 __global__ void copy_words_kernel(const uint32_t *src, uint32_t *dst, int n) {
@@ -335,6 +345,17 @@ hipError_t launch_copy_words(const void *src, void *dst, int n, hipStream_t st) 
   const int threads = 256, blocks = std::max(1, (n / 4 + threads - 1) / threads);
   hipLaunchKernelGGL(copy_words_kernel, dim3(blocks), dim3(threads), 0, st, reinterpret_cast<const uint32_t *>(src),
                      reinterpret_cast<uint32_t *>(dst), n);
+  return hipGetLastError();
+}
+
+hipError_t launch_gather_rows(const float *x, float *out, int d, const int *src, const int *dst, int n, hipStream_t st) {
+  for (int i0 = 0; i0 < n; i0 += kRowPairs) {
+    RowPairs p{};
+    const int c = std::min(n - i0, kRowPairs);
+    std::copy(src + i0, src + i0 + c, p.src);
+    std::copy(dst + i0, dst + i0 + c, p.dst);
+    hipLaunchKernelGGL(gather_rows_kernel, dim3(c), dim3(1024), 0, st, x, out, d, p);
+  }
   return hipGetLastError();
 }
 
