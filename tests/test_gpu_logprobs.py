@@ -69,6 +69,29 @@ def test_summarize_ties_go_to_the_lower_id(hip):
     assert abs(chosen[1] - (-np.log(3000.0))) <= 1e-12
 
 
+@pytest.mark.parametrize("vocab,count", [(16384, 5), (16385, 64), (65535, 10), (4097, 64), (61, 61), (16384, 64)])
+def test_summarize_few_entries(hip, vocab, count):
+    """Few entries of a row held in registers, at the edges of its sizes:
+    random rows, rows of many equal values (more candidates than the ranking
+    holds), equal values across the count boundary at the highest ids, and
+    infinities below the rest."""
+    rng = np.random.default_rng(vocab)
+    x = (rng.standard_normal((5, vocab)) * 4).astype(np.float32)
+    x[1] = np.round(x[1] / 8)
+    x[2] = -7.5
+    x[2, -3:] = 1.0
+    x[3, ::2] = -np.inf
+    x[4] = np.where(rng.random(vocab) < 0.9, np.float32(2.0), np.float32(3.0))
+    t = np.array([0, vocab - 1, vocab // 2, 1, 5])
+    chosen, ids, lp = hip.summarize_logits(x, t, count)
+    wc, wi, wl = expected(x, t, count)
+    assert np.array_equal(ids, wi)
+    assert np.max(np.abs(chosen - wc)) <= 1e-12 * np.max(np.abs(wc))
+    fin = np.isfinite(wl)
+    assert np.array_equal(np.isfinite(lp), fin)
+    assert np.max(np.abs(lp[fin] - wl[fin])) <= 1e-12 * np.max(np.abs(wl[fin]))
+
+
 @pytest.mark.parametrize("count", [3, 1500])
 def test_summarize_signed_zeros_tie(hip, count):
     """-0 and +0 compare equal in summarizeLogits (v > x and v == x), so
