@@ -16,6 +16,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "kernels.h"
@@ -324,6 +325,7 @@ void Profiler::clear() {
 
 // ---------------------------------------------------------------- StableLM
 StableModel::~StableModel() {
+  spare.release();
   free_kv();
   for (void *p : buffers) hipFree(p);
   if (h_pinned) hipHostFree(h_pinned);
@@ -603,6 +605,7 @@ int StableModel::ensure_kv(int needed) {
   const size_t esz = kv_half ? 2 : 4;
   const size_t per_head = (size_t)dims.hd * esz;
   std::vector<KVDev> grown(cfg.num_hidden_layers);
+  if (!open_branches) drop_spare_kv();
   for (auto &l : grown) {
     const size_t bytes = (size_t)dims.kv_heads * want * per_head;
     hipError_t e = hipMalloc(&l.k, bytes);
@@ -1217,6 +1220,12 @@ void Branches::drop_graphs() {
   graphs.clear();
 }
 
+void StableModel::drop_spare_kv() {
+  for (void *p : spare.kv) hipFree(p);
+  spare.kv.clear();
+  spare.kv_bytes = 0;
+}
+
 void Branches::free_kv() {
   for (auto &l : kv) {
     if (l.k) hipFree(l.k);
@@ -1245,15 +1254,39 @@ int StableModel::score_rows(int n) {
   return TINYOAI_OK;
 }
 
-Branches::~Branches() {
-  if (m && m->stream) hipStreamSynchronize(m->stream);
-  drop_graphs();
-  free_kv();
+void BranchBuffers::release() {
+  for (void *p : kv) hipFree(p);
   if (partials) hipFree(partials);
   if (counters) hipFree(counters);
+  if (logits_host) hipHostFree(logits_host);
+  *this = BranchBuffers();
+}
+
+Branches::~Branches() {
+  const bool drained = m && m->stream && hipStreamSynchronize(m->stream) == hipSuccess;
+  drop_graphs();
+  if (drained && !failed && kv_bytes * 2 * kv.size() <= BranchBuffers::kMost) {
+    // the model keeps them for its next session (one session's at most)
+    m->spare.release();
+    for (auto &l : kv) {
+      m->spare.kv.push_back(l.k);
+      m->spare.kv.push_back(l.v);
+    }
+    m->spare.kv_bytes = kv_bytes;
+    m->spare.partials = partials;
+    m->spare.partial_floats = partial_floats;
+    m->spare.counters = counters;
+    m->spare.counter_words = counter_words;
+    m->spare.logits_host = logits_host;
+    m->spare.logits_bytes = logits_bytes;
+  } else {
+    free_kv();
+    if (partials) hipFree(partials);
+    if (counters) hipFree(counters);
+    if (logits_host) hipHostFree(logits_host);
+  }
   if (last) hipFree(last);
   if (segs) hipFree(segs);
-  if (logits_host) hipHostFree(logits_host);
   if (m) m->open_branches--;
 }
 
@@ -1265,15 +1298,31 @@ int Branches::grow(int need) {
   if (want < need) return fail(TINYOAI_EINVAL, "branch suffix of %d positions exceeds its limit %d", need, max_len);
   const StableDims &s = m->dims;
   const size_t esz = m->kv_half ? 2 : 4, row = (size_t)s.hd * esz;
-  const size_t bytes = (size_t)s.kv_heads * count * want * row;
+  const size_t per = (size_t)s.kv_heads * count * row;  // bytes of one position of every branch
   std::vector<KVDev> grown(m->cfg.num_hidden_layers);
-  for (auto &l : grown) {
-    hipError_t e = hipMalloc(&l.k, bytes);
-    if (e == hipSuccess) e = hipMalloc(&l.v, bytes);
-    if (e != hipSuccess) {
-      for (auto &g : grown) { if (g.k) hipFree(g.k); if (g.v) hipFree(g.v); }
-      return fail(TINYOAI_ENOMEM, "branch KV of %d positions: %s", want, hipGetErrorString(e));
+  size_t bytes = per * want;
+  if (m->spare.kv.size() == 2 * grown.size() && m->spare.kv_bytes >= bytes) {
+    // the previous session's buffers, whole
+    bytes = m->spare.kv_bytes;
+    want = (int)std::min<size_t>(max_len, bytes / per);
+    for (size_t l = 0; l < grown.size(); l++) {
+      grown[l].k = m->spare.kv[2 * l];
+      grown[l].v = m->spare.kv[2 * l + 1];
     }
+    m->spare.kv.clear();
+    m->spare.kv_bytes = 0;
+  } else {
+    m->drop_spare_kv();
+    for (auto &l : grown) {
+      hipError_t e = hipMalloc(&l.k, bytes);
+      if (e == hipSuccess) e = hipMalloc(&l.v, bytes);
+      if (e != hipSuccess) {
+        for (auto &g : grown) { if (g.k) hipFree(g.k); if (g.v) hipFree(g.v); }
+        return fail(TINYOAI_ENOMEM, "branch KV of %d positions: %s", want, hipGetErrorString(e));
+      }
+    }
+  }
+  for (auto &l : grown) {
     l.cap = count * want;
     l.half = m->kv_half;
   }
@@ -1296,6 +1345,7 @@ int Branches::grow(int need) {
   drop_graphs();  // they name the old caches
   free_kv();
   kv = grown;
+  kv_bytes = bytes;
   scap = want;
   return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "branch KV growth");
 }
@@ -1841,6 +1891,7 @@ int tinyoai_stablelm_reset(tinyoai_model *m) {
   if (!m || !m->stable) return fail(TINYOAI_EINVAL, "not a StableLM handle");
   if (int rc = m->stable->busy_with_branches()) return rc;
   hipStreamSynchronize(m->stable->stream);
+  m->stable->spare.release();
   m->stable->free_kv();
   return TINYOAI_OK;
 }
@@ -1891,6 +1942,14 @@ int tinyoai_stablelm_branches_open(tinyoai_model *m, int32_t prefix, int32_t cou
   b.len.assign(count, 0);
   hipError_t e = hipMalloc(&b.last, (size_t)count * s.dims.d * 4);
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "branch rows: %s", hipGetErrorString(e));
+  // scratch the previous session left (the counters zero, as each launch
+  // leaves them)
+  b.partials = std::exchange(s.spare.partials, nullptr);
+  b.partial_floats = std::exchange(s.spare.partial_floats, 0);
+  b.counters = std::exchange(s.spare.counters, nullptr);
+  b.counter_words = std::exchange(s.spare.counter_words, 0);
+  b.logits_host = std::exchange(s.spare.logits_host, nullptr);
+  b.logits_bytes = std::exchange(s.spare.logits_bytes, 0);
   *out = h.release();
   return TINYOAI_OK;
 }
@@ -1910,7 +1969,10 @@ static int branches_run(tinyoai_branches *h, const int32_t *tokens, const int32_
                   j, add[j] + b.len[j], b.max_len, b.prefix);
   }
   const int rc = s.branch_rows(b, tokens, br, n, logits);
-  if (rc) h->b.reset();
+  if (rc) {
+    h->b->failed = true;
+    h->b.reset();
+  }
   return rc;
 }
 

@@ -77,6 +77,25 @@ struct Profiler {
   void clear();
 };
 
+// What a closed branch session leaves for the model's next one: its caches'
+// buffers (hipMalloc and hipFree of the 16-branch session's 4096-token
+// caches took 5 of its 21 ms), attention scratch and pinned logits. One
+// session's at most and no more than kMost bytes of caches; given back with
+// the model, at a reset, when the model's own cache grows, or when a session
+// needs larger ones.
+struct BranchBuffers {
+  static constexpr size_t kMost = (size_t)8 << 30;
+  std::vector<void *> kv;  // per layer K, V: kv_bytes each
+  size_t kv_bytes = 0;
+  float *partials = nullptr;
+  size_t partial_floats = 0;
+  unsigned *counters = nullptr;
+  size_t counter_words = 0;
+  float *logits_host = nullptr;
+  size_t logits_bytes = 0;
+  void release();
+};
+
 // A StableLM resident on one GPU with its KV cache (stableState,
 // stablelm.go:216-225, kept in HBM).
 struct StableModel {
@@ -100,6 +119,8 @@ struct StableModel {
   // the model gate (branches.go:16-22).
   int open_branches = 0;
   int busy_with_branches() const;
+  BranchBuffers spare;
+  void drop_spare_kv();
 
   // decode workspaces
   float *x = nullptr, *qbuf = nullptr, *mbuf = nullptr, *abuf = nullptr, *logits_dev = nullptr;
@@ -236,7 +257,7 @@ struct StableModel {
 // never written; branch j owns the suffix positions prefix + [0, len[j]),
 // held in per-layer caches laid out [kv_heads][count * scap][hd], so that
 // branch j's suffix entry s is slot j * scap + s. The caches grow (to a
-// power of two, at most max_len) when a branch needs more positions, as
+// power of two or what the previous session left, at most max_len) when a branch needs more positions, as
 // appendBranchKV allocates only the suffix length used
 // (mlx_branches.go:50-69).
 struct Branches {
@@ -244,6 +265,8 @@ struct Branches {
   int prefix = 0, count = 0, max_len = 0;
   std::vector<int> len;
   int scap = 0;
+  bool failed = false;           // a call failed: nothing is kept for the next session
+  size_t kv_bytes = 0;           // of each K and V buffer
   std::vector<KVDev> kv;
   float *partials = nullptr;     // split-K attention partials
   size_t partial_floats = 0;
