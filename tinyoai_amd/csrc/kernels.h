@@ -401,7 +401,7 @@ size_t logprob_scratch_bytes(int count);
 hipError_t launch_logprobs(const float *logits, int64_t ld, int rows, int vocab, const int *targets, int count,
                            double *chosen, int *top_ids, double *top_lp, void *scratch, hipStream_t st);
 
-// ---- the stories260K-shaped Llama, every token of a call in one launch ----
+// ---- the stories260K-shaped Llama: a token in one launch, or several side by side ----
 constexpr int kTinyDim = 64, kTinyHidden = 172, kTinyMaxLayers = 8, kTinyMaxSeq = 512, kTinyMaxVocab = 512,
               kTinyMaxTokens = 256;
 // Packed fp32 weights, per layer: [wq | wk | wv] (128 x 64), wo (64 x 64),
@@ -428,6 +428,10 @@ struct TinyLlamaArgs {
 };
 bool tiny_llama_supported(int dim, int hidden, int heads, int kv_heads, int layers, int vocab, int seq);
 hipError_t launch_tiny_llama(const TinyLlamaArgs &a, hipStream_t st);
+// One token (a.n == 1); several side by side, in layers + 1 launches: xbuf and
+// qbuf hold kTinyMaxTokens rows of kTinyDim floats, *arrived is zero before
+// and after.
+hipError_t launch_tiny_llama_many(const TinyLlamaArgs &a, float *xbuf, float *qbuf, unsigned *arrived, hipStream_t st);
 
 // ---- weights ----
 // Places raw GGUF-encoded bytes (already in device memory) of a

@@ -180,6 +180,11 @@ int LlamaModel::init(const tinyoai_llama_config &c, const float *w, uint64_t n_f
                                hipMemcpyDeviceToDevice, stream),
                 "packed weights");
       }
+    if ((rc = alloc((void **)&tiny_x, (size_t)kTinyMaxTokens * kTinyDim * 4)) ||
+        (rc = alloc((void **)&tiny_q, (size_t)kTinyMaxTokens * kTinyDim * 4)) ||
+        (rc = alloc((void **)&tiny_arrived, 256)))
+      return rc;
+    TRY_HIP(hipMemsetAsync(tiny_arrived, 0, 256, stream), "packed weights");
     TRY_HIP(hipStreamSynchronize(stream), "packed weights");
   }
   tiny = tiny_ok;
@@ -308,9 +313,10 @@ int LlamaModel::forward(int prefix, const int32_t *tokens, int n, bool all_logit
 
 constexpr int kTinySpinMs = 200;  // host wait for the completion word before waiting on the stream
 
-// forward for the stories260K shape: one launch per kTinyMaxTokens tokens
-// (every token of the call in one workgroup, in order), the logits rows
-// written by the kernel into mapped pinned host memory.
+// forward for the stories260K shape: a token in one launch; more of them side
+// by side, kTinyMaxTokens at a time (54 us for 2 to 16 tokens and 91 for 255,
+// where one workgroup took them in order at about 10 us each); the logits
+// rows written by the kernels into mapped pinned host memory.
 int LlamaModel::forward_tiny(int prefix, const int32_t *tokens, int n, bool all_logits, float *logits) {
   const int rows = all_logits ? n : 1, vocab = cfg.vocab_size;
   if (!done_host) {
@@ -360,7 +366,9 @@ int LlamaModel::forward_tiny(int prefix, const int32_t *tokens, int n, bool all_
     a.done = final ? done_dev : nullptr;
     a.seq = ++done_seq;
     std::memcpy(a.tokens, tokens + c0, (size_t)cnt * 4);
-    TRY_HIP(launch_tiny_llama(a, stream), "token launch");
+    TRY_HIP(cnt > 1 ? launch_tiny_llama_many(a, tiny_x, tiny_q, tiny_arrived, stream)
+                             : launch_tiny_llama(a, stream),
+            "token launch");
   }
   // The last launch sets the completion word after its rows: the rows are
   // read as soon as it appears (the stream's own completion comes later).

@@ -317,6 +317,8 @@ struct LlamaModel {
   // logits rows land in pinned host memory (out_host, out_rows rows).
   bool tiny_ok = false, tiny = false;
   uint8_t *tiny_w = nullptr;  // packed weights (layout in kernels.h)
+  float *tiny_x = nullptr, *tiny_q = nullptr;  // residual rows and queries of tokens taken side by side
+  unsigned *tiny_arrived = nullptr;
   void *kv_base = nullptr;    // every layer's K and V (kv[l] points into it)
   float *out_host = nullptr, *out_dev = nullptr;
   int out_rows = 0;
