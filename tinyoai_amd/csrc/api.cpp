@@ -813,7 +813,7 @@ int StableModel::project(const MatDesc &w, const float *x, int ldx, int n, float
     const ExactPlan plan = gemm_exact_plan(n, w, nullptr, splits ? std::max(1, max_splits) : 1);
     if (splits) *splits = plan.ks;
     const int ld = gemm_exact_ld(w);
-    STAGE(ST_PREFILL_GEMM, launch_split_f16(x, ldx, w.cols, n, XH, XL, ld, XU, stream), "fp16 split");
+    if (x) STAGE(ST_PREFILL_GEMM, launch_split_f16(x, ldx, w.cols, n, XH, XL, ld, XU, stream), "fp16 split");
     const ExactProduct p{w, XH, XL, ld, XU, y, ldy, plan.ks, (int64_t)n * ldy};
     STAGE(ST_PREFILL_GEMM, launch_gemm_exact(&p, 1, n, plan.tall, stream), "projection");
   } else if (gemm_mfma_supported(w)) {
@@ -948,17 +948,26 @@ bool StableModel::use_exact(const MatDesc &w, int n) const {
   return use_wide && n > 32 && !use_few(w, n) && gemm_exact_supported(w, n);
 }
 
-// The q/k/v and gate/up products of n rows (LayerNorm output H, split once)
-// as one launch of fp32-accurate products: *sa and *sm K splits at *ya and
-// *ym in Y.
-int StableModel::exact_in_products(const LayerDev &w, int n, float **ya, float **ym, int *sa, int *sm) {
+// Whether layer l's LayerNorm of n rows leaves as the fp16 planes of its
+// fp32-accurate in-product or pair of them (in XH, XL, XU).
+bool StableModel::norm_planes(int l, int n) const {
+  const LayerDev &w = layers[l];
+  return dims.norm == 0 && norm_rows_planes_ok(gemm_exact_ld(w.win)) && norm_rows_planes_ok(dims.d) &&
+         use_exact(w.win, n) &&
+         (!w.win2.rows || (use_exact(w.win2, n) && gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)));
+}
+
+// The q/k/v and gate/up products of n rows (LayerNorm output: with `split`
+// already in planes, else H, split once) as one launch of fp32-accurate
+// products: *sa and *sm K splits at *ya and *ym in Y.
+int StableModel::exact_in_products(const LayerDev &w, int n, bool split, float **ya, float **ym, int *sa, int *sm) {
   const int d = dims.d, ra = w.win.rows, rm = w.win2.rows, ld = gemm_exact_ld(w.win);
   const ExactPlan plan = gemm_exact_plan(n, w.win, &w.win2, std::max(1, chunk / n));
   *sa = plan.ks;
   *sm = plan.ks2;
   *ya = Y;
   *ym = Y + (size_t)*sa * n * ra;
-  STAGE(ST_PREFILL_GEMM, launch_split_f16(H, d, d, n, XH, XL, ld, XU, stream), "fp16 split");
+  if (!split) STAGE(ST_PREFILL_GEMM, launch_split_f16(H, d, d, n, XH, XL, ld, XU, stream), "fp16 split");
   const ExactProduct in[2] = {{w.win, XH, XL, ld, XU, *ya, ra, *sa, (int64_t)n * ra},
                               {w.win2, XH, XL, ld, XU, *ym, rm, *sm, (int64_t)n * rm}};
   STAGE(ST_PREFILL_GEMM, launch_gemm_exact(in, 2, n, plan.tall, stream), "projection");
@@ -1000,8 +1009,14 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
   STAGE(ST_EMBED, launch_embed(embed.desc, d_ids, n, X, stream), "embed");
   // Where layer l's LayerNorm output goes: bf16 planes XH, XL for a
   // matrix-core in-projection, else fp32 H.
-  auto ln_out = [&](int l, float *&out, uint16_t *&oh, uint16_t *&ol) {
+  auto ln_out = [&](int l, float *&out, uint16_t *&oh, uint16_t *&ol, Fp16Planes &fp) {
     const LayerDev &w = layers[l];
+    if (norm_planes(l, n)) {
+      out = nullptr;
+      oh = ol = nullptr;
+      fp = Fp16Planes{XH, XL, gemm_exact_ld(w.win), XU};
+      return;
+    }
     const bool planes = !few_layer(l, n) && (wide_layer(l) || (!w.win2.rows && gemm_mfma_supported(w.win)));
     out = planes ? nullptr : H;
     oh = planes ? XH : nullptr;
@@ -1013,18 +1028,19 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
     if (l + 1 < cfg.num_hidden_layers && dims.norm == 0) {
       float *out;
       uint16_t *oh, *ol;
-      ln_out(l + 1, out, oh, ol);
+      Fp16Planes fp;
+      ln_out(l + 1, out, oh, ol, fp);
       const LayerDev &nw = layers[l + 1];
       if (n <= kFewRowsMax) {
         // Few rows: a block per row would leave most of the chip idle while
         // it sums the partials (19 rows of 25 partials: 26 us).
         STAGE(ST_PREFILL_ELEMENTWISE, launch_residual(X, P, sp, D, sd, (int64_t)n * d, stream), "residual");
         STAGE(ST_PREFILL_NORM,
-              launch_layer_norm_rows(X, nw.ln_w, nw.ln_b, dims.eps, n, d, out, stream, oh, ol), "layer_norm");
+              launch_layer_norm_rows(X, nw.ln_w, nw.ln_b, dims.eps, n, d, out, stream, oh, ol, 0, fp), "layer_norm");
         return TINYOAI_OK;
       }
       STAGE(ST_PREFILL_ELEMENTWISE,
-            launch_residual_norm_rows(X, P, sp, D, sd, n, d, nw.ln_w, nw.ln_b, dims.eps, out, oh, ol, stream),
+            launch_residual_norm_rows(X, P, sp, D, sd, n, d, nw.ln_w, nw.ln_b, dims.eps, out, oh, ol, stream, fp),
             "residual + layer_norm");
       return TINYOAI_OK;
     }
@@ -1116,11 +1132,14 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       STAGE(ST_PREFILL_GEMM, launch_gemm_wide(prods, 2, n, omf, 8, stream), "projection");
       if ((rc = residual(l, so, sd))) return rc;
     } else {
-      if (!normed)
+      if (!normed) {
+        float *out;
+        uint16_t *oh, *ol;
+        Fp16Planes fp;
+        ln_out(l, out, oh, ol, fp);
         STAGE(ST_PREFILL_NORM,
-              launch_layer_norm_rows(X, w.ln_w, w.ln_b, dims.eps, n, d, pin ? nullptr : H, stream, pin ? XH : nullptr,
-                                     pin ? XL : nullptr),
-              "layer_norm");
+              launch_layer_norm_rows(X, w.ln_w, w.ln_b, dims.eps, n, d, out, stream, oh, ol, 0, fp), "layer_norm");
+      }
       float *m32 = pd && !tracing ? nullptr : M;
       if (split_in) {
         // [q | k | v] and the gate/up pairs in formats of their own: two
@@ -1133,7 +1152,7 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
         int sa = 1, sm = 1;
         float *Ya = Y, *Ym = Y;
         if (use_exact(w.win, n) && use_exact(w.win2, n) && gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)) {
-          if ((rc = exact_in_products(w, n, &Ya, &Ym, &sa, &sm))) return rc;
+          if ((rc = exact_in_products(w, n, norm_planes(l, n), &Ya, &Ym, &sa, &sm))) return rc;
         } else {
           Ym = Y + (size_t)n * ra;
           if ((rc = project(w.win, H, d, n, Ya, ra)) || (rc = project(w.win2, H, d, n, Ym, rm))) return rc;
@@ -1162,8 +1181,8 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       } else {
         int sy = 1;  // (5/6-bit and F16 products alone come in K splits here)
         if ((rc = pin ? project_planes(w.win, XH, lo_plane(w.win), n, Y, win_rows)
-                      : project(w.win, H, d, n, Y, win_rows, use_exact(w.win, n) ? &sy : nullptr, false,
-                                std::max(1, chunk / n))))
+                      : project(w.win, norm_planes(l, n) ? nullptr : H, d, n, Y, win_rows,
+                                use_exact(w.win, n) ? &sy : nullptr, false, std::max(1, chunk / n))))
           return rc;
         STAGE(ST_PREFILL_EPILOGUE,
               launch_in_epilogue(dims, kv[l], Y, win_rows, rope, d_pos0, n, Q, m32, stream, pd ? MH : nullptr,
@@ -1507,7 +1526,7 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
             STAGE(ST_PREFILL_GEMM, launch_kq_rows_pair(pa, pm, nc, stream), "projection");
           } else if (use_exact(w.win, nc) && use_exact(w.win2, nc) &&
                      gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)) {
-            if ((rc = exact_in_products(w, nc, &Ya, &Ym, &sa, &sm))) return rc;
+            if ((rc = exact_in_products(w, nc, false, &Ya, &Ym, &sa, &sm))) return rc;
           } else if ((rc = project(w.win, H, d, nc, Ya, ra, few ? &sa : nullptr, true,
                                    (int)(ycap / 2 / ((size_t)nc * ra)), &staged)) ||
                      (rc = project(w.win2, H, d, nc, Ym, rm, few ? &sm : nullptr, true,
@@ -2313,9 +2332,13 @@ int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, 
   if (!w || !x_dev || !out_dev || n <= 0) return fail(TINYOAI_EINVAL, "invalid product arguments");
   hipStream_t st = stream ? (hipStream_t)stream : w->stream;
   const MatDesc &m = w->m.desc;
+  hipError_t e = hipSuccess;
+  if (n == 1) {  // a few microseconds: no more host work than the launch
+    e = product_launch(Product{Route::row}, m, x_dev, n, out_dev, nullptr, st);
+    return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
+  }
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  hipError_t e = hipStreamIsCapturing(st, &cap);
-  if (e != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
+  if ((e = hipStreamIsCapturing(st, &cap)) != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
   const bool capturing = cap != hipStreamCaptureStatusNone;
   const Product p = plan_product(m, x_dev, n, capturing);
   if (!p.bytes()) {

@@ -37,10 +37,7 @@ constexpr int kThreads = 512, kBN = 256;
 constexpr uint32_t kNone = 0x80000000u, kPast = 0x40000000u;
 constexpr int kPlane = kBN * 64;  // bytes of one weight plane of a step
 
-// One block per row: x (fp32) -> fp16 hi and lo = s x - hi with s a power of
-// two that takes the row's largest finite magnitude to [2^14, 2^15) (22
-// bits of every value near it, no overflow), zeros past k, and 1 / s. An
-// infinity or NaN stays in the hi plane alone.
+// One block per row: x (fp32) -> its fp16 planes (Fp16Planes), zeros past k.
 __global__ __launch_bounds__(256) void split_f16_kernel(const float *x, int64_t ldx, int k, uint16_t *hi, uint16_t *lo,
                                                         int ldo, float *unscale) {
   const int64_t row = blockIdx.x;
@@ -56,43 +53,35 @@ __global__ __launch_bounds__(256) void split_f16_kernel(const float *x, int64_t 
       v[u] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
     }
   };
-  auto mag = [](float f) {
-    const int u = __float_as_int(f) & 0x7fffffff;
-    return u < 0x7f800000 ? u : 0;
-  };
   __shared__ int wave_most[4];
   int most = 0;
   for (int i0 = 0; i0 < k; i0 += U * 1024) {
     load(i0);
 #pragma unroll
-    for (int u = 0; u < U; u++) most = max(max(most, max(mag(v[u].x), mag(v[u].y))), max(mag(v[u].z), mag(v[u].w)));
+    for (int u = 0; u < U; u++)
+      most = max(max(most, max(fp16_magnitude(v[u].x), fp16_magnitude(v[u].y))),
+                 max(fp16_magnitude(v[u].z), fp16_magnitude(v[u].w)));
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o));
   if ((threadIdx.x & 63) == 0) wave_most[threadIdx.x >> 6] = most;
   __syncthreads();
   most = max(max(wave_most[0], wave_most[1]), max(wave_most[2], wave_most[3]));
-  const int e = min(max((most >> 23) - 127, -112), 127);
-  const float s = __int_as_float((127 + 14 - e) << 23);
+  float inverse;
+  const float s = fp16_scale(most, inverse);
   for (int i0 = 0; i0 < ldo; i0 += U * 1024) {
     if (k > U * 1024) load(i0);
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int i = i0 + 4 * ((int)threadIdx.x + 256 * u);
       if (i >= ldo) break;
-      const float f[4] = {v[u].x * s, v[u].y * s, v[u].z * s, v[u].w * s};
-      uint32_t a[4], b[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const _Float16 t = (_Float16)f[q];
-        a[q] = __builtin_bit_cast(uint16_t, t);
-        b[q] = (a[q] & 0x7c00u) == 0x7c00u ? 0u : __builtin_bit_cast(uint16_t, (_Float16)(f[q] - (float)t));
-      }
-      *reinterpret_cast<uint2 *>(h + i) = make_uint2(a[0] | a[1] << 16, a[2] | a[3] << 16);
-      *reinterpret_cast<uint2 *>(l + i) = make_uint2(b[0] | b[1] << 16, b[2] | b[3] << 16);
+      uint2 a, b;
+      fp16_split4(v[u], s, a, b);
+      *reinterpret_cast<uint2 *>(h + i) = a;
+      *reinterpret_cast<uint2 *>(l + i) = b;
     }
   }
-  if (threadIdx.x == 0) unscale[row] = __int_as_float((127 - 14 + e) << 23);
+  if (threadIdx.x == 0) unscale[row] = inverse;
 }
 
 template <int WF>

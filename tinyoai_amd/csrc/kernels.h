@@ -193,12 +193,46 @@ hipError_t launch_ln_matvec(const MatDesc &w, const float *ln_w, const float *ln
 hipError_t launch_embed(const MatDesc &emb, const int *ids, int n, float *x, hipStream_t st);
 
 
+// The fp16 operand planes of a row for the fp32-accurate products
+// (launch_split_f16): hi + lo of the row times a power of two that takes its
+// largest finite magnitude (ordered bits: fp16_magnitude) to [2^14, 2^15), so
+// hi + lo hold 22 bits and more and nothing overflows; an infinity or NaN
+// stays in the hi plane alone. unscale[row] is the inverse factor.
+struct Fp16Planes {
+  uint16_t *hi = nullptr, *lo = nullptr;
+  int ld = 0;  // values between rows, zeros past the row
+  float *unscale = nullptr;
+};
+__device__ __forceinline__ int fp16_magnitude(float f) {
+  const int u = __float_as_int(f) & 0x7fffffff;
+  return u < 0x7f800000 ? u : 0;
+}
+__device__ __forceinline__ float fp16_scale(int most, float &inverse) {
+  const int e = min(max((most >> 23) - 127, -112), 127);  // both factors normal numbers
+  inverse = __int_as_float((127 - 14 + e) << 23);
+  return __int_as_float((127 + 14 - e) << 23);
+}
+__device__ __forceinline__ void fp16_split4(float4 v, float scale, uint2 &hi, uint2 &lo) {
+  const float f[4] = {v.x * scale, v.y * scale, v.z * scale, v.w * scale};
+  uint32_t a[4], b[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    const _Float16 t = (_Float16)f[q];
+    a[q] = __builtin_bit_cast(uint16_t, t);
+    b[q] = (a[q] & 0x7c00u) == 0x7c00u ? 0u : __builtin_bit_cast(uint16_t, (_Float16)(f[q] - (float)t));
+  }
+  hi = make_uint2(a[0] | a[1] << 16, a[2] | a[3] << 16);
+  lo = make_uint2(b[0] | b[1] << 16, b[2] | b[3] << 16);
+}
+
 // ---- prefill (n tokens) ----
+// Whether rows of d values may leave a LayerNorm launch as fp16 planes.
+bool norm_rows_planes_ok(int d);
 // out (fp32, may be null) and / or bf16 operand planes oh, ol (null: none)
 // with rows ldo values apart (0: d).
 hipError_t launch_layer_norm_rows(const float *x, const float *w, const float *b, double eps, int n, int d,
                                   float *out, hipStream_t st, uint16_t *oh = nullptr, uint16_t *ol = nullptr,
-                                  int ldo = 0);
+                                  int ldo = 0, Fp16Planes fp = {});
 // out[n][rows] = x[n][cols] * W^T on the vector units (any format/shape).
 hipError_t launch_gemm(const MatDesc &w, const float *x, int n, float *out, hipStream_t st);
 // The matrix-core product: y[M][N] (row stride ldy) = X * W^T with X given
@@ -377,7 +411,7 @@ hipError_t launch_residual(float *x, const float *p, int sp, const float *d, int
 // the two launches.
 hipError_t launch_residual_norm_rows(float *x, const float *p, int sp, const float *dd, int sd, int n, int d,
                                      const float *w, const float *b, double eps, float *out, uint16_t *oh,
-                                     uint16_t *ol, hipStream_t st);
+                                     uint16_t *ol, hipStream_t st, Fp16Planes fp = {});
 // out[i] = sum over s < sp of p[s * n + i], in order of s.
 hipError_t launch_sum_splits(float *out, const float *p, int sp, int64_t n, hipStream_t st);
 // Rows src[i] of x -> rows dst[i] of out, i < n (host arrays; d values a row),

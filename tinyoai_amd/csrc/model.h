@@ -195,6 +195,7 @@ struct StableModel {
   // kRowStreamMax rows in another format without a matrix-core path as one
   // row-streaming matvec per row; otherwise every chunk size takes the
   // same arithmetic.
+  // A null x (fp32-accurate products only): its fp16 planes are in XH, XL, XU.
   // staged (few-row 5/6-bit products): in, the workspace already holds
   // this x from the previous product of the same shape; out, it does now.
   int project(const MatDesc &w, const float *x, int ldx, int n, float *y, int ldy, int *splits = nullptr,
@@ -215,7 +216,8 @@ struct StableModel {
   bool wide_layer(int l) const;
   bool use_few(const MatDesc &w, int n) const;
   bool use_exact(const MatDesc &w, int n) const;
-  int exact_in_products(const LayerDev &w, int n, float **ya, float **ym, int *sa, int *sm);
+  bool norm_planes(int l, int n) const;
+  int exact_in_products(const LayerDev &w, int n, bool split, float **ya, float **ym, int *sa, int *sm);
   int exact_out_products(const MatDesc &wo, const MatDesc &wd, int n, int max_splits, int *sp, int *sd);
   bool few_layer(int l, int n) const;
   // The wide-tile in-projection forms its epilogue as a kernel of its own
