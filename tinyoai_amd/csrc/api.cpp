@@ -125,7 +125,7 @@ int DevMatrix::create(int32_t dtype, int64_t rows, int64_t cols, hipStream_t st)
     return fail(TINYOAI_EINVAL, "unsupported tensor type %d", dtype);
   if (gguf_bytes(dtype, 1, cols) < 0)
     return fail(TINYOAI_EINVAL, "rows of type %d must hold whole quant blocks (%lld values)", dtype, (long long)cols);
-  MatDesc m{};
+  Matrix m{};
   m.fmt = dtype;
   m.rows = (int32_t)rows;
   m.cols = (int32_t)cols;
@@ -222,7 +222,7 @@ int DevMatrix::place(int32_t dtype, int64_t rows, int64_t cols, const void *data
 }
 
 int DevMatrix::finish(hipStream_t st) {
-  MatDesc &m = desc;
+  Matrix &m = desc;
   if (m.fmt == FMT_Q8_0 || m.fmt == FMT_BF16) return TINYOAI_OK;
   unsigned special = 0, *flag = reinterpret_cast<unsigned *>((uint8_t *)mem + bytes - 256);
   float *scales = m.fmt == FMT_F16 ? nullptr : reinterpret_cast<float *>((uint8_t *)flag - ((size_t)m.rows * 4 + 255) / 256 * 256);
@@ -245,8 +245,8 @@ int DevMatrix::upload(int32_t dtype, int64_t rows, int64_t cols, const void *dat
   return rc ? rc : finish(st);
 }
 
-MatDesc column_view(const MatDesc &m, int64_t col0, int64_t cols) {
-  MatDesc v = m;
+Matrix column_view(const Matrix &m, int64_t col0, int64_t cols) {
+  Matrix v = m;
   if (is_kquant(m.fmt)) {
     const RowPtr r = row_ptr(m, 0, col0 / 32);
     v.vals = r.v;
@@ -482,11 +482,11 @@ int StableModel::init(const tinyoai_stablelm_config &c, const tinyoai_tensor *te
       return rc;
     for (DevMatrix *m : {&win, &wout, &win2, &wout2})
       if (m->mem && (rc = m->finish(stream))) return rc;
-    LayerDev &L = layers[l];
+    Layer &L = layers[l];
     L.win = win.desc;
     L.wout = wout.desc;
-    L.win2 = split_in ? win2.desc : MatDesc{};
-    L.wout2 = split_out ? wout2.desc : MatDesc{};
+    L.win2 = split_in ? win2.desc : Matrix{};
+    L.wout2 = split_out ? wout2.desc : Matrix{};
     mixed_layers |= split_in || split_out;
     if ((rc = load_vec(p + "input_layernorm.weight", &L.ln_w))) return rc;
     if ((rc = load_vec(p + "input_layernorm.bias", &L.ln_b))) return rc;
@@ -577,8 +577,8 @@ int StableModel::check_wait_error(int rc) {
 // attention inside its decode_in launch.
 bool StableModel::decode_fused(int steps) const {
   if (!fuse_attention) return false;
-  for (const LayerDev &w : layers)
-    if (decode_in_att_supported(w, dims, threads_in, steps)) return true;
+  for (const Layer &w : layers)
+    if (decode_in_att_supported(w.dev(), dims, threads_in, steps)) return true;
   return false;
 }
 
@@ -675,7 +675,7 @@ int StableModel::enqueue_decode(int steps, int splits, bool want_logits) {
   const int io_params = io_words_logits();
   TRY_HIP(launch_copy_words((const uint32_t *)d_io + io_params, params, 16 + dims.rot, stream), "parameters");
   for (int l = 0; l < cfg.num_hidden_layers; l++) {
-    const LayerDev &w = layers[l];
+    const LayerDev w = layers[l].dev();
     const float *rope_row = reinterpret_cast<const float *>(params + 16);
     const MatDesc *emb = l == 0 ? &embed.desc : nullptr;
     if (fuse_attention && decode_in_att_supported(w, dims, threads_in, steps)) {
@@ -799,7 +799,7 @@ static void wide_shape(int n, int N, int *mf, int *nf) {
 // GEMM. Without rowstream every output row depends only on its own input
 // row, whatever the chunk size (a prefix reused from the cache gives the
 // same results).
-int StableModel::project(const MatDesc &w, const float *x, int ldx, int n, float *y, int ldy, int *splits,
+int StableModel::project(const Matrix &w, const float *x, int ldx, int n, float *y, int ldy, int *splits,
                          bool rowstream, int max_splits, bool *staged) {
   if (splits) *splits = 1;
   const bool reuse = staged && *staged;
@@ -924,7 +924,7 @@ int StableModel::project_planes(const MatDesc &w, const uint16_t *xh, const uint
 // Whether layer l's prefill takes the wide-tile BF16 path: fused BF16
 // win and wout, operands in bf16 planes from their producers.
 bool StableModel::wide_layer(int l) const {
-  const LayerDev &w = layers[l];
+  const Layer &w = layers[l];
   const bool bf16 = w.win.fmt == FMT_BF16 && w.wout.fmt == FMT_BF16;
   // Q8_0: the down section of wout starts on an even quant block (d % 64)
   const bool q8 = q8_wide && w.win.fmt == FMT_Q8_0 && w.wout.fmt == FMT_Q8_0 && wide_q8_ok(w.win) &&
@@ -937,21 +937,21 @@ bool StableModel::wide_layer(int l) const {
 // Whether an n-row product with w may take the few-row kernel: the format's
 // wide tiles switched on (launch stages 7 and 10 select the 128 x 256 tiles
 // at every size) and, for BF16, two activation planes.
-bool StableModel::use_few(const MatDesc &w, int n) const {
+bool StableModel::use_few(const Matrix &w, int n) const {
   return n >= 2 && n <= kFewRowsMax && use_wide &&
          (w.fmt == FMT_F16 || (w.fmt == FMT_Q8_0 && q8_wide) || (w.fmt == FMT_BF16 && !bf16_acts));
 }
 
 // Whether an n-row product takes the fp32-accurate matrix-core kernel: more
 // rows than the few-row kernels (F16: 64, 5/6-bit formats: 32).
-bool StableModel::use_exact(const MatDesc &w, int n) const {
+bool StableModel::use_exact(const Matrix &w, int n) const {
   return use_wide && n > 32 && !use_few(w, n) && gemm_exact_supported(w, n);
 }
 
 // Whether layer l's LayerNorm of n rows leaves as the fp16 planes of its
 // fp32-accurate in-product or pair of them (in XH, XL, XU).
 bool StableModel::norm_planes(int l, int n) const {
-  const LayerDev &w = layers[l];
+  const Layer &w = layers[l];
   return dims.norm == 0 && norm_rows_planes_ok(gemm_exact_ld(w.win)) && norm_rows_planes_ok(dims.d) &&
          use_exact(w.win, n) &&
          (!w.win2.rows || (use_exact(w.win2, n) && gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)));
@@ -960,7 +960,7 @@ bool StableModel::norm_planes(int l, int n) const {
 // The q/k/v and gate/up products of n rows (LayerNorm output: with `split`
 // already in planes, else H, split once) as one launch of fp32-accurate
 // products: *sa and *sm K splits at *ya and *ym in Y.
-int StableModel::exact_in_products(const LayerDev &w, int n, bool split, float **ya, float **ym, int *sa, int *sm) {
+int StableModel::exact_in_products(const Layer &w, int n, bool split, float **ya, float **ym, int *sa, int *sm) {
   const int d = dims.d, ra = w.win.rows, rm = w.win2.rows, ld = gemm_exact_ld(w.win);
   const ExactPlan plan = gemm_exact_plan(n, w.win, &w.win2, std::max(1, chunk / n));
   *sa = plan.ks;
@@ -976,7 +976,7 @@ int StableModel::exact_in_products(const LayerDev &w, int n, bool split, float *
 
 // The o and down products of n rows (inputs A and M, fp32) as one launch of
 // fp32-accurate products, in *sp and *sd K splits into P and D.
-int StableModel::exact_out_products(const MatDesc &wo, const MatDesc &wd, int n, int max_splits, int *sp, int *sd) {
+int StableModel::exact_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd) {
   const int d = dims.d, I = dims.inter, lo = gemm_exact_ld(wo), ld = gemm_exact_ld(wd);
   const ExactPlan plan = gemm_exact_plan(n, wo, &wd, max_splits);
   *sp = plan.ks;
@@ -992,7 +992,7 @@ int StableModel::exact_out_products(const MatDesc &wo, const MatDesc &wd, int n,
 // Whether layer l takes an n-token chunk through the few-row kernel: fused
 // win and wout of one of its formats.
 bool StableModel::few_layer(int l, int n) const {
-  const LayerDev &w = layers[l];
+  const Layer &w = layers[l];
   return !w.win2.rows && !w.wout2.rows && dims.heads * dims.hd == dims.d && use_few(w.win, n) && use_few(w.wout, n) &&
          few_rows_supported(w.win, n, dims.d) && few_rows_supported(w.wout, n, std::max(dims.d, dims.inter));
 }
@@ -1010,7 +1010,7 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
   // Where layer l's LayerNorm output goes: bf16 planes XH, XL for a
   // matrix-core in-projection, else fp32 H.
   auto ln_out = [&](int l, float *&out, uint16_t *&oh, uint16_t *&ol, Fp16Planes &fp) {
-    const LayerDev &w = layers[l];
+    const Layer &w = layers[l];
     if (norm_planes(l, n)) {
       out = nullptr;
       oh = ol = nullptr;
@@ -1030,7 +1030,7 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       uint16_t *oh, *ol;
       Fp16Planes fp;
       ln_out(l + 1, out, oh, ol, fp);
-      const LayerDev &nw = layers[l + 1];
+      const Layer &nw = layers[l + 1];
       if (n <= kFewRowsMax) {
         // Few rows: a block per row would leave most of the chip idle while
         // it sums the partials (19 rows of 25 partials: 26 us).
@@ -1048,12 +1048,12 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
     return TINYOAI_OK;
   };
   for (int l = 0; l < cfg.num_hidden_layers; l++) {
-    const LayerDev &w = layers[l];
+    const Layer &w = layers[l];
     const bool split_in = w.win2.rows > 0, split_out = w.wout2.rows > 0;
     const int64_t vpc = values_per_chunk(w.wout.fmt), down0 = (d + vpc - 1) / vpc * vpc;
-    const MatDesc wo = split_out ? w.wout : column_view(w.wout, 0, d);
+    const Matrix wo = split_out ? w.wout : column_view(w.wout, 0, d);
     const bool normed = l > 0 && dims.norm == 0;  // formed with the previous layer's residual
-    const MatDesc wd = split_out ? w.wout2 : column_view(w.wout, down0, I);
+    const Matrix wd = split_out ? w.wout2 : column_view(w.wout, down0, I);
     int rc;
     // Inputs of matrix-core projections leave their producers as bf16
     // planes (no separate split pass); the fp32 copies are kept where
@@ -1485,11 +1485,11 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
     auto enqueue_chunk = [&]() -> int {
       TRY_HIP(launch_embed(embed.desc, d_ids, nc, X, stream), "embed");
       for (int l = 0; l < cfg.num_hidden_layers; l++) {
-        const LayerDev &w = layers[l];
+        const Layer &w = layers[l];
         const bool split_in = w.win2.rows > 0, split_out = w.wout2.rows > 0;
         const int64_t vpc = values_per_chunk(w.wout.fmt), down0 = (d + vpc - 1) / vpc * vpc;
-        const MatDesc wo = split_out ? w.wout : column_view(w.wout, 0, d);
-        const MatDesc wd = split_out ? w.wout2 : column_view(w.wout, down0, I);
+        const Matrix wo = split_out ? w.wout : column_view(w.wout, 0, d);
+        const Matrix wd = split_out ? w.wout2 : column_view(w.wout, down0, I);
         int rc;
         // Y holds chunk * win_rows floats: with few rows, K-split partials of
         // the in-products fit within it (half each when the two groups are
@@ -2257,7 +2257,7 @@ struct Product {
   size_t planes = 0, partials = 0;  // bytes
   size_t bytes() const { return planes + partials; }
 };
-static Product plan_product(const MatDesc &m, const float *x_dev, int n, bool capturing) {
+static Product plan_product(const Matrix &m, const float *x_dev, int n, bool capturing) {
   Product p;
   auto round256 = [](size_t v) { return (v + 255) / 256 * 256; };
   auto split = [&](int ks, size_t limit = kProductPartialBytes) {
@@ -2289,7 +2289,7 @@ static Product plan_product(const MatDesc &m, const float *x_dev, int n, bool ca
 }
 
 // out = x * W^T as planned, with `scratch` of p.bytes() bytes.
-static hipError_t product_launch(const Product &p, const MatDesc &m, const float *x, int n, float *out, void *scratch,
+static hipError_t product_launch(const Product &p, const Matrix &m, const float *x, int n, float *out, void *scratch,
                                  hipStream_t st) {
   uint8_t *planes = (uint8_t *)scratch;
   float *y = p.ks > 1 ? reinterpret_cast<float *>(planes + p.planes) : out;
@@ -2331,7 +2331,7 @@ extern "C" {
 int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, float *out_dev, void *stream) try {
   if (!w || !x_dev || !out_dev || n <= 0) return fail(TINYOAI_EINVAL, "invalid product arguments");
   hipStream_t st = stream ? (hipStream_t)stream : w->stream;
-  const MatDesc &m = w->m.desc;
+  const Matrix &m = w->m.desc;
   hipError_t e = hipSuccess;
   if (n == 1) {  // a few microseconds: no more host work than the launch
     e = product_launch(Product{Route::row}, m, x_dev, n, out_dev, nullptr, st);
@@ -2432,7 +2432,7 @@ extern "C" {
 
 int tinyoai_weight_mul_device_noalloc(tinyoai_weight *w, const float *x_dev, int32_t n, float *out_dev, void *stream) {
   if (!w || !x_dev || !out_dev || n <= 0) return fail(TINYOAI_EINVAL, "invalid product arguments");
-  const MatDesc &m = w->m.desc;
+  const Matrix &m = w->m.desc;
   if ((size_t)n * m.cols > kScratchValues)
     return fail(TINYOAI_EINVAL, "product of %d x %d activation values exceeds the no-allocation limit of %zu", n, m.cols,
                 kScratchValues);
@@ -2463,7 +2463,7 @@ int tinyoai_weight_mul_device_noalloc(tinyoai_weight *w, const float *x_dev, int
 
 int tinyoai_weight_mul(tinyoai_weight *w, const float *x, int32_t n, float *out) {
   if (!w || !x || !out || n <= 0) return fail(TINYOAI_EINVAL, "invalid product arguments");
-  const MatDesc &m = w->m.desc;
+  const Matrix &m = w->m.desc;
   float *dx = nullptr, *dout = nullptr;
   hipError_t e = hipMalloc(&dx, (size_t)n * m.cols * 4);
   if (e == hipSuccess) e = hipMalloc(&dout, (size_t)n * m.rows * 4);

@@ -390,7 +390,7 @@ double launch_cost(int blocks, int kb, int fmt, double partial_bytes) {
 
 }  // namespace
 
-bool few_rows_supported(const MatDesc &w, int M, int64_t ldx) {
+bool few_rows_supported(const Matrix &w, int M, int64_t ldx) {
   if (M < 2 || M > kFewRowsMax || w.cols < 1 || w.vstride % 16 || (reinterpret_cast<uintptr_t>(w.vals) & 15) ||
       (int64_t)w.rows * w.vstride > 0x7fffffff || (int64_t)M * ldx * 4 > 0x7fffffff)
     return false;

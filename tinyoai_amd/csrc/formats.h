@@ -36,8 +36,16 @@ struct MatDesc {
   int32_t chunks;       // 16-byte chunks per row = vstride / 16
   const uint8_t *hbits; // [rows][hstride] bytes (Q5_1, Q5_K, Q6_K)
   int64_t hstride;
-  int32_t special;      // an F16, F32 or 5/6-bit matrix holding an infinity or NaN (DevMatrix::finish)
-  const float *rscale;  // F32 and 5/6-bit: per row the power of two that takes its largest value to [2^14, 2^15)
+};
+
+// A matrix as the host keeps it: with what the fp32-accurate matrix-core
+// products need to know (DevMatrix::finish). The kernels that do not take a
+// MatDesc alone: 16 more bytes of each matrix in the decode kernels' arguments
+// cost a step 0.7%.
+struct Matrix : MatDesc {
+  int32_t special = 0;            // an F16, F32 or 5/6-bit matrix holding an infinity or NaN
+  const float *rscale = nullptr;  // F32 and 5/6-bit: per row the power of two that takes its largest value to
+                                  // [2^14, 2^15)
 };
 
 __host__ __device__ inline bool is_kquant(int fmt) {

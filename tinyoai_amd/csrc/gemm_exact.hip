@@ -10,7 +10,7 @@
 // Operands: X comes as fp16 hi + lo planes of rows scaled by a power of two
 // (launch_split_f16: 22 bits and more of every value). F16 weights are used
 // as stored. Other formats are decoded once per block to the fp32 values of
-// mat_value, scaled by the row's power of two (MatDesc::rscale, from the
+// mat_value, scaled by the row's power of two (Matrix::rscale, from the
 // row's largest value) and split into fp16 hi + lo planes; the products are
 // hi hi + lo hi + hi lo. A K step of 32 columns is summed on the matrix
 // cores from zero and added to the fp32 totals, so a total rounds once per
@@ -440,7 +440,7 @@ hipError_t launch_split_f16(const float *x, int64_t ldx, int k, int rows, uint16
   return hipGetLastError();
 }
 
-bool gemm_exact_supported(const MatDesc &w, int M) {
+bool gemm_exact_supported(const Matrix &w, int M) {
   constexpr int64_t kGiB = int64_t(1) << 30;
   const bool fmt = w.fmt == FMT_F16 || ((w.fmt == FMT_F32 || is_kquant(w.fmt)) && w.rscale);
   return fmt && !w.special && M >= 2 && w.cols >= 2 * kWK && w.vstride % 16 == 0 &&

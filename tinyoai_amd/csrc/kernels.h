@@ -292,14 +292,14 @@ hipError_t launch_kq_stage_norm(const float *x, int ldx, int M, int K, const flo
 // device for one product or two in a launch (at most max_splits each).
 constexpr int kFewRowsMax = 64;
 struct FewProduct {
-  MatDesc w;
+  Matrix w;
   const float *x;
   int64_t ldx;
   float *y;
   int ldy, ks;
   int64_t split_stride;
 };
-bool few_rows_supported(const MatDesc &w, int M, int64_t ldx);
+bool few_rows_supported(const Matrix &w, int M, int64_t ldx);
 int few_rows_splits(const MatDesc &w, int M, int max_splits);
 void few_rows_pair_splits(const MatDesc &a, const MatDesc &b, int M, int max_splits, int *sa, int *sb);
 hipError_t launch_few_rows(const FewProduct *p, int nprod, int M, hipStream_t st);
@@ -358,7 +358,7 @@ hipError_t launch_gemm_wide_in_epilogue(const MatDesc &w, const uint16_t *xh, co
 // i cuts its K range in ksplit parts whose results go to
 // y + s * split_stride.
 struct ExactProduct {
-  MatDesc w;
+  Matrix w;
   const uint16_t *xh, *xl;
   int lda;
   const float *unscale;
@@ -366,7 +366,7 @@ struct ExactProduct {
   int ldy, ksplit;
   int64_t split_stride;
 };
-bool gemm_exact_supported(const MatDesc &w, int M);
+bool gemm_exact_supported(const Matrix &w, int M);
 bool gemm_exact_pair_supported(int a, int b);
 inline int gemm_exact_ld(const MatDesc &w) { return (w.cols + 31) / 32 * 32; }
 // The tiles of 256 rows (tall) or 128 and the K splits of one product or of
@@ -476,7 +476,7 @@ hipError_t launch_repack(int fmt, const uint8_t *raw, int64_t rows, int64_t cols
 // dst_stride) at byte col0b of the mapped row: placement of one plane.
 hipError_t launch_place_bytes(const uint8_t *src, int64_t rows, int64_t row_bytes, uint8_t *dst, int64_t dst_stride,
                               int64_t col0b, const RowMap &map, hipStream_t st);
-// The row scales of m (see MatDesc::rscale; not for F16) into rscale, and
+// The row scales of m (see Matrix::rscale; not for F16) into rscale, and
 // *flag (device memory) nonzero if m holds an infinity or NaN.
 hipError_t launch_row_scales(const MatDesc &m, float *rscale, unsigned *flag, hipStream_t st);
 hipError_t launch_read_values(const MatDesc &m, int64_t offset, int64_t n, float *out, hipStream_t st);

@@ -19,7 +19,7 @@ int hip_fail(hipError_t e, const char *what);
 
 // One weight matrix in HBM, in the plane layout of formats.h.
 struct DevMatrix {
-  MatDesc desc{};
+  Matrix desc{};
   void *mem = nullptr;
   size_t bytes = 0;
   DevMatrix() = default;
@@ -45,7 +45,7 @@ struct DevMatrix {
 
 // A column range [col0, col0 + cols) of a matrix as a matrix of its own
 // (col0 on a 16-byte chunk boundary, and on a block boundary for Q8_0).
-MatDesc column_view(const MatDesc &m, int64_t col0, int64_t cols);
+Matrix column_view(const Matrix &m, int64_t col0, int64_t cols);
 
 // Stage timings with hipEvents on the model's stream, the device-side
 // counterpart of stableProfile (stablelm.go:227-250). Off by default; when
@@ -77,6 +77,15 @@ struct Profiler {
   void clear();
 };
 
+// A StableLM layer's matrices as the host keeps them (LayerDev: as the decode
+// kernels take them).
+struct Layer {
+  Matrix win, wout;
+  const float *ln_w = nullptr, *ln_b = nullptr;
+  Matrix win2, wout2;
+  LayerDev dev() const { return LayerDev{win, wout, ln_w, ln_b, win2, wout2}; }
+};
+
 // What a closed branch session leaves for the model's next one: its caches'
 // buffers (hipMalloc and hipFree of the 16-branch session's 4096-token
 // caches took 5 of its 21 ms), attention scratch and pinned logits. One
@@ -105,7 +114,7 @@ struct StableModel {
   DevMatrix embed, head;
   std::vector<DevMatrix> mats;  // win, wout, win2, wout2 of each layer
   bool mixed_layers = false;    // some layer keeps its MLP (or down) matrices as sections of their own
-  std::vector<LayerDev> layers;
+  std::vector<Layer> layers;
   const float *norm_w = nullptr, *norm_b = nullptr;
   float *rope = nullptr;
   std::vector<float> rope_host;  // [pos][rot]: a decode token's row travels with its parameters
@@ -198,7 +207,7 @@ struct StableModel {
   // A null x (fp32-accurate products only): its fp16 planes are in XH, XL, XU.
   // staged (few-row 5/6-bit products): in, the workspace already holds
   // this x from the previous product of the same shape; out, it does now.
-  int project(const MatDesc &w, const float *x, int ldx, int n, float *y, int ldy, int *splits = nullptr,
+  int project(const Matrix &w, const float *x, int ldx, int n, float *y, int ldy, int *splits = nullptr,
               bool rowstream = false, int max_splits = kPrefillSplits, bool *staged = nullptr);
   // y = X * W^T with X already in bf16 planes xh, xl (matrix-core formats).
   // BF16-weight prefill products take bf16 activations (one plane) when
@@ -214,11 +223,11 @@ struct StableModel {
   // layer's whole prefill takes the wide-tile path.
   bool use_wide = true;
   bool wide_layer(int l) const;
-  bool use_few(const MatDesc &w, int n) const;
-  bool use_exact(const MatDesc &w, int n) const;
+  bool use_few(const Matrix &w, int n) const;
+  bool use_exact(const Matrix &w, int n) const;
   bool norm_planes(int l, int n) const;
-  int exact_in_products(const LayerDev &w, int n, bool split, float **ya, float **ym, int *sa, int *sm);
-  int exact_out_products(const MatDesc &wo, const MatDesc &wd, int n, int max_splits, int *sp, int *sd);
+  int exact_in_products(const Layer &w, int n, bool split, float **ya, float **ym, int *sa, int *sm);
+  int exact_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd);
   bool few_layer(int l, int n) const;
   // The wide-tile in-projection forms its epilogue as a kernel of its own
   // from the product's output (the default), or in the product's own
