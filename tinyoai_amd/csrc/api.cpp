@@ -989,6 +989,15 @@ int StableModel::exact_out_products(const Matrix &wo, const Matrix &wd, int n, i
   return TINYOAI_OK;
 }
 
+// The same as one launch of few-row products.
+int StableModel::few_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd) {
+  const int d = dims.d, I = dims.inter;
+  few_rows_pair_splits(wo, wd, n, max_splits, sp, sd);
+  const FewProduct out[2] = {{wo, A, d, P, d, *sp, (int64_t)n * d}, {wd, M, I, D, d, *sd, (int64_t)n * d}};
+  STAGE(ST_PREFILL_GEMM, launch_few_rows(out, 2, n, stream), "projection");
+  return TINYOAI_OK;
+}
+
 // Whether layer l takes an n-token chunk through the few-row kernel: fused
 // win and wout of one of its formats.
 bool StableModel::few_layer(int l, int n) const {
@@ -1083,9 +1092,7 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
         STAGE(ST_PREFILL_ATTENTION,
               launch_attention(dims, kv[l], Q, d_pos0, n, start + n - 1, partials, counters, A, stream), "attention");
       int so, sd;
-      few_rows_pair_splits(wo, wd, n, pd_splits, &so, &sd);
-      const FewProduct out[2] = {{wo, A, d, P, d, so, (int64_t)n * d}, {wd, M, I, D, d, sd, (int64_t)n * d}};
-      STAGE(ST_PREFILL_GEMM, launch_few_rows(out, 2, n, stream), "projection");
+      if ((rc = few_out_products(wo, wd, n, pd_splits, &so, &sd))) return rc;
       if ((rc = residual(l, so, sd))) return rc;
     } else if (wide_layer(l)) {
       // BF16 layers on wide tiles: LayerNorm -> planes; win, then its
@@ -1568,7 +1575,9 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
                               st_a + kq_rows_stage_bytes(I, nc) <= cap;
         const bool exact_out = !out_pair && use_exact(wo, nc) && use_exact(wd, nc) &&
                                gemm_exact_pair_supported(wo.fmt, wd.fmt);
-        if (!out_pair && !exact_out && (rc = project(wd, M, I, nc, D, d, &sd, true, pd_splits))) return rc;
+        const bool few_out = !split_out && use_few(wo, nc) && use_few(wd, nc) && few_rows_supported(wo, nc, d) &&
+                             few_rows_supported(wd, nc, I);
+        if (!out_pair && !exact_out && !few_out && (rc = project(wd, M, I, nc, D, d, &sd, true, pd_splits))) return rc;
         if (use_flash) {
           TRY_HIP(launch_flash_prefill(dims, kv[l], Q, d_rows, longest, A, stream, nullptr, nullptr, &b.kv[l], pfx, 0, 0,
                                        b.segs, (int)seg.size() - 1),
@@ -1585,6 +1594,8 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
           STAGE(ST_PREFILL_GEMM, launch_kq_stage_pair(A, d, d, sa, M, I, I, sm, nc, stream), "staging");
           const KqProduct po{wo, sa, P, d, sp, 0}, pm{wd, sm, D, d, sd, 0};
           STAGE(ST_PREFILL_GEMM, launch_kq_rows_pair(po, pm, nc, stream), "projection");
+        } else if (few_out) {
+          if ((rc = few_out_products(wo, wd, nc, pd_splits, &sp, &sd))) return rc;
         } else if ((rc = exact_out ? exact_out_products(wo, wd, nc, pd_splits, &sp, &sd)
                                    : project(wo, A, d, nc, P, d, &sp, true, pd_splits))) {
           return rc;

@@ -16,9 +16,10 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 
 __global__ void embed_kernel(MatDesc emb, const int *ids, float *x) {
-  const int j = blockIdx.x;
-  const int64_t row = ids[j];
-  for (int c = threadIdx.x; c < emb.cols; c += blockDim.x) x[(int64_t)j * emb.cols + c] = mat_value(emb, row, c);
+  // one value a thread: a loop over the row waited for each value's bytes in
+  // turn (11 us for 18 rows of 2816)
+  const int j = blockIdx.x, c = blockIdx.y * blockDim.x + threadIdx.x;
+  if (c < emb.cols) x[(int64_t)j * emb.cols + c] = mat_value(emb, ids[j], c);
 }
 
 // ---------------------------------------------------------------- attention
@@ -269,6 +270,6 @@ hipError_t launch_ln_matvec(const MatDesc &w, const float *ln_w, const float *ln
 }
 
 hipError_t launch_embed(const MatDesc &emb, const int *ids, int n, float *x, hipStream_t st) {
-  hipLaunchKernelGGL(embed_kernel, dim3(n), dim3(256), 0, st, emb, ids, x);
+  hipLaunchKernelGGL(embed_kernel, dim3(n, (emb.cols + 255) / 256), dim3(256), 0, st, emb, ids, x);
   return hipGetLastError();
 }

@@ -195,19 +195,19 @@ __global__ __launch_bounds__(kT) void logprob_kernel(const float *logits, int64_
 // adds nearly every value to one counter: 277 us for 160 rows of 65536,
 // against 103 here (64 float64 exponentials a thread).
 //
-// The count-th largest of the threads' maxima is a lower bound of the
-// count-th largest value (count threads hold one at least as large), so the
-// values from it on are the candidates: about count of them unless many are
-// equal. Past kCand of them, the threshold and then the highest id taken
+// The count-th largest of the maxima of 64 groups of threads is a lower bound
+// of the count-th largest value (count groups hold one at least as large), so
+// the values from it on are the candidates: few more than count unless many
+// are equal (about 300 for count 64). Past kCand of them, the threshold and then the highest id taken
 // among its equals are found by bisection over the registers.
-constexpr int kFew = 64, kCand = 1024;
+constexpr int kFew = kT / 16, kCand = 1024;  // at most as many entries as groups
 
 template <int J>
 __global__ __launch_bounds__(kT) void logprob_few_kernel(const float *logits, int64_t ld, int V, const int *targets,
                                                          int count, double *chosen, int *top_ids, double *top_lp,
                                                          int *bad) {
   __shared__ double red[kT / 64];
-  __shared__ __align__(16) uint32_t tmax[kT];
+  __shared__ uint32_t gmax[kT / 16];
   __shared__ uint32_t wcount[kT / 64], s_bound;
   __shared__ int s_ncand;
   __shared__ uint32_t ckey[kCand];
@@ -262,20 +262,19 @@ __global__ __launch_bounds__(kT) void logprob_few_kernel(const float *logits, in
       mykey = max(mykey, x[j][e]);
       __builtin_amdgcn_sched_barrier(0);
     }
-  tmax[tid] = mykey;
   total = block_sum_d(total, red);
   const double z = best + log(total);
-  // The bound: the thread maximum that fewer than `count` others exceed,
-  // ties by thread, so exactly one thread ranks count - 1 (with fewer
-  // threads holding a value than `count`, it is a key below every value).
-  int above = 0;
-  for (int i = 0; i < kT / 4; i++) {
-    const uint4 t = reinterpret_cast<const uint4 *>(tmax)[i];
-    const uint32_t k[4] = {t.x, t.y, t.z, t.w};
-#pragma unroll
-    for (int e = 0; e < 4; e++) above += k[e] > mykey || (k[e] == mykey && 4 * i + e < tid);
+  // The bound: of the 64 groups' maxima, the one that exactly count - 1 others
+  // precede (larger, or equal and of a lower group).
+  for (int o = 8; o > 0; o >>= 1) mykey = max(mykey, (uint32_t)__shfl_xor((int)mykey, o));
+  if ((tid & 15) == 0) gmax[tid >> 4] = mykey;
+  __syncthreads();
+  if (tid < 64) {
+    const uint32_t k = gmax[tid];
+    int above = 0;
+    for (int i = 0; i < 64; i++) above += gmax[i] > k || (gmax[i] == k && i < tid);
+    if (above == count - 1) s_bound = k;
   }
-  if (above == count - 1) s_bound = mykey;
   __syncthreads();
   uint32_t bound = max(s_bound, 1u), n = 0;
   int last = V;  // of the entries equal to bound, those up to id `last` are candidates
@@ -354,6 +353,9 @@ hipError_t launch_logprobs(const float *logits, int64_t ld, int rows, int vocab,
   int *bad = reinterpret_cast<int *>(scratch);
   if (count <= kFew && vocab <= 4096 * 4) {
     hipLaunchKernelGGL(logprob_few_kernel<4>, dim3(rows), dim3(kT), 0, st, logits, ld, vocab, targets, count, chosen,
+                       top_ids, top_lp, bad);
+  } else if (count <= kFew && vocab <= 4096 * 8) {
+    hipLaunchKernelGGL(logprob_few_kernel<8>, dim3(rows), dim3(kT), 0, st, logits, ld, vocab, targets, count, chosen,
                        top_ids, top_lp, bad);
   } else if (count <= kFew && vocab <= 4096 * 16) {
     hipLaunchKernelGGL(logprob_few_kernel<16>, dim3(rows), dim3(kT), 0, st, logits, ld, vocab, targets, count, chosen,

@@ -227,6 +227,7 @@ struct StableModel {
   bool use_exact(const Matrix &w, int n) const;
   bool norm_planes(int l, int n) const;
   int exact_in_products(const Layer &w, int n, bool split, float **ya, float **ym, int *sa, int *sm);
+  int few_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd);
   int exact_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd);
   bool few_layer(int l, int n) const;
   // The wide-tile in-projection forms its epilogue as a kernel of its own

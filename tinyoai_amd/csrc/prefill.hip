@@ -366,7 +366,8 @@ __global__ void sum_splits_kernel(float *out, const float *p, int sp, int64_t n)
 }
 
 __global__ void copy_kernel(const float *src, float *dst, int n) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) dst[i] = src[i];
 }
 
 struct RowPairs {
@@ -508,6 +509,6 @@ hipError_t launch_gather_rows(const float *x, float *out, int d, const int *src,
 }
 
 hipError_t launch_copy_row(const float *src, float *dst, int n, hipStream_t st) {
-  hipLaunchKernelGGL(copy_kernel, dim3(1), dim3(256), 0, st, src, dst, n);
+  hipLaunchKernelGGL(copy_kernel, dim3((n + 255) / 256), dim3(256), 0, st, src, dst, n);
   return hipGetLastError();
 }
