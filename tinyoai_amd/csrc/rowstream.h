@@ -145,12 +145,92 @@ __device__ __forceinline__ void rows_issue(RowBatch<CPL, R> &b, const LaneChunks
   }
 }
 
+// ---- 5/6-bit chunks against x in registers
+//
+// What bounds these rows is vector instructions (with every value decoded to
+// fp32, about seven a value, the 21504 x 2560 Q5_K launch took 41 us, 0.9
+// TB/s). Here a value costs two and a half (Q4_K) to three and a half: pairs of
+// quants become fp16 numbers q - c by bit operations (q below 0x6400 is the
+// fp16 number 1024 + q; c = 8, 16 or 32, the middle of their range, so the
+// difference is an exact small integer) and feed mixed-precision multiply-adds
+// with fp32 x. With t = sum (q - c) x over a sub-block,
+//   sum (a q - b) x = a t + (c a - b) sum x,   sum (q - 32) a x = a t,
+// where sum x is formed once per chunk (load_x) and a = d scale, b = dmin min
+// are exact; the sums round as often as those over decoded values did.
+typedef _Float16 kq_f16x2 __attribute__((ext_vector_type(2)));
+
+// q (bits 0-5 and 16-21) - C as two fp16 numbers; bits OR'd in from `high`.
+template <int C>
+__device__ __forceinline__ kq_f16x2 kq_pair(uint32_t low, uint32_t high) {
+  const uint32_t v = (low & 0x000F000Fu) | 0x64006400u | high;
+  return __builtin_bit_cast(kq_f16x2, v) - kq_f16x2{(_Float16)(1024.f + C), (_Float16)(1024.f + C)};
+}
+
+template <int F>
+__device__ __forceinline__ float kq_chunk_acc(const uint4 w, uint32_t s, uint2 h, const uint4 mt, int cc,
+                                              const float *x, float xsum, float acc) {
+  constexpr int C = F == FMT_Q6_K ? 32 : F == FMT_Q4_K ? 8 : 16;
+  const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+  // High bits of the pair (j, j + 2) at bits 4 (5) of both halves, for j = 4k
+  // and 4k + 1: words whose halves hold them 2 (4) bits apart, shifted right.
+  uint32_t b0[2], b1[2];  // [values 0-15, 16-31]: Q5: pairs j < 4 and j >= 4; Q6: values 0-7 and 8-15 of the half
+#pragma unroll
+  for (int p = 0; p < 2; p++) {
+    if constexpr (F == FMT_Q6_K) {
+      const uint32_t v = p ? h.y : h.x;
+      b0[p] = ((v << 4) & 0xFFFFu) | v << 16;
+      b1[p] = ((v >> 12) & 0xFFFFu) | (v & 0xFFFF0000u);
+    } else if constexpr (F != FMT_Q4_K) {
+      const uint32_t v = p ? h.x >> 16 : h.x & 0xFFFFu;
+      b0[p] = ((v << 4) & 0xFFFFu) | v << 18;
+      b1[p] = v | (v >> 2) << 16;
+    }
+  }
+  float t[2] = {0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+#pragma unroll
+    for (int p = 0; p < 2; p++)
+#pragma unroll
+      for (int o = 0; o < 2; o++) {  // values 16 p + j and 16 p + j + 2
+        const int j = 4 * k + o;
+        uint32_t high = 0;
+        if constexpr (F == FMT_Q6_K) high = ((j < 8 ? b0[p] : b1[p]) >> (2 * (j & 7))) & 0x00300030u;
+        else if constexpr (F != FMT_Q4_K) high = (j < 4 ? b0[p] >> j : b1[p] >> (j - 4)) & 0x00100010u;
+        const kq_f16x2 q = kq_pair<C>(ws[k] >> (8 * o + 4 * p), high);
+        t[p] = fmaf((float)q.x, x[16 * p + j], t[p]);
+        t[p] = fmaf((float)q.y, x[16 * p + j + 2], t[p]);
+      }
+  // the chunk's constants (kquant_const's values)
+  if constexpr (F == FMT_Q6_K) {
+    const float d = hw_half((uint16_t)s);
+    const uint32_t lo = cc & 2 ? mt.y : mt.x, hi = cc & 2 ? mt.w : mt.z;
+    const uint32_t sc = (cc & 4 ? hi : lo) >> (16 * (cc & 1));
+    acc = fmaf(d * (float)(int8_t)sc, t[0], acc);
+    return fmaf(d * (float)(int8_t)(sc >> 8), t[1], acc);
+  } else {
+    float a, b;
+    if constexpr (F == FMT_Q5_1) {
+      a = hw_half((uint16_t)mt.x);
+      b = fmaf((float)C, a, hw_half((uint16_t)(mt.x >> 16)));
+    } else {
+      const uint32_t sw = cc & 4 ? (mt.w & 0x0F0F0F0Fu) | ((mt.y >> 2) & 0x30303030u) : mt.y & 0x3F3F3F3Fu;
+      const uint32_t mw = cc & 4 ? ((mt.w >> 4) & 0x0F0F0F0Fu) | ((mt.z >> 2) & 0x30303030u) : mt.z & 0x3F3F3F3Fu;
+      const int sh = 8 * (cc & 3);
+      a = hw_half((uint16_t)mt.x) * (float)((sw >> sh) & 255u);
+      b = fmaf((float)C, a, -(hw_half((uint16_t)(mt.x >> 16)) * (float)((mw >> sh) & 255u)));
+    }
+    acc = fmaf(a, t[0] + t[1], acc);
+    return fmaf(b, xsum, acc);
+  }
+}
+
 // Adds one chunk's products with its x values in registers to acc: one
 // chain of fused multiply-adds per row (Q8_0: the chunk's sum times its
 // block scale, fused into acc).
 template <int F>
 __device__ __forceinline__ float reg_chunk_acc(const uint4 w, uint32_t s, uint2 h, const uint4 mt, int cc,
-                                               const float *x, float acc) {
+                                               const float *x, float xsum, float acc) {
   const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
   if constexpr (F == FMT_Q8_0) {
     float a = 0.f;
@@ -182,30 +262,20 @@ __device__ __forceinline__ float reg_chunk_acc(const uint4 w, uint32_t s, uint2 
     for (int k = 0; k < 4; k++) acc = fmaf(__uint_as_float(ws[k]), x[k], acc);
     return acc;
   } else {
-    const KConst k = kquant_const<F>(mt, (uint16_t)s, cc);
-#pragma unroll
-    for (int qd = 0; qd < 4; qd++) {
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const uint32_t byte = (ws[qd] >> (8 * e)) & 255;
-        const int j = 4 * qd + e;
-        acc = fmaf(kquant_value<F>(k, kquant_q<F>(byte, j, h), j), x[j], acc);
-        acc = fmaf(kquant_value<F>(k, kquant_q<F>(byte, j + 16, h), j + 16), x[j + 16], acc);
-      }
-    }
-    return acc;
+    return kq_chunk_acc<F>(w, s, h, mt, cc, x, xsum, acc);
   }
 }
 
 // Adds the batch's rows' products to acc[row].
 template <int F, int CPL, int R>
 __device__ __forceinline__ void rows_consume(const RowBatch<CPL, R> &b, const LaneChunks<CPL> &L,
-                                             const float (&x)[CPL][Fmt<F>::VPC], float (&acc)[R]) {
+                                             const float (&x)[CPL][Fmt<F>::VPC], const float (&xs)[CPL],
+                                             float (&acc)[R]) {
 #pragma unroll
   for (int i = 0; i < R; i++)
 #pragma unroll
     for (int j = 0; j < CPL; j++)
-      acc[i] = reg_chunk_acc<F>(b.w[i][j], b.s[i][j], b.h[i][j], b.mt[i][j], L.cc[j], x[j], acc[i]);
+      acc[i] = reg_chunk_acc<F>(b.w[i][j], b.s[i][j], b.h[i][j], b.mt[i][j], L.cc[j], x[j], xs[j], acc[i]);
 }
 
 // Column slices of a row of `nch` chunks split in two parts at chunk
@@ -302,7 +372,7 @@ __device__ __forceinline__ void stream_rows(const MatDesc &M, int n_units, int s
   const PendingSink<decltype(record)> sink{record};
   const Planes P = make_planes(M);
   const LaneChunks<CPL> L = lane_chunks<F, CPL>(c0, width, lane);
-  float x[CPL][VPC];
+  float x[CPL][VPC], xs[CPL] = {};  // xs (5/6-bit formats but Q6_K): each chunk's sum of x
   auto load_x = [&]() {
 #pragma unroll
     for (int j = 0; j < CPL; j++) {
@@ -311,6 +381,10 @@ __device__ __forceinline__ void stream_rows(const MatDesc &M, int n_units, int s
       } else {
 #pragma unroll
         for (int v = 0; v < VPC; v++) x[j][v] = 0.f;
+      }
+      if constexpr (F == FMT_Q4_K || F == FMT_Q5_K || F == FMT_Q5_1) {
+#pragma unroll
+        for (int v = 0; v < VPC; v++) xs[j] += x[j][v];
       }
     }
   };
@@ -357,7 +431,7 @@ __device__ __forceinline__ void stream_rows(const MatDesc &M, int n_units, int s
       float acc[R];
 #pragma unroll
       for (int i = 0; i < R; i++) acc[i] = 0.f;
-      rows_consume<F, CPL, R>(b[k], L, x, acc);
+      rows_consume<F, CPL, R>(b[k], L, x, xs, acc);
 #pragma unroll
       for (int i = 0; i < R; i++) r[k][i] = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wave_total(acc[i])));
     }
