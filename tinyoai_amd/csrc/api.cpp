@@ -1161,8 +1161,12 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
         if (use_exact(w.win, n) && use_exact(w.win2, n) && gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)) {
           if ((rc = exact_in_products(w, n, norm_planes(l, n), &Ya, &Ym, &sa, &sm))) return rc;
         } else {
-          Ym = Y + (size_t)n * ra;
-          if ((rc = project(w.win, H, d, n, Ya, ra)) || (rc = project(w.win2, H, d, n, Ym, rm))) return rc;
+          // K splits for the epilogue to sum (24 rows of Q6_K q/k/v as one
+          // range on 60 blocks: 68 us)
+          const int room = std::max(1, chunk / n);
+          if ((rc = project(w.win, H, d, n, Ya, ra, &sa, false, room))) return rc;
+          Ym = Y + (size_t)sa * n * ra;
+          if ((rc = project(w.win2, H, d, n, Ym, rm, &sm, false, room))) return rc;
         }
         STAGE(ST_PREFILL_EPILOGUE,
               launch_in_epilogue(da, kv[l], Ya, ra, rope, d_pos0, n, Q, M, stream, nullptr, nullptr, nullptr, sa),
@@ -1186,10 +1190,10 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
         STAGE(ST_PREFILL_GEMM, launch_gemm_in_epilogue(w.win, XH, lo_plane(w.win), n, e, stream),
               "projection + epilogue");
       } else {
-        int sy = 1;  // (5/6-bit and F16 products alone come in K splits here)
+        int sy = 1;
         if ((rc = pin ? project_planes(w.win, XH, lo_plane(w.win), n, Y, win_rows)
                       : project(w.win, norm_planes(l, n) ? nullptr : H, d, n, Y, win_rows,
-                                use_exact(w.win, n) ? &sy : nullptr, false, std::max(1, chunk / n))))
+                                &sy, false, std::max(1, chunk / n))))
           return rc;
         STAGE(ST_PREFILL_EPILOGUE,
               launch_in_epilogue(dims, kv[l], Y, win_rows, rope, d_pos0, n, Q, m32, stream, pd ? MH : nullptr,
