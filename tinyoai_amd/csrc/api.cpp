@@ -998,6 +998,37 @@ int StableModel::few_out_products(const Matrix &wo, const Matrix &wd, int n, int
   return TINYOAI_OK;
 }
 
+// Whether layer l's in-products of n <= 32 rows run on the few-row 5/6-bit
+// kernel, their shared staging of X forming the LayerNorm (the conditions
+// under which project() takes that kernel for each).
+bool StableModel::kq_norm_in_stage(int l, int n) const {
+  const Layer &w = layers[l];
+  return dims.norm == 0 && w.ln_b && dims.d % 256 == 0 && kq_rows_supported(w.win, n) &&
+         (!w.win2.rows || kq_rows_supported(w.win2, n)) &&
+         kq_rows_stage_bytes(dims.d, n) <= (size_t)chunk * std::max(dims.d, dims.inter) * 2;
+}
+
+// Whether the o and down products of n rows run as one launch of few-row
+// 5/6-bit products (each taking that kernel alone too), their inputs, the
+// attention output and m, staged together side by side in XH.
+bool StableModel::kq_out_pair(const Matrix &wo, const Matrix &wd, int n) const {
+  const int d = dims.d, I = dims.inter;
+  const size_t cap = (size_t)chunk * std::max(d, I) * 2, st_a = (kq_rows_stage_bytes(d, n) + 255) / 256 * 256;
+  return kq_pair && n <= 32 && kq_rows_pair_supported(wo.fmt, wd.fmt) && kq_rows_supported(wo, n) &&
+         kq_rows_supported(wd, n) && ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(M)) & 15) == 0 &&
+         d % 4 == 0 && I % 4 == 0 && st_a + kq_rows_stage_bytes(I, n) <= cap;
+}
+int StableModel::kq_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd) {
+  const int d = dims.d, I = dims.inter;
+  uint8_t *sa = reinterpret_cast<uint8_t *>(XH), *sm = sa + (kq_rows_stage_bytes(d, n) + 255) / 256 * 256;
+  *sp = kq_rows_splits(wo, max_splits);
+  *sd = kq_rows_splits(wd, max_splits);
+  STAGE(ST_PREFILL_GEMM, launch_kq_stage_pair(A, d, d, sa, M, I, I, sm, n, stream), "staging");
+  const KqProduct po{wo, sa, P, d, *sp, 0}, pm{wd, sm, D, d, *sd, 0};
+  STAGE(ST_PREFILL_GEMM, launch_kq_rows_pair(po, pm, n, stream), "projection");
+  return TINYOAI_OK;
+}
+
 // Whether layer l takes an n-token chunk through the few-row kernel: fused
 // win and wout of one of its formats.
 bool StableModel::few_layer(int l, int n) const {
@@ -1031,10 +1062,16 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
     oh = planes ? XH : nullptr;
     ol = planes ? XL : nullptr;
   };
+  // Few rows of two 5/6-bit in-products: the LayerNorm is formed in their
+  // staging, and the two run as one launch.
+  auto kq_in_pair = [&](int l) {
+    const Layer &w = layers[l];
+    return kq_pair && n <= 32 && w.win2.rows && kq_rows_pair_supported(w.win.fmt, w.win2.fmt) && kq_norm_in_stage(l, n);
+  };
   // The residual of layer l and the LayerNorm of layer l + 1 in one launch
   // (LayerNorm models); normed: layer l's LayerNorm is already formed.
   auto residual = [&](int l, int sp, int sd) -> int {
-    if (l + 1 < cfg.num_hidden_layers && dims.norm == 0) {
+    if (l + 1 < cfg.num_hidden_layers && dims.norm == 0 && !kq_in_pair(l + 1)) {
       float *out;
       uint16_t *oh, *ol;
       Fp16Planes fp;
@@ -1139,7 +1176,7 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       STAGE(ST_PREFILL_GEMM, launch_gemm_wide(prods, 2, n, omf, 8, stream), "projection");
       if ((rc = residual(l, so, sd))) return rc;
     } else {
-      if (!normed) {
+      if (!normed && !kq_in_pair(l)) {
         float *out;
         uint16_t *oh, *ol;
         Fp16Planes fp;
@@ -1160,6 +1197,15 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
         float *Ya = Y, *Ym = Y;
         if (use_exact(w.win, n) && use_exact(w.win2, n) && gemm_exact_pair_supported(w.win.fmt, w.win2.fmt)) {
           if ((rc = exact_in_products(w, n, norm_planes(l, n), &Ya, &Ym, &sa, &sm))) return rc;
+        } else if (kq_in_pair(l)) {
+          const int room = std::max(1, chunk / n);
+          sa = kq_rows_splits(w.win, room);
+          sm = kq_rows_splits(w.win2, room);
+          Ym = Y + (size_t)sa * n * ra;
+          STAGE(ST_PREFILL_NORM, launch_kq_stage_norm(X, d, n, d, w.ln_w, w.ln_b, dims.eps, XH, stream),
+                "layer_norm + staging");
+          const KqProduct pa{w.win, XH, Ya, ra, sa, 0}, pm{w.win2, XH, Ym, rm, sm, 0};
+          STAGE(ST_PREFILL_GEMM, launch_kq_rows_pair(pa, pm, n, stream), "projection");
         } else {
           // K splits for the epilogue to sum (24 rows of Q6_K q/k/v as one
           // range on 60 blocks: 68 us)
@@ -1202,7 +1248,8 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       }
       int sp = 1, sd = 1;
       const bool exact_out = use_exact(wo, n) && use_exact(wd, n) && gemm_exact_pair_supported(wo.fmt, wd.fmt);
-      if (exact_out) {
+      const bool kq_out = !exact_out && kq_out_pair(wo, wd, n);
+      if (exact_out || kq_out) {
         // with the o product, after the attention
       } else if ((rc = pd ? project_planes(wd, MH, gemm_planes(wd, bf16_acts) == 2 ? ML : nullptr, n, D, d, &sd) : project(wd, M, I, n, D, d, &sd)))
         return rc;
@@ -1216,8 +1263,11 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       else
         STAGE(ST_PREFILL_ATTENTION,
               launch_attention(dims, kv[l], Q, d_pos0, n, start + n - 1, partials, counters, A, stream), "attention");
-      if (exact_out) {
-        if ((rc = exact_out_products(wo, wd, n, kPrefillSplits, &sp, &sd))) return rc;
+      if (exact_out || kq_out) {
+        if ((rc = exact_out ? exact_out_products(wo, wd, n, kPrefillSplits, &sp, &sd)
+                            : kq_out_products(wo, wd, n, (int)std::min<int64_t>(64, (int64_t)kPrefillSplits * chunk / n),
+                                              &sp, &sd)))
+          return rc;
       } else if ((rc = po ? project_planes(wo, XH, lo_plane(wo), n, P, d, &sp) : project(wo, A, d, n, P, d, &sp))) {
         return rc;
       }
@@ -1510,9 +1560,7 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
         // When the in-products run on the few-row kernel, the LayerNorm is
         // formed in their shared staging of X (no LayerNorm launch); the
         // conditions are those under which project() takes that kernel.
-        const bool norm_in_stage = few && dims.norm == 0 && w.ln_b && d % 256 == 0 && kq_rows_supported(w.win, nc) &&
-                                   (!split_in || kq_rows_supported(w.win2, nc)) &&
-                                   kq_rows_stage_bytes(d, nc) <= (size_t)chunk * std::max(dims.d, dims.inter) * 2;
+        const bool norm_in_stage = few && kq_norm_in_stage(l, nc);
         bool staged = false;  // XH holds this layer's staged LayerNorm output
         if (norm_in_stage) {
           TRY_HIP(launch_kq_stage_norm(X, d, nc, d, w.ln_w, w.ln_b, dims.eps, XH, stream), "layer_norm + staging");
@@ -1558,25 +1606,14 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
           }
         } else {
           int sy = 1;
-          if ((rc = project(w.win, H, d, nc, Y, win_rows, few ? &sy : nullptr, true,
-                            (int)(ycap / ((size_t)nc * win_rows)), &staged)))
+          if ((rc = project(w.win, H, d, nc, Y, win_rows, &sy, true, (int)(ycap / ((size_t)nc * win_rows)), &staged)))
             return rc;
           TRY_HIP(launch_in_epilogue(dims, b.kv[l], Y, win_rows, rope, nullptr, nc, Q, M, stream, nullptr, nullptr,
                                      d_rows, sy),
                   "in_epilogue");
         }
         int sp = 1, sd = 1;
-        // Few rows with two K-quant output-side matrices: the attention
-        // output and m staged together after the attention, and the o and
-        // down products as one launch (the conditions under which project()
-        // takes the few-row kernel for each; the two staged inputs side by
-        // side in XH).
-        const size_t cap = (size_t)chunk * std::max(dims.d, dims.inter) * 2;
-        const size_t st_a = (kq_rows_stage_bytes(d, nc) + 255) / 256 * 256;
-        const bool out_pair = kq_pair && few && kq_rows_pair_supported(wo.fmt, wd.fmt) && kq_rows_supported(wo, nc) &&
-                              kq_rows_supported(wd, nc) && (reinterpret_cast<uintptr_t>(A) & 15) == 0 &&
-                              (reinterpret_cast<uintptr_t>(M) & 15) == 0 && d % 4 == 0 && I % 4 == 0 &&
-                              st_a + kq_rows_stage_bytes(I, nc) <= cap;
+        const bool out_pair = kq_out_pair(wo, wd, nc);
         const bool exact_out = !out_pair && use_exact(wo, nc) && use_exact(wd, nc) &&
                                gemm_exact_pair_supported(wo.fmt, wd.fmt);
         const bool few_out = !split_out && use_few(wo, nc) && use_few(wd, nc) && few_rows_supported(wo, nc, d) &&
@@ -1592,12 +1629,7 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
                   "branch attention");
         }
         if (out_pair) {
-          uint8_t *sa = reinterpret_cast<uint8_t *>(XH), *sm = sa + st_a;
-          sp = kq_rows_splits(wo, pd_splits);
-          sd = kq_rows_splits(wd, pd_splits);
-          STAGE(ST_PREFILL_GEMM, launch_kq_stage_pair(A, d, d, sa, M, I, I, sm, nc, stream), "staging");
-          const KqProduct po{wo, sa, P, d, sp, 0}, pm{wd, sm, D, d, sd, 0};
-          STAGE(ST_PREFILL_GEMM, launch_kq_rows_pair(po, pm, nc, stream), "projection");
+          if ((rc = kq_out_products(wo, wd, nc, pd_splits, &sp, &sd))) return rc;
         } else if (few_out) {
           if ((rc = few_out_products(wo, wd, nc, pd_splits, &sp, &sd))) return rc;
         } else if ((rc = exact_out ? exact_out_products(wo, wd, nc, pd_splits, &sp, &sd)

@@ -227,6 +227,9 @@ struct StableModel {
   bool use_exact(const Matrix &w, int n) const;
   bool norm_planes(int l, int n) const;
   int exact_in_products(const Layer &w, int n, bool split, float **ya, float **ym, int *sa, int *sm);
+  bool kq_norm_in_stage(int l, int n) const;
+  bool kq_out_pair(const Matrix &wo, const Matrix &wd, int n) const;
+  int kq_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd);
   int few_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd);
   int exact_out_products(const Matrix &wo, const Matrix &wd, int n, int max_splits, int *sp, int *sd);
   bool few_layer(int l, int n) const;
