@@ -2308,7 +2308,7 @@ static Product plan_product(const Matrix &m, const float *x_dev, int n, bool cap
   Product p;
   auto round256 = [](size_t v) { return (v + 255) / 256 * 256; };
   auto split = [&](int ks, size_t limit = kProductPartialBytes) {
-    while (ks > 1 && (size_t)ks * n * m.rows * 4 > limit) ks--;
+    while (ks > 1 && (size_t)ks * n * m.rows * 4 > std::min(limit, kProductPartialBytes)) ks--;
     p.ks = ks;
     p.partials = ks > 1 ? round256((size_t)ks * n * m.rows * 4) : 0;
   };
@@ -2322,8 +2322,13 @@ static Product plan_product(const Matrix &m, const float *x_dev, int n, bool cap
     p.planes = round256((size_t)n * m.cols * 2 * gemm_planes(m));
     split(gemm_splits(m, n, StableModel::kPrefillSplits));
   } else if (kq_rows_supported(m, n) && (reinterpret_cast<uintptr_t>(x_dev) & 15) == 0 && m.cols % 4 == 0) {
+    // (in splits since 27 blocks for 3475 x 1792 left the chip idle: 3 rows 25
+    // us as one range, 10 so; below 1024 columns the splits' sum costs what
+    // they save; under capture one range, in the scratch it always took)
     p.route = Route::kq;
-    p.planes = kq_rows_stage_bytes(m.cols, n);
+    p.planes = round256(kq_rows_stage_bytes(m.cols, n));
+    split(capturing || m.cols < 1024 ? 1 : kq_rows_splits(m, 32),
+          kProductScratchBytes - std::min(p.planes + 256, kProductScratchBytes));
   } else if (!capturing && gemm_exact_supported(m, n)) {
     p.route = Route::exact;
     p.planes = round256((size_t)n * gemm_exact_ld(m) * 4) + round256((size_t)n * 4);
@@ -2366,7 +2371,7 @@ static hipError_t product_launch(const Product &p, const Matrix &m, const float 
       if (e == hipSuccess) e = launch_gemm_exact(&q, 1, n, p.tall, st);
       break;
     }
-    case Route::kq: return launch_kq_rows(m, x, m.cols, n, out, m.rows, 1, scratch, st);
+    case Route::kq: e = launch_kq_rows(m, x, m.cols, n, y, m.rows, p.ks, scratch, st); break;
     case Route::simt: return launch_gemm(m, x, n, out, st);
   }
   if (e == hipSuccess && p.ks > 1) e = launch_sum_splits(out, y, p.ks, (int64_t)n * m.rows, st);
