@@ -223,7 +223,10 @@ int tinyoai_stablelm_profile(tinyoai_model *m, int32_t enable);
  * zero (the default) keeps two bf16 planes per activation (16 significant
  * bits). Stage 7: grid nonzero (the default) runs the BF16-weight prefill
  * products on wide matrix-core tiles (the o and down products together
- * as K splits of one launch), zero on 128 x 256 tiles (fp32 accumulation
+ * as K splits of one launch), those of 2 to 64 rows of BF16, F16 and Q8_0
+ * layers on the few-row kernel, and F16, F32 and (beyond 32 rows) 5/6-bit
+ * products on the fp32-accurate tiles; zero runs BF16 and Q8_0 on 128 x 256
+ * tiles and the rest as they ran without those kernels (fp32 accumulation
  * either way; the sums' order differs). Stage 8: grid nonzero forms the wide-tile in-projection's
  * epilogue in the product's own launch, zero (the default) as a kernel of
  * its own (same arithmetic). Stage 9: grid nonzero (the default) splits a
@@ -261,9 +264,10 @@ int tinyoai_llama_close(tinyoai_model *m);  /* Close (mlx_llama.go:34) */
  * switch, like tinyoai_stablelm_set_launch). Stage 0: value nonzero (the
  * default where the model fits: dim 64, 8 query / 4 kv heads, MLP 172, at
  * most 8 layers, 512 positions and a 512-token vocabulary, the stories260K
- * shape) runs every token of a forward call in one launch of one
- * workgroup; zero runs five kernels per layer and token. The sums' order
- * differs between the two. Returns 0, or TINYOAI_EINVAL for another stage,
+ * shape) runs a token in one launch of one workgroup and several tokens of
+ * a call side by side, a workgroup each, in a launch per layer; zero runs
+ * five kernels per layer and token. The sums' order differs between the
+ * two choices. Returns 0, or TINYOAI_EINVAL for another stage,
  * or for value nonzero on a model of another shape. */
 int tinyoai_llama_set_launch(tinyoai_model *m, int32_t stage, int32_t value);
 
@@ -277,7 +281,9 @@ int tinyoai_weight_read_values(tinyoai_weight *w, int64_t offset, int64_t n, flo
  * matmul.go:55-95): out[n][rows] = x[n][cols] * W^T, host buffers. */
 int tinyoai_weight_mul(tinyoai_weight *w, const float *x, int32_t n, float *out);
 /* The same product on device-resident buffers, enqueued on `stream`
- * (a hipStream_t; NULL = the weight's own stream) without synchronizing. */
+ * (a hipStream_t; NULL = the weight's own stream) without synchronizing.
+ * Operand planes and K-split partials live in a buffer per stream that the
+ * weight keeps. */
 int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, float *out_dev, void *stream);
 /* tinyoai_weight_mul_device without any allocation, for callers that
  * cannot allocate (code under HIP graph capture, tight serving loops,

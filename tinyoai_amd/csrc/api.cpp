@@ -1382,9 +1382,11 @@ int Branches::grow(int need) {
   std::vector<KVDev> grown(m->cfg.num_hidden_layers);
   size_t bytes = per * want;
   if (m->spare.kv.size() == 2 * grown.size() && m->spare.kv_bytes >= bytes) {
-    // the previous session's buffers, whole
+    // the previous session's buffers; with room for up to four times the
+    // positions, while the caches stay within 2 GiB (a small session after a
+    // large one addresses no more than it would have grown to)
     bytes = m->spare.kv_bytes;
-    want = (int)std::min<size_t>(max_len, bytes / per);
+    if (4 * per * want <= (size_t)INT32_MAX) want = (int)std::min<size_t>({(size_t)max_len, bytes / per, (size_t)want * 4});
     for (size_t l = 0; l < grown.size(); l++) {
       grown[l].k = m->spare.kv[2 * l];
       grown[l].v = m->spare.kv[2 * l + 1];
@@ -2406,6 +2408,15 @@ int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, 
       it = w->scratch.erase(it);
     }
   }
+  // Capture cannot allocate: a call captured on a stream of its own takes the
+  // buffer that an eager call of its size left on another stream.
+  if (capturing && (!w->scratch.count(st) || w->scratch[st].bytes < p.bytes()))
+    for (auto &other : w->scratch)
+      if (other.second.bytes >= p.bytes()) {
+        other.second.captured = true;
+        e = product_launch(p, m, x_dev, n, out_dev, other.second.ptr, st);
+        return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
+      }
   // A stream's scratch grows on demand (the stream is drained before an old
   // buffer is released).
   tinyoai_weight::Scratch &s = w->scratch[st];
