@@ -221,3 +221,44 @@ def test_paired_in_products_match_separate_launches(hip, mlp, attn, count):
     for s, (a, b) in enumerate(zip(*runs)):
         assert np.all(np.isfinite(a)), s
         assert np.array_equal(a, b), s
+
+
+@pytest.mark.parametrize("kv_bits", [16, 32])
+def test_sessions_after_other_sessions(hip, kv_bits):
+    """A session's results do not depend on the sessions before it, whose
+    caches and scratch it may take over: a small one, a larger one and a small
+    one again, each bit for bit as on a model of its own; and after a reset."""
+    config = W.validate_stablelm_config(dict(W.STABLELM_3B, num_hidden_layers=2, vocab_size=512,
+                                             max_position_embeddings=512))
+    tensors = W.synthetic_stablelm(config, W.Q8_0, seed=3)
+    rng = np.random.default_rng(kv_bits)
+    prefix = rng.integers(0, 512, 70).astype(np.int32)
+    cases = [[rng.integers(0, 512, n).astype(np.int32) for n in lengths] for lengths in
+             ([3, 1], [40, 2, 33, 90, 17], [5, 2, 9])]
+    steps = rng.integers(0, 512, (4, 5)).astype(np.int32)
+
+    def model():
+        f = hip.StableLMForwarder(config, tensors)
+        f.set_kv_bits(kv_bits)
+        return f
+
+    def session(f, suffixes):
+        f.forward(0, prefix, want_logits=False)
+        b = f.new_branches(len(prefix), len(suffixes))
+        rows = [b.append(suffixes).copy()] + [b.forward(t[:len(suffixes)]).copy() for t in steps]
+        b.close()
+        return rows
+
+    want = []
+    for c in cases:
+        f = model()
+        want.append(session(f, c))
+        f.close()
+    f = model()
+    for k in (0, 1, 2, 0, 1):
+        for got, w in zip(session(f, cases[k]), want[k]):
+            assert np.array_equal(got, w), k
+    f.reset()
+    for got, w in zip(session(f, cases[2]), want[2]):
+        assert np.array_equal(got, w)
+    f.close()

@@ -118,3 +118,51 @@ def test_no_alloc_calls_on_two_weights_are_ordered():
         w2.close()
         buf.close()
 
+
+@pytest.mark.parametrize("dtype,n", [(W.F16, 5), (W.F16, 80), (W.Q8_0, 20), (W.Q8_0, 80), (W.Q4_K, 9), (W.F32, 40)])
+def test_captured_products(dtype, n):
+    """tinyoai_weight_mul_device under stream capture, on a stream that has
+    made no call (its scratch, where the product needs any, is what an eager
+    call on another stream left): replays with new inputs, eager calls between
+    them, against float64."""
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    rows, cols = 300, 1280
+    v = rng.standard_normal((rows, cols), dtype=np.float32) * np.float32(0.02)
+    t = {W.F16: lambda: W.Tensor(W.F16, rows, cols, v.astype(np.float16).reshape(-1).view(np.uint8)),
+         W.F32: lambda: W.Tensor(W.F32, rows, cols, v.reshape(-1).view(np.uint8)),
+         W.Q8_0: lambda: W.synthetic_q8_0(rows, cols, rng),
+         W.Q4_K: lambda: W.synthetic_kquant(W.Q4_K, rows, cols, rng)}[dtype]()
+    buf = DeviceBuffers()
+    rt, w = buf.rt, hip.Weight(t)
+    dense = w.read_values(0, rows * cols).reshape(rows, cols).astype(np.float64)
+    st, graph, ex = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    try:
+        x = buf.upload(np.zeros((n, cols), np.float32))
+        y, y2 = buf.alloc(n * rows * 4), buf.alloc(n * rows * 4)
+        w.mul_device(x, n, y)  # eager, on the weight's own stream
+        assert rt.hipDeviceSynchronize() == 0
+        assert rt.hipStreamCreateWithFlags(C.byref(st), 1) == 0
+        assert rt.hipStreamBeginCapture(st, 2) == 0  # relaxed: other threads may call the runtime
+        w.mul_device(x, n, y, st.value)
+        assert rt.hipStreamEndCapture(st, C.byref(graph)) == 0
+        assert rt.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+        for _ in range(3):
+            a = rng.standard_normal((n, cols)).astype(np.float32)
+            assert rt.hipMemcpy(C.c_void_p(x), a.ctypes.data, a.nbytes, 1) == 0
+            assert rt.hipGraphLaunch(ex, st) == 0 and rt.hipStreamSynchronize(st) == 0
+            got = buf.download(y, (n, rows))
+            w.mul_device(x, n, y2)
+            eager = buf.download(y2, (n, rows))
+            want, mag = a.astype(np.float64) @ dense.T, np.abs(a).astype(np.float64) @ np.abs(dense).T
+            for r in (got, eager):  # 2^-16: bf16 planes of Q8_0 beyond 64 rows; the rest is closer
+                assert np.all(np.abs(r - want) <= 2.0 ** -16 * mag)
+    finally:
+        if ex.value:
+            rt.hipGraphExecDestroy(ex)
+        if graph.value:
+            rt.hipGraphDestroy(graph)
+        if st.value:
+            rt.hipStreamDestroy(st)
+        w.close()
+        buf.close()

@@ -193,7 +193,7 @@ __global__ __launch_bounds__(kT) void logprob_kernel(const float *logits, int64_
 // once, into registers (J float4 a thread). The kernel above reads it eight
 // times, twice with a stride between lanes, and its first histogram pass
 // adds nearly every value to one counter: 277 us for 160 rows of 65536,
-// against 103 here (64 float64 exponentials a thread).
+// against 56 here (64 float64 exponentials a thread).
 //
 // The count-th largest of the maxima of 64 groups of threads is a lower bound
 // of the count-th largest value (count groups hold one at least as large), so
