@@ -1279,9 +1279,10 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
       TRY_HIP(launch_copy_row(M + (size_t)(n - 1) * I, trace_gate + (size_t)l * I, I, stream), "trace");
     }
   }
+  bool have_logits = false;
   if (scoring.targets)
-    if (int rc = score_rows(n)) return rc;
-  if (want_logits) {
+    if (int rc = score_rows(n, want_logits ? &have_logits : nullptr)) return rc;
+  if (want_logits && !have_logits) {
     TRY_HIP(launch_copy_row(X + (size_t)(n - 1) * d, x, d, stream), "last row");
     STAGE(ST_LM_HEAD, launch_ln_matvec(head.desc, norm_w, norm_b, dims.eps, 0, x, logits_dev, grid_head, threads_head, stream),
           "lm_head");
@@ -1317,7 +1318,11 @@ void Branches::free_kv() {
 
 // Every row of the chunk through the final LayerNorm and the classifier,
 // in batches that fit the product buffer Y, then its log probabilities.
-int StableModel::score_rows(int n) {
+// `last` asks for the last row in logits_dev: the batch's product gives it
+// where it is fp32-accurate (55 us of the one-row classifier at 65536 entries
+// of F16); two bf16 planes are less than the one-row product holds, and leave
+// *last false.
+int StableModel::score_rows(int n, bool *last) {
   const int d = dims.d, V = cfg.vocab_size;
   TRY_HIP(launch_layer_norm_rows(X, norm_w, norm_b, dims.eps, n, d, H, stream), "final norm");
   const int per = (int)std::max<int64_t>(1, (int64_t)chunk * win_rows / V);
@@ -1329,6 +1334,10 @@ int StableModel::score_rows(int n) {
     TRY_HIP(launch_logprobs(Y, V, nr, V, scoring.targets + row, scoring.count, scoring.chosen + row,
                             scoring.top_ids + row * c, scoring.top_lp + row * c, scoring.scratch, stream),
             "log probabilities");
+    if (last && r0 + nr == n && use_exact(head.desc, nr)) {
+      TRY_HIP(launch_copy_row(Y + (size_t)(nr - 1) * V, logits_dev, V, stream), "last row's logits");
+      *last = true;
+    }
   }
   scoring.row += n;
   return TINYOAI_OK;

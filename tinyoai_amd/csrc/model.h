@@ -257,7 +257,7 @@ struct StableModel {
   } scoring;
   void *score_mem = nullptr;
   size_t score_bytes = 0;
-  int score_rows(int n);
+  int score_rows(int n, bool *last);
   int forward_logprobs(int prefix, const int32_t *tokens, const int32_t *targets, int n, int count, float *logits,
                        double *chosen, int32_t *top_ids, double *top_lp);
   int forward(int prefix, const int32_t *tokens, int n, bool want_logits, float *logits);
