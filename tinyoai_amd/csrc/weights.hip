@@ -78,7 +78,10 @@ __global__ __launch_bounds__(256) void row_scales_kernel(MatDesc m, float *rscal
   if (threadIdx.x) return;
   most = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
   if (most >= 0x7f800000) atomicOr(flag, 1u);
-  const int e = min(max((most >> 23) - 127, -112), 127);
+  // A row of zeros takes 1: its blocks' constants are scaled too, and a large
+  // scale would take those of a 5/6-bit row (any size: zero is a d - b) past
+  // the range. Values that are not zero are no smaller than 2^-24 there.
+  const int e = most ? min(max((most >> 23) - 127, -112), 127) : 14;
   if (rscale) rscale[row] = __int_as_float((127 + 14 - e) << 23);
 }
 
