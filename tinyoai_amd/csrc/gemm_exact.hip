@@ -335,14 +335,13 @@ __device__ __forceinline__ void exact_body(const ExactArgs &g, const ExactProduc
 
   // D fragment: lane holds column lane % 32 of rows (v / 4) * 8 + (lane / 32) * 4 + v % 4.
   float *y = P.y + (int64_t)split * P.split_stride;
-  float uw[NW];
+  // Both factors as one exponent: a total of 1e36 times X's factor alone may
+  // pass the range before the weights' brings it back.
+  int ew[NW];
 #pragma unroll
   for (int j = 0; j < NW; j++) {
-    uw[j] = 1.f;
-    if constexpr (WF != FMT_F16) {
-      const float r = P.w.rscale[min(n0 + brow + j * 32, N - 1)];  // 2^e with |e| <= 126: 2^-e by its exponent field
-      uw[j] = __uint_as_float((254u << 23) - __float_as_uint(r));
-    }
+    ew[j] = 0;
+    if constexpr (WF != FMT_F16) ew[j] = 127 - (int)(__float_as_uint(P.w.rscale[min(n0 + brow + j * 32, N - 1)]) >> 23);
   }
 #pragma unroll
   for (int f = 0; f < WM; f++)
@@ -350,11 +349,11 @@ __device__ __forceinline__ void exact_body(const ExactArgs &g, const ExactProduc
     for (int v = 0; v < 16; v++) {
       const int m = m0 + wm * 32 * WM + f * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
       if (m >= g.M) continue;
-      const float ux = P.unscale[m];
+      const int ex = (int)(__float_as_uint(P.unscale[m]) >> 23) - 127;
 #pragma unroll
       for (int j = 0; j < NW; j++) {
         const int c = n0 + brow + j * 32;
-        if (c < N) y[(int64_t)m * P.ldy + c] = acc[f][j][v] * ux * uw[j];
+        if (c < N) y[(int64_t)m * P.ldy + c] = __builtin_ldexpf(acc[f][j][v], ex + ew[j]);
       }
     }
 }
