@@ -69,3 +69,111 @@ def test_rows_of_any_size(fmt, n):
     assert np.abs(want).max() > 1e36 and np.abs(want).max() < 3e38
     # 22 bits of each operand and 96 sums of 24; a total below 2^-126 in steps of 2^-149
     assert np.all(np.abs(got - want) <= (3 * 2.0 ** -22 + 96 * 2.0 ** -24) * mag + 2.0 ** -148)
+
+
+def _same_kind(got, want):
+    """NaN where want is, infinities where want has them and of their sign."""
+    return (np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want)) and
+            np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)])))
+
+
+@pytest.mark.parametrize("fmt,n", [(W.F32, 5), (W.F32, 300)] + [(f, n) for f in KQUANTS + (W.F16,) for n in (40, 300)])
+def test_infinite_rows(fmt, n):
+    """An infinity or NaN in a row of X gives what fp32 products and sums give,
+    and leaves the other rows alone: with a column of weights that are zero
+    (F32, F16), with weights of both signs, and beside another infinity."""
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    rows, cols = 300, 768
+    t = _tensor(fmt, rows, cols, rng)
+    if fmt in (W.F32, W.F16):
+        t.data.view(np.float32 if fmt == W.F32 else np.float16).reshape(rows, cols)[:, 11] = 0
+    w = hip.Weight(t)
+    dense = w.read_values(0, rows * cols).reshape(rows, cols).astype(np.float64)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    want = x.astype(np.float64) @ dense.T
+    x[0, 7], x[1, 600], x[2, 11], x[3, 9] = np.inf, -np.inf, np.inf, np.nan
+    x[4, 70], x[4, 71] = np.inf, -np.inf
+    x[n - 1, cols - 1], x[n - 1, 0] = -np.inf, 3e38
+    got = w.mul(x)
+    w.close()
+    special = [0, 1, 2, 3, 4, n - 1]
+    with np.errstate(invalid="ignore", over="ignore"):
+        for r in special:
+            want[r] = (x[r].astype(np.float64) * dense).sum(1)
+            assert _same_kind(got[r], want[r]), r
+    rest = np.setdiff1d(np.arange(n), special)
+    mag = np.abs(x[rest].astype(np.float64)) @ np.abs(dense).T
+    assert np.all(np.abs(got[rest] - want[rest]) <= (3 * 2.0 ** -22 + 128 * 2.0 ** -24) * mag)
+
+
+@pytest.mark.parametrize("fmt,n", [(W.F32, 3), (W.F32, 70), (W.F32, 257), (W.F16, 65), (W.F16, 300), (W.Q6_K, 40),
+                                   (W.Q6_K, 300)])
+def test_values_beside_an_outlier(fmt, n):
+    """Rows of X with values up to 1e20 times the rest, where every weight
+    is zero, keep the precision of the rest (the bound has no term of the
+    row's largest value); rows of every size at once too, and only some rows
+    of a tile."""
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    rows, cols, col = 300, 1024, 9
+    t = _tensor(fmt, rows, cols, rng)
+    if fmt == W.Q6_K:  # quant 32: value 0
+        b = t.data.reshape(-1, 210)
+        b[:, col] &= 0xF0
+        b[:, 128 + col] = (b[:, 128 + col] & 0xFC) | 2
+    else:
+        t.data.view(np.float32 if fmt == W.F32 else np.float16).reshape(rows, cols)[:, col::256] = 0
+    w = hip.Weight(t)
+    dense = w.read_values(0, rows * cols).reshape(rows, cols).astype(np.float64)
+    assert not np.any(dense[:, col::256])
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[:, col::256] = 10.0 ** rng.uniform(0, 20, (n, 1))
+    x[::3, col::256] = 0
+    x[1] *= 10.0 ** rng.uniform(-15, 15, cols).astype(np.float32)
+    got = w.mul(x)
+    w.close()
+    x64 = x.astype(np.float64)
+    want, mag = x64 @ dense.T, np.abs(x64) @ np.abs(dense).T
+    err = np.abs(got - want)
+    ordinary = np.arange(n) != 1
+    # values of at least 2^-16 of the largest hold 22 bits; the rest of a row
+    # that is not marked err by 2^-39 of the largest, where most are larger
+    # than 2^-16 of it: 2^-22 of their mean
+    assert np.all(err[ordinary] <= (4 * 2.0 ** -22 + 160 * 2.0 ** -24) * mag[ordinary])
+    assert np.all(err[1] <= 2.0 ** -22 * mag[1])
+
+
+@pytest.mark.parametrize("attn,mlp", [(W.F16, W.F16), (W.Q6_K, W.Q4_K)])
+def test_layer_norm_with_an_outlier(attn, mlp):
+    """A LayerNorm whose output has one value of 1e12 beside ordinary ones, at
+    a column where the matrices that take it are zero: the logits are those of
+    the same model with an ordinary value there."""
+    from tinyoai_amd import hip
+    config = W.validate_stablelm_config(dict(W.STABLELM_3B, hidden_size=256, intermediate_size=512, num_attention_heads=4,
+                                             num_key_value_heads=4, num_hidden_layers=2, vocab_size=256,
+                                             max_position_embeddings=512))
+    ids = np.random.default_rng(1).integers(0, 256, 100).astype(np.int32)
+    got = []
+    for size in (1.0, 1e12):
+        tensors = W.synthetic_stablelm(config, mlp, seed=5, attn_dtype=attn)
+        for name, t in tensors.items():
+            if "input_layernorm" in name:
+                v = t.data.view(np.float32)
+                v[9] = size if name.endswith("weight") else 0
+            elif any(k in name for k in ("q_proj", "k_proj", "v_proj", "gate_proj", "up_proj")):
+                if t.dtype == W.F16:
+                    t.data.view(np.float16).reshape(-1, 256)[:, 9] = 0
+                elif t.dtype == W.Q6_K:
+                    b = t.data.reshape(-1, 210)
+                    b[:, 9] &= 0xF0
+                    b[:, 137] = (b[:, 137] & 0xFC) | 2
+                else:  # Q4_K: the sub-block's minimum and the quant are zero
+                    b = t.data.reshape(-1, 144)
+                    b[:, 8] &= 0xC0
+                    b[:, 16 + 9] &= 0xF0
+        f = hip.StableLMForwarder(config, tensors)
+        got.append(f.forward(0, ids))
+        f.close()
+    assert np.all(np.isfinite(got[0])) and np.std(got[0]) > 0
+    assert np.max(np.abs(got[0] - got[1])) <= 1e-5 * np.max(np.abs(got[0]))

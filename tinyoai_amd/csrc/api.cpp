@@ -814,7 +814,7 @@ int StableModel::project(const Matrix &w, const float *x, int ldx, int n, float 
     if (splits) *splits = plan.ks;
     const int ld = gemm_exact_ld(w);
     if (x) STAGE(ST_PREFILL_GEMM, launch_split_f16(x, ldx, w.cols, n, XH, XL, ld, XU, stream), "fp16 split");
-    const ExactProduct p{w, XH, XL, ld, XU, y, ldy, plan.ks, (int64_t)n * ldy};
+    const ExactProduct p{w, x ? x : H, ldx, XH, XL, ld, XU, y, ldy, plan.ks, (int64_t)n * ldy};
     STAGE(ST_PREFILL_GEMM, launch_gemm_exact(&p, 1, n, plan.tall, stream), "projection");
   } else if (gemm_mfma_supported(w)) {
     const bool two = gemm_planes(w, bf16_acts) == 2;
@@ -968,8 +968,8 @@ int StableModel::exact_in_products(const Layer &w, int n, bool split, float **ya
   *ya = Y;
   *ym = Y + (size_t)*sa * n * ra;
   if (!split) STAGE(ST_PREFILL_GEMM, launch_split_f16(H, d, d, n, XH, XL, ld, XU, stream), "fp16 split");
-  const ExactProduct in[2] = {{w.win, XH, XL, ld, XU, *ya, ra, *sa, (int64_t)n * ra},
-                              {w.win2, XH, XL, ld, XU, *ym, rm, *sm, (int64_t)n * rm}};
+  const ExactProduct in[2] = {{w.win, H, d, XH, XL, ld, XU, *ya, ra, *sa, (int64_t)n * ra},
+                              {w.win2, H, d, XH, XL, ld, XU, *ym, rm, *sm, (int64_t)n * rm}};
   STAGE(ST_PREFILL_GEMM, launch_gemm_exact(in, 2, n, plan.tall, stream), "projection");
   return TINYOAI_OK;
 }
@@ -983,8 +983,8 @@ int StableModel::exact_out_products(const Matrix &wo, const Matrix &wd, int n, i
   *sd = plan.ks2;
   STAGE(ST_PREFILL_GEMM, launch_split_f16(A, d, d, n, XH, XL, lo, XU, stream), "fp16 split");
   STAGE(ST_PREFILL_GEMM, launch_split_f16(M, I, I, n, MH, ML, ld, XU + chunk, stream), "fp16 split");
-  const ExactProduct out[2] = {{wo, XH, XL, lo, XU, P, d, *sp, (int64_t)n * d},
-                               {wd, MH, ML, ld, XU + chunk, D, d, *sd, (int64_t)n * d}};
+  const ExactProduct out[2] = {{wo, A, d, XH, XL, lo, XU, P, d, *sp, (int64_t)n * d},
+                               {wd, M, I, MH, ML, ld, XU + chunk, D, d, *sd, (int64_t)n * d}};
   STAGE(ST_PREFILL_GEMM, launch_gemm_exact(out, 2, n, plan.tall, stream), "projection");
   return TINYOAI_OK;
 }
@@ -1054,7 +1054,7 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
     if (norm_planes(l, n)) {
       out = nullptr;
       oh = ol = nullptr;
-      fp = Fp16Planes{XH, XL, gemm_exact_ld(w.win), XU};
+      fp = Fp16Planes{XH, XL, gemm_exact_ld(w.win), XU, H};
       return;
     }
     const bool planes = !few_layer(l, n) && (wide_layer(l) || (!w.win2.rows && gemm_mfma_supported(w.win)));
@@ -2378,7 +2378,7 @@ static hipError_t product_launch(const Product &p, const Matrix &m, const float 
       uint16_t *hi = (uint16_t *)planes, *lo = hi + (size_t)n * ld;
       float *unscale = reinterpret_cast<float *>(planes + ((size_t)n * ld * 4 + 255) / 256 * 256);
       e = launch_split_f16(x, m.cols, m.cols, n, hi, lo, ld, unscale, st);
-      const ExactProduct q{m, hi, lo, ld, unscale, y, m.rows, p.ks, (int64_t)n * m.rows};
+      const ExactProduct q{m, x, m.cols, hi, lo, ld, unscale, y, m.rows, p.ks, (int64_t)n * m.rows};
       if (e == hipSuccess) e = launch_gemm_exact(&q, 1, n, p.tall, st);
       break;
     }

@@ -8,8 +8,9 @@
 // matrix once per slice.
 //
 // Operands: X comes as fp16 hi + lo planes of rows scaled by a power of two
-// (launch_split_f16: 22 bits and more of every value). F16 weights are used
-// as stored. Other formats are decoded once per block to the fp32 values of
+// (Fp16Planes: 22 bits of a value down to 2^-16 of its row's largest; a row
+// that the planes do not serve is marked, and its outputs come from its fp32
+// values). F16 weights are used as stored. Other formats are decoded once per block to the fp32 values of
 // mat_value, scaled by the row's power of two (Matrix::rscale, from the
 // row's largest value) and split into fp16 hi + lo planes; the products are
 // hi hi + lo hi + hi lo. A K step of 32 columns is summed on the matrix
@@ -24,6 +25,7 @@
 #include <algorithm>
 
 #include "gemm_wide.h"
+#include "plain_rows.h"
 
 using namespace tinyoai_gemm;
 
@@ -53,8 +55,8 @@ __global__ __launch_bounds__(256) void split_f16_kernel(const float *x, int64_t 
       v[u] = make_float4(__uint_as_float(w.x), __uint_as_float(w.y), __uint_as_float(w.z), __uint_as_float(w.w));
     }
   };
-  __shared__ int wave_most[4];
-  int most = 0;
+  __shared__ int wave_most[4], wave_vote[4];
+  int most = 0, vote = 0;
   for (int i0 = 0; i0 < k; i0 += U * 1024) {
     load(i0);
 #pragma unroll
@@ -77,11 +79,17 @@ __global__ __launch_bounds__(256) void split_f16_kernel(const float *x, int64_t 
       if (i >= ldo) break;
       uint2 a, b;
       fp16_split4(v[u], s, a, b);
+      vote += (fp16_vote(v[u].x * s) + fp16_vote(v[u].y * s)) + (fp16_vote(v[u].z * s) + fp16_vote(v[u].w * s));
       *reinterpret_cast<uint2 *>(h + i) = a;
       *reinterpret_cast<uint2 *>(l + i) = b;
     }
   }
-  if (threadIdx.x == 0) unscale[row] = inverse;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) vote += __shfl_xor(vote, o);
+  if ((threadIdx.x & 63) == 0) wave_vote[threadIdx.x >> 6] = vote;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    unscale[row] = (wave_vote[0] + wave_vote[1]) + (wave_vote[2] + wave_vote[3]) > 0 ? -inverse : inverse;
 }
 
 template <int WF>
@@ -335,6 +343,7 @@ __device__ __forceinline__ void exact_body(const ExactArgs &g, const ExactProduc
 
   // D fragment: lane holds column lane % 32 of rows (v / 4) * 8 + (lane / 32) * 4 + v % 4.
   float *y = P.y + (int64_t)split * P.split_stride;
+  bool marked = false;
   // Both factors as one exponent: a total of 1e36 times X's factor alone may
   // pass the range before the weights' brings it back.
   int ew[NW];
@@ -349,13 +358,19 @@ __device__ __forceinline__ void exact_body(const ExactArgs &g, const ExactProduc
     for (int v = 0; v < 16; v++) {
       const int m = m0 + wm * 32 * WM + f * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
       if (m >= g.M) continue;
-      const int ex = (int)(__float_as_uint(P.unscale[m]) >> 23) - 127;
+      const int u = __float_as_int(P.unscale[m]), ex = (u >> 23) - 127;
+      marked |= u < 0;
+      if (u < 0) continue;
 #pragma unroll
       for (int j = 0; j < NW; j++) {
         const int c = n0 + brow + j * 32;
         if (c < N) y[(int64_t)m * P.ldy + c] = __builtin_ldexpf(acc[f][j][v], ex + ew[j]);
       }
     }
+  if (!__any(marked)) return;
+  const int mw = m0 + wm * 32 * WM, c0 = n0 + wn * 128;
+  const uint64_t rows = __ballot(lane < 32 * WM && mw + lane < g.M && P.unscale[min(mw + lane, g.M - 1)] < 0.f);
+  plain_rows<WF>(P.w, P.x, P.ldx, rows, mw, c0, min(c0 + 128, N), k_lo * kWK, min(K, k_hi * kWK), y, P.ldy);
 }
 
 template <int WM>
@@ -481,7 +496,7 @@ hipError_t launch_gemm_exact(const ExactProduct *p, int nprod, int M, bool tall,
   g.M = M;
   for (int i = 0; i < nprod; i++) {
     const ExactProduct &q = p[i];
-    if (!gemm_exact_supported(q.w, M) || !q.xh || !q.xl || !q.unscale || !q.y || q.lda < gemm_exact_ld(q.w) ||
+    if (!gemm_exact_supported(q.w, M) || !q.x || q.ldx < q.w.cols || !q.xh || !q.xl || !q.unscale || !q.y || q.lda < gemm_exact_ld(q.w) ||
         q.lda % 8 || ((reinterpret_cast<uintptr_t>(q.xh) | reinterpret_cast<uintptr_t>(q.xl)) & 15) || q.ksplit < 1 ||
         q.ksplit > (q.w.cols + kWK - 1) / kWK || (q.ksplit > 1 && q.split_stride < (int64_t)M * q.ldy))
       return hipErrorInvalidValue;

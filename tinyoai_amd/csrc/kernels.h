@@ -196,13 +196,25 @@ hipError_t launch_embed(const MatDesc &emb, const int *ids, int n, float *x, hip
 // The fp16 operand planes of a row for the fp32-accurate products
 // (launch_split_f16): hi + lo of the row times a power of two that takes its
 // largest finite magnitude (ordered bits: fp16_magnitude) to [2^14, 2^15), so
-// hi + lo hold 22 bits and more and nothing overflows; an infinity or NaN
-// stays in the hi plane alone. unscale[row] is the inverse factor.
+// nothing overflows; an infinity or NaN stays in the hi plane alone.
+// unscale[row] is the inverse factor. hi + lo hold 22 bits of a value down to
+// 2^-16 of the row's largest, and any value to 2^-39 of it. A row that this
+// does not serve is marked by a negative unscale, and its outputs are formed
+// from its fp32 values (plain_rows): one where most of the values that are not
+// zero lie below 2^-16 of the largest, and one with an infinity, whose product
+// with a weight's lo plane would be a NaN or an infinity of the wrong sign.
 struct Fp16Planes {
   uint16_t *hi = nullptr, *lo = nullptr;
   int ld = 0;  // values between rows, zeros past the row
   float *unscale = nullptr;
+  float *rows = nullptr;  // a launch that forms the rows itself leaves the marked ones here (d values each)
 };
+// What a value, scaled, adds to its row's vote; the row is marked if the sum
+// is positive (rows of less than 2^20 values).
+__device__ __forceinline__ int fp16_vote(float scaled) {
+  const int u = __float_as_int(scaled) & 0x7fffffff;
+  return u == 0x7f800000 ? 1 << 21 : u == 0 ? 0 : u < 0x3e800000 ? 1 : -1;  // 2^-2: 2^-16 of 2^14
+}
 __device__ __forceinline__ int fp16_magnitude(float f) {
   const int u = __float_as_int(f) & 0x7fffffff;
   return u < 0x7f800000 ? u : 0;
@@ -359,6 +371,8 @@ hipError_t launch_gemm_wide_in_epilogue(const MatDesc &w, const uint16_t *xh, co
 // y + s * split_stride.
 struct ExactProduct {
   Matrix w;
+  const float *x;  // the rows in fp32 (read where unscale marks them)
+  int64_t ldx;
   const uint16_t *xh, *xl;
   int lda;
   const float *unscale;

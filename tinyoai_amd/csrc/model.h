@@ -204,7 +204,8 @@ struct StableModel {
   // kRowStreamMax rows in another format without a matrix-core path as one
   // row-streaming matvec per row; otherwise every chunk size takes the
   // same arithmetic.
-  // A null x (fp32-accurate products only): its fp16 planes are in XH, XL, XU.
+  // A null x (fp32-accurate products only): its fp16 planes are in XH, XL, XU
+  // and its marked rows in H.
   // staged (few-row 5/6-bit products): in, the workspace already holds
   // this x from the previous product of the same shape; out, it does now.
   int project(const Matrix &w, const float *x, int ldx, int n, float *y, int ldy, int *splits = nullptr,

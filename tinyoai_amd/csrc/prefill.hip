@@ -243,7 +243,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(float *x, const float *p
                                                         float *out, uint16_t *oh, uint16_t *ol, int ldo,
                                                         Fp16Planes fp) {
   __shared__ double red[4];
-  __shared__ int most[4];
+  __shared__ int most[4], votes[4];
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x;
   auto at = [&](int g) { return 4 * (tid + 256 * g); };
@@ -340,15 +340,25 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(float *x, const float *p
   mag = max(max(most[0], most[1]), max(most[2], most[3]));
   float down;
   const float up = fp16_scale(mag, down);
+  int vote = 0;
 #pragma unroll
   for (int g = 0; g < kNormG; g++) {
     if (at(g) >= fp.ld) continue;
     uint2 hi, lo;
     fp16_split4(v[g], up, hi, lo);
+    vote += (fp16_vote(v[g].x * up) + fp16_vote(v[g].y * up)) + (fp16_vote(v[g].z * up) + fp16_vote(v[g].w * up));
     *reinterpret_cast<uint2 *>(fp.hi + row * fp.ld + at(g)) = hi;
     *reinterpret_cast<uint2 *>(fp.lo + row * fp.ld + at(g)) = lo;
   }
-  if (tid == 0) fp.unscale[row] = down;
+  for (int o = 32; o > 0; o >>= 1) vote += __shfl_xor(vote, o);
+  if ((tid & 63) == 0) votes[tid >> 6] = vote;
+  __syncthreads();
+  const bool marked = (votes[0] + votes[1]) + (votes[2] + votes[3]) > 0;
+  if (tid == 0) fp.unscale[row] = marked ? -down : down;
+  if (!marked) return;
+#pragma unroll
+  for (int g = 0; g < kNormG; g++)
+    if (at(g) < d) *reinterpret_cast<float4 *>(fp.rows + row * d + at(g)) = v[g];
 }
 
 __global__ void residual_kernel(float *x, const float *p, int sp, const float *d, int sd, int64_t n) {
@@ -404,7 +414,7 @@ bool norm_rows_ok(int d, std::initializer_list<const void *> ptrs) {
   return norm_rows_planes_ok(d) && !(bits & 15);
 }
 bool fp16_planes_ok(const Fp16Planes &f, int d) {
-  return f.lo && f.unscale && f.ld >= d && f.ld % 4 == 0 && f.ld <= 1024 * kNormG;
+  return f.lo && f.unscale && f.rows && !(reinterpret_cast<uintptr_t>(f.rows) & 15) && f.ld >= d && f.ld % 4 == 0 && f.ld <= 1024 * kNormG;
 }
 }  // namespace
 
