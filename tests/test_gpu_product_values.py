@@ -40,6 +40,8 @@ def test_rows_of_zeros(fmt, n):
 
 
 def _tensor(fmt, rows, cols, rng):
+    if fmt == W.Q8_0:
+        return W.synthetic_q8_0(rows, cols, rng)
     if fmt in (W.Q4_K, W.Q5_K, W.Q6_K):
         return W.synthetic_kquant(fmt, rows, cols, rng)
     if fmt == W.Q5_1:
@@ -108,9 +110,9 @@ def test_infinite_rows(fmt, n):
 
 
 @pytest.mark.parametrize("fmt,n", [(W.F32, 3), (W.F32, 70), (W.F32, 257), (W.F16, 65), (W.F16, 300), (W.Q6_K, 40),
-                                   (W.Q6_K, 300)])
+                                   (W.Q6_K, 300)] + [(f, n) for f in (W.F16, W.Q8_0) for n in (2, 5, 17, 33, 64)])
 def test_values_beside_an_outlier(fmt, n):
-    """Rows of X with values up to 1e20 times the rest, where every weight
+    """Rows of X with values up to 1e60 times the rest, where every weight
     is zero, keep the precision of the rest (the bound has no term of the
     row's largest value); rows of every size at once too, and only some rows
     of a tile."""
@@ -122,6 +124,8 @@ def test_values_beside_an_outlier(fmt, n):
         b = t.data.reshape(-1, 210)
         b[:, col] &= 0xF0
         b[:, 128 + col] = (b[:, 128 + col] & 0xFC) | 2
+    elif fmt == W.Q8_0:
+        t.data.reshape(-1, 34)[::8, 2 + col] = 0
     else:
         t.data.view(np.float32 if fmt == W.F32 else np.float16).reshape(rows, cols)[:, col::256] = 0
     w = hip.Weight(t)
@@ -130,6 +134,8 @@ def test_values_beside_an_outlier(fmt, n):
     x = rng.standard_normal((n, cols)).astype(np.float32)
     x[:, col::256] = 10.0 ** rng.uniform(0, 20, (n, 1))
     x[::3, col::256] = 0
+    x[0] *= 1e-25
+    x[0, col::256] = 1e35  # the rest is 2^-199 of it
     x[1] *= 10.0 ** rng.uniform(-15, 15, cols).astype(np.float32)
     got = w.mul(x)
     w.close()
@@ -139,9 +145,9 @@ def test_values_beside_an_outlier(fmt, n):
     ordinary = np.arange(n) != 1
     # values of at least 2^-16 of the largest hold 22 bits; the rest of a row
     # that is not marked err by 2^-39 of the largest, where most are larger
-    # than 2^-16 of it: 2^-22 of their mean
-    assert np.all(err[ordinary] <= (4 * 2.0 ** -22 + 160 * 2.0 ** -24) * mag[ordinary])
-    assert np.all(err[1] <= 2.0 ** -22 * mag[1])
+    # than 2^-16 of it: 2^-22 of their mean (Q8_0: 16 bits and 2^-22)
+    assert np.all(err[ordinary] <= (4 * 2.0 ** (-16 if fmt == W.Q8_0 else -22) + 160 * 2.0 ** -24) * mag[ordinary])
+    assert np.all(err[1] <= (4 if fmt == W.Q8_0 and n > 2 else 1) * 2.0 ** -22 * mag[1])
 
 
 @pytest.mark.parametrize("attn,mlp", [(W.F16, W.F16), (W.Q6_K, W.Q4_K)])

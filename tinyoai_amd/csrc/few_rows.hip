@@ -17,7 +17,12 @@
 //
 // Operands: F16 and Q8_0 weights take X as fp16 hi + lo planes of the row
 // scaled by a power of two (its largest value in the segment lands in
-// [2^14, 2^15), so hi + lo carry 22 bits and nothing overflows); Q8_0
+// [2^14, 2^15), so nothing overflows, and hi + lo carry 22 bits of a value
+// down to 2^-16 of the largest, 16 down to 2^-22). A row with 256 columns that
+// this does not serve is marked, and its outputs come from its fp32 values
+// (plain_rows): where most of the groups of four values that are not all zero
+// lie below 2^-16 of the segment's largest (Q8_0: 2^-22, since two bf16 planes
+// would carry 16 bits of every value). Q8_0
 // quants are exact in fp16, each quant block's product is formed unscaled
 // and added as acc += d * block. BF16 weights take bf16 hi + lo planes (16
 // bits, as the wide tiles). Each segment's sums are unscaled and added to
@@ -29,6 +34,7 @@
 #include <type_traits>
 
 #include "kernels.h"
+#include "plain_rows.h"
 
 namespace {
 
@@ -106,6 +112,7 @@ template <int WF, int MT>
 __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void few_rows_kernel(FewArgs g) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ uint32_t item_max[kWaves * kItems];
+  __shared__ uint32_t marks[2];  // rows to take from their fp32 values
   __shared__ __align__(16) float unscale[MT * 32];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int b = blockIdx.x, pi = 0;
@@ -243,6 +250,8 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 #pragma unroll
   for (int j = 0; j < kStages; j++) issue(ring[j], kb_lo + j);
   bool first = true;
+  constexpr uint32_t kSmall = (Q8 ? 22u : 16u) << 23;  // 2^22, 2^16 in the bits of a ratio
+  if (WF != FMT_BF16 && tid < 2) marks[tid] = 0;
 #pragma unroll 1
   for (int kb0 = kb_lo; kb0 < kb_hi; kb0 += segb) {
     // X columns [kStep kb0, + seg) of every row -> planes in LDS (zeros past
@@ -274,6 +283,9 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       }
       __syncthreads();
     }
+    uint32_t l4 = lane * 4;
+    if constexpr (MT > 1) asm volatile("" : "+v"(l4));  // (addresses held from segment to segment were spilled)
+    uint32_t small = 0;
 #pragma unroll
     for (int j = 0; j < kItems; j++) {
       const int it = wave + kWaves * j;
@@ -287,6 +299,10 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
         const int e = min(max((int)(m >> 23) - 127, -112), 127);
         s = __uint_as_float((uint32_t)(127 + 14 - e) << 23);
         if (q == 0 && lane == 0) unscale[row] = __uint_as_float((uint32_t)(127 - 14 + e) << 23);
+        // a lane's group of four below kSmall of the largest, but not zero
+        // (0 - 1 is the largest number)
+        const float a = fmaxf(fmaxf(fabsf(xv[j].x), fabsf(xv[j].y)), fmaxf(fabsf(xv[j].z), fabsf(xv[j].w)));
+        small += __float_as_uint(a) - 1 < max(m, kSmall + 1) - kSmall - 1;
       }
       const float f[4] = {xv[j].x * s, xv[j].y * s, xv[j].z * s, xv[j].w * s};
       uint32_t hi[4], lo[4];
@@ -303,10 +319,28 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
           lo[e] = (hi[e] & 0x7c00u) == 0x7c00u ? 0u : __builtin_bit_cast(uint16_t, (_Float16)(f[e] - (float)a));
         }
       }
-      const uint32_t c = (uint32_t)(q * kItem + lane * 4) >> 3;  // the 16-byte chunk of the row's segment
+      const uint32_t c = ((uint32_t)(q * kItem) + l4) >> 3;  // the 16-byte chunk of the row's segment
       uint8_t *d = lds + row * pitch + (c >> 4) * 512 + (((c & 15) ^ (row & 15)) << 4) + (lane & 1) * 8;
       *reinterpret_cast<uint2 *>(d) = make_uint2(hi[0] | hi[1] << 16, hi[2] | hi[3] << 16);
       *reinterpret_cast<uint2 *>(d + 256) = make_uint2(lo[0] | lo[1] << 16, lo[2] | lo[3] << 16);
+    }
+    if constexpr (WF != FMT_BF16) {
+      // Only where some lane's group is that small (hardly ever) they are
+      // counted by item, the values read again: kept until here they would
+      // cost registers.
+      if (__builtin_expect(__any(small), 0)) {
+#pragma unroll 1
+        for (int it = wave; it < items; it += kWaves) {
+          const int row = it / ipr, k = kb0 * kStep + (it - row * ipr) * kItem + lane * 4;
+          const int most = (int)wave_max(lane < ipr ? item_max[row * ipr + lane] : 0u);
+          const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(
+              rx, k < k_end ? (int)(((uint32_t)row * (uint32_t)P.ldx + k) * 4) : (int)kNone, 0, 0);
+          auto mag = [&](uint32_t u, int e) { return k + e < k_end ? (int)(u & 0x7fffffffu) : 0; };
+          const int a = max(max(mag(v.x, 0), mag(v.y, 1)), max(mag(v.z, 2), mag(v.w, 3)));
+          const uint64_t some = __ballot(a > 0), less = __ballot(a > 0 && a < most - (int)kSmall);
+          if (lane == 0 && 2 * __popcll(less) > __popcll(some)) atomicOr(&marks[row >> 5], 1u << (row & 31));
+        }
+      }
     }
     __syncthreads();
     // The segment's batches in rounds of kStages (past the range both
@@ -350,15 +384,35 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       }
   }
   // D fragment: lane holds column lane % 32 of rows (v / 4) * 8 + (lane / 32) * 4 + v % 4.
-  if (n >= N) return;
-  float *y = P.y + (int64_t)split * P.split_stride + n;
+  float *y = P.y + (int64_t)split * P.split_stride;
 #pragma unroll
   for (int mt = 0; mt < MT; mt++)
 #pragma unroll
     for (int v = 0; v < 16; v++) {
       const int m = mt * 32 + (v >> 2) * 8 + h * 4 + (v & 3);
-      if (m < M) y[(int64_t)m * P.ldy] = tot[mt][v];
+      if (m < M && n < N) y[(int64_t)m * P.ldy + n] = tot[mt][v];
     }
+  if constexpr (WF != FMT_BF16) {
+    // (the marks were made before the barrier that ended the last staging)
+    const uint64_t rows = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)marks[1]) << 32 |
+                          (uint32_t)__builtin_amdgcn_readfirstlane((int)marks[0]);
+    if (__builtin_expect(!rows, 1)) return;
+    wait_vmcnt<0>();  // the stores above, which the marked rows' outputs replace
+    asm volatile("" ::: "memory");
+    // The arguments are read again: kept in registers through the loops above
+    // they would not fit beside what those need.
+    const FewArgs *args = reinterpret_cast<const FewArgs *>((const void *)__builtin_amdgcn_kernarg_segment_ptr());
+    asm volatile("" : "+s"(args));
+    int bq = blockIdx.x;
+    asm volatile("" : "+s"(bq));
+    const int first_blocks = args->p[0].ks * ((args->p[0].w.rows + kBlockRows - 1) / kBlockRows);
+    const FewProduct &Q = args->p[bq >= first_blocks];
+    if (bq >= first_blocks) bq -= first_blocks;
+    const int rb = (Q.w.rows + kBlockRows - 1) / kBlockRows, sq = bq / rb, nkq = (Q.w.cols + kStep - 1) / kStep;
+    const int c0 = (bq - sq * rb) * kBlockRows + wave * kTile;
+    plain_rows<WF>(Q.w, Q.x, Q.ldx, rows, 0, c0, min(c0 + kTile, Q.w.rows), (int)((int64_t)nkq * sq / Q.ks) * kStep,
+                   min(Q.w.cols, (int)((int64_t)nkq * (sq + 1) / Q.ks) * kStep), Q.y + (int64_t)sq * Q.split_stride, Q.ldy);
+  }
 }
 
 template <int WF>

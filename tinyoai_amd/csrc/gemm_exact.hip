@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256) void split_f16_kernel(const float *x, int64_t 
       if (i >= ldo) break;
       uint2 a, b;
       fp16_split4(v[u], s, a, b);
-      vote += (fp16_vote(v[u].x * s) + fp16_vote(v[u].y * s)) + (fp16_vote(v[u].z * s) + fp16_vote(v[u].w * s));
+      vote += (fp16_vote(v[u].x, most) + fp16_vote(v[u].y, most)) + (fp16_vote(v[u].z, most) + fp16_vote(v[u].w, most));
       *reinterpret_cast<uint2 *>(h + i) = a;
       *reinterpret_cast<uint2 *>(l + i) = b;
     }

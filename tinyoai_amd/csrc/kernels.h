@@ -209,11 +209,11 @@ struct Fp16Planes {
   float *unscale = nullptr;
   float *rows = nullptr;  // a launch that forms the rows itself leaves the marked ones here (d values each)
 };
-// What a value, scaled, adds to its row's vote; the row is marked if the sum
-// is positive (rows of less than 2^20 values).
-__device__ __forceinline__ int fp16_vote(float scaled) {
-  const int u = __float_as_int(scaled) & 0x7fffffff;
-  return u == 0x7f800000 ? 1 << 21 : u == 0 ? 0 : u < 0x3e800000 ? 1 : -1;  // 2^-2: 2^-16 of 2^14
+// What a value adds to its row's vote (most: the row's fp16_magnitude); the
+// row is marked if the sum is positive (rows of less than 2^20 values).
+__device__ __forceinline__ int fp16_vote(float f, int most) {
+  const int u = __float_as_int(f) & 0x7fffffff;
+  return u == 0x7f800000 ? 1 << 21 : u == 0 ? 0 : u < most - (16 << 23) ? 1 : -1;
 }
 __device__ __forceinline__ int fp16_magnitude(float f) {
   const int u = __float_as_int(f) & 0x7fffffff;

@@ -346,7 +346,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(float *x, const float *p
     if (at(g) >= fp.ld) continue;
     uint2 hi, lo;
     fp16_split4(v[g], up, hi, lo);
-    vote += (fp16_vote(v[g].x * up) + fp16_vote(v[g].y * up)) + (fp16_vote(v[g].z * up) + fp16_vote(v[g].w * up));
+    vote += (fp16_vote(v[g].x, mag) + fp16_vote(v[g].y, mag)) + (fp16_vote(v[g].z, mag) + fp16_vote(v[g].w, mag));
     *reinterpret_cast<uint2 *>(fp.hi + row * fp.ld + at(g)) = hi;
     *reinterpret_cast<uint2 *>(fp.lo + row * fp.ld + at(g)) = lo;
   }
