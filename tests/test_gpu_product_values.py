@@ -150,6 +150,40 @@ def test_values_beside_an_outlier(fmt, n):
     assert np.all(err[1] <= (4 if fmt == W.Q8_0 and n > 2 else 1) * 2.0 ** -22 * mag[1])
 
 
+@pytest.mark.parametrize("n", [40, 300])
+@pytest.mark.parametrize("fmt", (W.F32,) + KQUANTS)
+def test_weights_beside_an_outlier(fmt, n):
+    """Weights of up to 2^36 times the rest, in some rows' last block, where X
+    is zero: the rest of the matrix keeps its precision (the bound has no term
+    of the row's largest weight)."""
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    rows, cols = 300, 1024
+    t = _tensor(fmt, rows, cols, rng)
+    big = slice(rows // 3, None)
+    if fmt == W.F32:
+        t.data.view(np.float32).reshape(rows, cols)[big, -1] = 2.0 ** 30
+    else:
+        per, size = W.BLOCKS[fmt]
+        b = t.data.reshape(rows, cols // per, size)
+        at = {W.Q5_1: [0, 2], W.Q4_K: [0, 2], W.Q5_K: [0, 2], W.Q6_K: [208]}[fmt]
+        for o in at:  # block scales and minima
+            b[:, :-1, o:o + 2] = np.float16(2.0 ** -20).reshape(1).view(np.uint8)
+            b[big, -1, o:o + 2] = np.float16(2.0 ** 15).reshape(1).view(np.uint8)
+    w = hip.Weight(t)
+    dense = w.read_values(0, rows * cols).reshape(rows, cols).astype(np.float64)
+    zero = 1 if fmt == W.F32 else W.BLOCKS[fmt][0]
+    rest = dense[:, :-zero]
+    assert np.abs(dense[big]).max() > 2.0 ** 22 * np.abs(rest).max()
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    x[:, cols - zero:] = 0
+    got = w.mul(x)
+    w.close()
+    x64 = x.astype(np.float64)
+    want, mag = x64 @ dense.T, np.abs(x64) @ np.abs(dense).T
+    assert np.all(np.abs(got - want) <= (3 * 2.0 ** -22 + 160 * 2.0 ** -24) * mag)
+
+
 @pytest.mark.parametrize("attn,mlp", [(W.F16, W.F16), (W.Q6_K, W.Q4_K)])
 def test_layer_norm_with_an_outlier(attn, mlp):
     """A LayerNorm whose output has one value of 1e12 beside ordinary ones, at

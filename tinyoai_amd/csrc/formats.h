@@ -43,7 +43,7 @@ struct MatDesc {
 // MatDesc alone: 16 more bytes of each matrix in the decode kernels' arguments
 // cost a step 0.7%.
 struct Matrix : MatDesc {
-  int32_t special = 0;            // an F16, F32 or 5/6-bit matrix holding an infinity or NaN
+  int32_t special = 0;            // an F16, F32 or 5/6-bit matrix not for the fp16-plane products
   const float *rscale = nullptr;  // F32 and 5/6-bit: per row the power of two that takes its largest value to
                                   // [2^14, 2^15)
 };

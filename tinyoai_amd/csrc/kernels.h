@@ -491,7 +491,9 @@ hipError_t launch_repack(int fmt, const uint8_t *raw, int64_t rows, int64_t cols
 hipError_t launch_place_bytes(const uint8_t *src, int64_t rows, int64_t row_bytes, uint8_t *dst, int64_t dst_stride,
                               int64_t col0b, const RowMap &map, hipStream_t st);
 // The row scales of m (see Matrix::rscale; not for F16) into rscale, and
-// *flag (device memory) nonzero if m holds an infinity or NaN.
+// *flag (device memory) nonzero if m holds an infinity or NaN, or (not for
+// F16) a row that two fp16 planes of one scale do not hold: more than a
+// sixteenth of its values that are not zero below 2^-16 of the largest.
 hipError_t launch_row_scales(const MatDesc &m, float *rscale, unsigned *flag, hipStream_t st);
 hipError_t launch_read_values(const MatDesc &m, int64_t offset, int64_t n, float *out, hipStream_t st);
 

@@ -36,8 +36,10 @@ struct DevMatrix {
   // Once every tensor is placed: the row scales of F32 and 5/6-bit matrices,
   // and whether an F16, F32 or 5/6-bit matrix holds an infinity or NaN (the
   // matrix-core products multiply every weight by both planes of a value,
-  // where an infinite result would become NaN: such a matrix is marked and
-  // keeps to the vector-unit products).
+  // where an infinite result would become NaN), or F32 or 5/6-bit values so
+  // far below their row's largest that its scale leaves them too few bits (an
+  // outlier column, or the smaller of two sections of a row): such a matrix
+  // is marked and keeps to the other products.
   int finish(hipStream_t st);
   // create + place of a whole matrix.
   int upload(int32_t dtype, int64_t rows, int64_t cols, const void *data, uint64_t nbytes, hipStream_t st);

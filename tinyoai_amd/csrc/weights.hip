@@ -75,8 +75,23 @@ __global__ __launch_bounds__(256) void row_scales_kernel(MatDesc m, float *rscal
   __shared__ int waves[4];
   if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = most;
   __syncthreads();
-  if (threadIdx.x) return;
   most = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
+  if (rscale) {
+    // 16 votes for a value below 2^-16 of the row's largest, 1 against for
+    // each that is not zero
+    int vote = 0;
+    for (int c = threadIdx.x; c < m.cols; c += 256) {
+      const int u = __float_as_int(mat_value(m, row, c)) & 0x7fffffff;
+      vote += u == 0 ? 0 : u < most - (16 << 23) ? 15 : -1;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) vote += __shfl_xor(vote, o);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) waves[threadIdx.x >> 6] = vote;
+    __syncthreads();
+    if (threadIdx.x == 0 && (int64_t)waves[0] + waves[1] + waves[2] + waves[3] > 0) atomicOr(flag, 2u);
+  }
+  if (threadIdx.x) return;
   if (most >= 0x7f800000) atomicOr(flag, 1u);
   // A row of zeros takes 1: its blocks' constants are scaled too, and a large
   // scale would take those of a 5/6-bit row (any size: zero is a d - b) past
