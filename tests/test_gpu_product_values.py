@@ -217,3 +217,41 @@ def test_layer_norm_with_an_outlier(attn, mlp):
         f.close()
     assert np.all(np.isfinite(got[0])) and np.std(got[0]) > 0
     assert np.max(np.abs(got[0] - got[1])) <= 1e-5 * np.max(np.abs(got[0]))
+
+
+@pytest.mark.parametrize("fmt,rows,cols,n", [(W.F32, 96, 65536, 70), (W.F32, 64, 16385, 300), (W.F16, 96, 65536, 70),
+                                             (W.Q6_K, 64, 65536, 200), (W.Q4_K, 64, 32768, 400)])
+def test_long_rows(fmt, rows, cols, n):
+    """Rows of many columns round no more than fp32 sums of 512 columns in
+    float64 totals do: 512 products' chain, its error as of a random walk (in
+    the norm: a quarter of sqrt(512) half-ulps of its final size, with a
+    margin of a half)."""
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    w = hip.Weight(_tensor(fmt, rows, cols, rng))
+    dense = w.read_values(0, rows * cols).reshape(rows, cols).astype(np.float64)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    got = w.mul(x)
+    w.close()
+    want = x.astype(np.float64) @ dense.T
+    bound = 1.5 * 0.25 * np.sqrt(512.0) * 2.0 ** -24
+    assert np.linalg.norm(got - want) <= bound * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("n", [2, 5])
+def test_long_rows_of_few(n):
+    """The same of the few-row F16 product, where the matrix alone fills the
+    device and each block takes its rows' whole length."""
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    rows, cols = 65536, 4096
+    v = rng.integers(0, 65536, rows * cols, dtype=np.uint16)
+    v &= 0x8FFF  # sign, two exponents bits and the mantissa
+    v += 0x2000
+    w = hip.Weight(W.Tensor(W.F16, rows, cols, v.view(np.uint8)))
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    got = w.mul(x)[:, ::64]
+    w.close()
+    want = x.astype(np.float64) @ v.reshape(rows, cols)[::64].view(np.float16).astype(np.float64).T
+    bound = 1.5 * 0.25 * np.sqrt(512.0) * 2.0 ** -24
+    assert np.linalg.norm(got - want) <= bound * np.linalg.norm(want)

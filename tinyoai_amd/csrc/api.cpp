@@ -803,14 +803,16 @@ int StableModel::project(const Matrix &w, const float *x, int ldx, int n, float 
                          bool rowstream, int max_splits, bool *staged) {
   if (splits) *splits = 1;
   const bool reuse = staged && *staged;
+  const int room = splits ? std::max(1, max_splits) : 1;
   if (staged) *staged = false;
   if (use_few(w, n) && few_rows_supported(w, n, ldx)) {
     const int ks = splits ? few_rows_splits(w, n, std::max(1, max_splits)) : 1;
     if (splits) *splits = ks;
     const FewProduct p{w, x, ldx, y, ldy, ks, (int64_t)n * ldy};
     STAGE(ST_PREFILL_GEMM, launch_few_rows(&p, 1, n, stream), "projection");
-  } else if (use_exact(w, n) || (!rowstream && w.fmt == FMT_F32 && use_wide && gemm_exact_supported(w, n))) {
-    const ExactPlan plan = gemm_exact_plan(n, w, nullptr, splits ? std::max(1, max_splits) : 1);
+  } else if (use_exact(w, n, room) ||
+             (!rowstream && w.fmt == FMT_F32 && use_wide && gemm_exact_supported(w, n, room))) {
+    const ExactPlan plan = gemm_exact_plan(n, w, nullptr, room);
     if (splits) *splits = plan.ks;
     const int ld = gemm_exact_ld(w);
     if (x) STAGE(ST_PREFILL_GEMM, launch_split_f16(x, ldx, w.cols, n, XH, XL, ld, XU, stream), "fp16 split");
@@ -943,9 +945,10 @@ bool StableModel::use_few(const Matrix &w, int n) const {
 }
 
 // Whether an n-row product takes the fp32-accurate matrix-core kernel: more
-// rows than the few-row kernels (F16: 64, 5/6-bit formats: 32).
-bool StableModel::use_exact(const Matrix &w, int n) const {
-  return use_wide && n > 32 && !use_few(w, n) && gemm_exact_supported(w, n);
+// rows than the few-row kernels (F16: 64, 5/6-bit formats: 32), in up to
+// max_splits K splits.
+bool StableModel::use_exact(const Matrix &w, int n, int max_splits) const {
+  return use_wide && n > 32 && !use_few(w, n) && gemm_exact_supported(w, n, max_splits);
 }
 
 // Whether layer l's LayerNorm of n rows leaves as the fp16 planes of its
@@ -1247,7 +1250,7 @@ int StableModel::prefill_chunk(const int32_t *ids, int n, int start, bool want_l
               "in_epilogue");
       }
       int sp = 1, sd = 1;
-      const bool exact_out = use_exact(wo, n) && use_exact(wd, n) && gemm_exact_pair_supported(wo.fmt, wd.fmt);
+      const bool exact_out = use_exact(wo, n) && use_exact(wd, n, kPrefillSplits) && gemm_exact_pair_supported(wo.fmt, wd.fmt);
       const bool kq_out = !exact_out && kq_out_pair(wo, wd, n);
       if (exact_out || kq_out) {
         // with the o product, after the attention
@@ -1625,7 +1628,7 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
         }
         int sp = 1, sd = 1;
         const bool out_pair = kq_out_pair(wo, wd, nc);
-        const bool exact_out = !out_pair && use_exact(wo, nc) && use_exact(wd, nc) &&
+        const bool exact_out = !out_pair && use_exact(wo, nc) && use_exact(wd, nc, pd_splits) &&
                                gemm_exact_pair_supported(wo.fmt, wd.fmt);
         const bool few_out = !split_out && use_few(wo, nc) && use_few(wd, nc) && few_rows_supported(wo, nc, d) &&
                              few_rows_supported(wd, nc, I);
@@ -2340,13 +2343,14 @@ static Product plan_product(const Matrix &m, const float *x_dev, int n, bool cap
     p.planes = round256(kq_rows_stage_bytes(m.cols, n));
     split(capturing || m.cols < 1024 ? 1 : kq_rows_splits(m, 32),
           kProductScratchBytes - std::min(p.planes + 256, kProductScratchBytes));
-  } else if (!capturing && gemm_exact_supported(m, n)) {
+  } else if (!capturing && gemm_exact_supported(m, n, 32)) {
     p.route = Route::exact;
     p.planes = round256((size_t)n * gemm_exact_ld(m) * 4) + round256((size_t)n * 4);
     // planes and partials together within the no-allocation array
     const ExactPlan plan = gemm_exact_plan(n, m, nullptr, 32);
     p.tall = plan.tall;
     split(plan.ks, kProductScratchBytes - std::min(p.planes + 256, kProductScratchBytes));
+    if (p.ks < gemm_exact_min_splits(m)) p = Product{};  // no room for the splits
   }
   return p;
 }

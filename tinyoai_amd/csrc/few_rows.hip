@@ -25,8 +25,8 @@
 // would carry 16 bits of every value). Q8_0
 // quants are exact in fp16, each quant block's product is formed unscaled
 // and added as acc += d * block. BF16 weights take bf16 hi + lo planes (16
-// bits, as the wide tiles). Each segment's sums are unscaled and added to
-// fp32 totals.
+// bits, as the wide tiles). Each segment's sums (F16: every 1024 columns') are
+// unscaled and added to fp32 totals.
 //
 // K ranges (splits) write partial outputs, split s at y + s * split_stride,
 // which the consumer sums in order.
@@ -243,6 +243,23 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     }
   };
 
+  // The sums so far, unscaled, to the totals.
+  auto fold = [&]() {
+#pragma unroll
+    for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        float4 u = make_float4(1.f, 1.f, 1.f, 1.f);
+        if constexpr (WF != FMT_BF16) u = *reinterpret_cast<const float4 *>(&unscale[mt * 32 + r * 8 + h * 4]);
+        const float us[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          tot[mt][r * 4 + e] = fmaf(acc[mt][r * 4 + e], us[e], tot[mt][r * 4 + e]);
+          acc[mt][r * 4 + e] = 0.f;
+        }
+      }
+  };
+
   const __amdgpu_buffer_rsrc_t rx =
       plane_rsrc(reinterpret_cast<const uint8_t *>(P.x), ((int64_t)(M - 1) * P.ldx + K) * 4);
   const int ipr = g.seg / kItem, items = M * ipr, segb = g.seg / kStep, k_end = min(K, kb_hi * kStep);
@@ -368,20 +385,12 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
           compute(f[u & 1]);
         }
       }
+      // F16: every 1024 columns (the chain of products on the matrix cores,
+      // of 4096 columns, erred by 6.0e-7; so 3.1e-7)
+      if constexpr (WF == FMT_F16 && MT == 1)
+        if ((kb + kStages) * kStep % 1024 == 0 && kb + kStages < nb) fold();
     }
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        float4 u = make_float4(1.f, 1.f, 1.f, 1.f);
-        if constexpr (WF != FMT_BF16) u = *reinterpret_cast<const float4 *>(&unscale[mt * 32 + r * 8 + h * 4]);
-        const float us[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          tot[mt][r * 4 + e] = fmaf(acc[mt][r * 4 + e], us[e], tot[mt][r * 4 + e]);
-          acc[mt][r * 4 + e] = 0.f;
-        }
-      }
+    fold();
   }
   // D fragment: lane holds column lane % 32 of rows (v / 4) * 8 + (lane / 32) * 4 + v % 4.
   float *y = P.y + (int64_t)split * P.split_stride;

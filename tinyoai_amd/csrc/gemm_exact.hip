@@ -454,10 +454,10 @@ hipError_t launch_split_f16(const float *x, int64_t ldx, int k, int rows, uint16
   return hipGetLastError();
 }
 
-bool gemm_exact_supported(const Matrix &w, int M) {
+bool gemm_exact_supported(const Matrix &w, int M, int max_splits) {
   constexpr int64_t kGiB = int64_t(1) << 30;
   const bool fmt = w.fmt == FMT_F16 || ((w.fmt == FMT_F32 || is_kquant(w.fmt)) && w.rscale);
-  return fmt && !w.special && M >= 2 && w.cols >= 2 * kWK && w.vstride % 16 == 0 &&
+  return fmt && !w.special && M >= 2 && gemm_exact_min_splits(w) <= max_splits && w.cols >= 2 * kWK && w.vstride % 16 == 0 &&
          (reinterpret_cast<uintptr_t>(w.vals) & 15) == 0 && (int64_t)w.rows * w.vstride < kGiB &&
          (int64_t)w.rows * w.mstride < kGiB && (int64_t)M * gemm_exact_ld(w) * 2 < kGiB;
 }
@@ -474,7 +474,7 @@ ExactPlan gemm_exact_plan(int M, const MatDesc &a, const MatDesc *b, int max_spl
                   tb = b ? mt * ((b->rows + kBN - 1) / kBN) : 0;
     const int ka = (a.cols + kWK - 1) / kWK, kb = b ? (b->cols + kWK - 1) / kWK : 0;
     // blocks of at most `steps` K steps each, whichever product they work for
-    for (int steps = 8; steps <= std::max({ka, kb, 8}); steps++) {
+    for (int steps = 8; steps <= std::min(std::max({ka, kb, 8}), kExactRun / kWK); steps++) {
       const int sa = std::min((ka + steps - 1) / steps, max_splits);
       const int sb = b ? std::min((kb + steps - 1) / steps, max_splits) : 0;
       const int longest = std::max((ka + sa - 1) / sa, b ? (kb + sb - 1) / sb : 0);
@@ -496,7 +496,7 @@ hipError_t launch_gemm_exact(const ExactProduct *p, int nprod, int M, bool tall,
   g.M = M;
   for (int i = 0; i < nprod; i++) {
     const ExactProduct &q = p[i];
-    if (!gemm_exact_supported(q.w, M) || !q.x || q.ldx < q.w.cols || !q.xh || !q.xl || !q.unscale || !q.y || q.lda < gemm_exact_ld(q.w) ||
+    if (!gemm_exact_supported(q.w, M, q.ksplit) || !q.x || q.ldx < q.w.cols || !q.xh || !q.xl || !q.unscale || !q.y || q.lda < gemm_exact_ld(q.w) ||
         q.lda % 8 || ((reinterpret_cast<uintptr_t>(q.xh) | reinterpret_cast<uintptr_t>(q.xl)) & 15) || q.ksplit < 1 ||
         q.ksplit > (q.w.cols + kWK - 1) / kWK || (q.ksplit > 1 && q.split_stride < (int64_t)M * q.ldy))
       return hipErrorInvalidValue;

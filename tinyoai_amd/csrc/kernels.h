@@ -380,7 +380,15 @@ struct ExactProduct {
   int ldy, ksplit;
   int64_t split_stride;
 };
-bool gemm_exact_supported(const Matrix &w, int M);
+// A K range of one block is at most kExactRun columns: its fp32 totals round
+// once per step of 32, so their error grows with the root of its length, and
+// past 16384 columns it would be more than that of the vector-unit GEMM's
+// 512-column fp32 sums (relative to float64: 2.1e-7 at 16384 and 8.7e-7 at
+// 65536 in one range, against 4.1e-7). Longer rows need the splits that bring
+// them under it.
+constexpr int kExactRun = 16384;
+inline int gemm_exact_min_splits(const MatDesc &w) { return (w.cols + kExactRun - 1) / kExactRun; }
+bool gemm_exact_supported(const Matrix &w, int M, int max_splits = 1);
 bool gemm_exact_pair_supported(int a, int b);
 inline int gemm_exact_ld(const MatDesc &w) { return (w.cols + 31) / 32 * 32; }
 // The tiles of 256 rows (tall) or 128 and the K splits of one product or of

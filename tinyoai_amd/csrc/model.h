@@ -227,7 +227,7 @@ struct StableModel {
   bool use_wide = true;
   bool wide_layer(int l) const;
   bool use_few(const Matrix &w, int n) const;
-  bool use_exact(const Matrix &w, int n) const;
+  bool use_exact(const Matrix &w, int n, int max_splits = 1) const;
   bool norm_planes(int l, int n) const;
   int exact_in_products(const Layer &w, int n, bool split, float **ya, float **ym, int *sa, int *sm);
   bool kq_norm_in_stage(int l, int n) const;
