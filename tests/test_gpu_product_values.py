@@ -255,3 +255,35 @@ def test_long_rows_of_few(n):
     want = x.astype(np.float64) @ v.reshape(rows, cols)[::64].view(np.float16).astype(np.float64).T
     bound = 1.5 * 0.25 * np.sqrt(512.0) * 2.0 ** -24
     assert np.linalg.norm(got - want) <= bound * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("fmt", KQUANTS)
+@pytest.mark.parametrize("cols", [256, 2560, 12288])
+def test_large_values_in_one_row(fmt, cols):
+    """One row times a 5/6-bit matrix, with infinities (what fp32 products and
+    sums give) and values up to 1e38 whose products with small weights are
+    finite, in one lane's chunk and in every one."""
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(cols)
+    rows = 37
+    w = hip.Weight(_tensor(fmt, rows, cols, rng))
+    dense = w.read_values(0, rows * cols).reshape(rows, cols).astype(np.float64)
+    x = rng.standard_normal((1, cols)).astype(np.float32)
+    for at, value in ((7, np.inf), (cols - 1, -np.inf), (40, np.nan)):
+        y = x.copy()
+        y[0, at] = value
+        got = w.mul(y)
+        with np.errstate(invalid="ignore"):
+            assert _same_kind(got[0], (y.astype(np.float64) * dense).sum(1)), (at, value)
+    y = x.copy()
+    y[0, [3, 4]] = np.inf, -np.inf
+    with np.errstate(invalid="ignore"):
+        assert _same_kind(w.mul(y)[0], (y.astype(np.float64) * dense).sum(1))
+    one = x.copy()
+    one[0, cols // 2] = 3e37 / max(1.0, np.abs(dense).max())
+    every = x * np.float32(3e37 / (np.abs(x[0]) * np.abs(dense)).sum(1).max())
+    for y in (one, every):
+        got, y64 = w.mul(y), y.astype(np.float64)
+        want, mag = y64 @ dense.T, np.abs(y64) @ np.abs(dense).T
+        assert np.all(np.abs(got - want) <= (cols / 64 + 64) * 2.0 ** -24 * mag)
+    w.close()

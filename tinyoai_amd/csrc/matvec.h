@@ -124,6 +124,12 @@ __device__ __forceinline__ void x_chunk(const float *src, int len, int c, float 
   }
 }
 
+// Value v of chunk c of the same.
+template <int VPC>
+__device__ __forceinline__ float x_value(const float *src, int len, int c, int v) {
+  return c * VPC + v < len ? src[c * VPC + v] : 0.f;
+}
+
 // The slice partials' LDS (floats) of a launch: units_per_block * slot
 // when the rows span more than one slice.
 template <int F>
@@ -189,12 +195,13 @@ __device__ __forceinline__ void decode_in_body(const InArgs &a, float *lds_raw, 
     row[1] = 2 * u + 1;
   };
   auto xload = [&](int c, float *out) { x_chunk<VPC>(lds, s.d, c, out); };
+  auto xat = [&](int c, int v) { return x_value<VPC>(lds, s.d, c, v); };
   auto noaux = [](int) { return 0.f; };
   auto done = [&](int u, const float (&r)[2][2], const float (&)[2], const auto &out) {
     in_pair_outputs(s, kv, rope_row, pos, u, r[0][0], r[1][0], a.q_out, a.m_out, out);
   };
   stream_rows<F, T, cpl_for<F>(), 2, false, true, 1, false, COH, COH>(W, W.rows / 2, W.chunks, part, pend, rows,
-                                                                  xload, noaux, pre, prologue, done, hook, blocks);
+                                                                  xload, xat, noaux, pre, prologue, done, hook, blocks);
 }
 
 template <int F, int T>
@@ -312,6 +319,9 @@ __global__ __launch_bounds__(T, (F == FMT_Q8_0 ? 3 : 2)) void decode_out_kernel(
     if (c < p.na) x_chunk<VPC>(p.a, p.ka, c, out);
     else x_chunk<VPC>(p.m, p.km, c - p.na, out);
   };
+  auto xat = [&](int c, int v) {
+    return c < p.na ? x_value<VPC>(p.a, p.ka, c, v) : x_value<VPC>(p.m, p.km, c - p.na, v);
+  };
   // The residual x[r] is loaded with the unit's batch, not in done().
   auto aux = [&](int r) { return p.x[r]; };
   auto done = [&](int u, const float (&r)[2][2], const float (&x0)[2], const auto &out) {
@@ -319,7 +329,7 @@ __global__ __launch_bounds__(T, (F == FMT_Q8_0 ? 3 : 2)) void decode_out_kernel(
     if (2 * u + 1 < W.rows) out.f32(p.x + 2 * u + 1, __fadd_rn(__fadd_rn(x0[1], r[1][0]), r[1][1]));
   };
   stream_rows<F, T, cpl_for<F>(), 2, true, false, 0, true, false, false, F == FMT_Q8_0>(
-      W, (W.rows + 1) / 2, p.na, part, pend, rows, xload, aux, [] {}, [] {}, done);
+      W, (W.rows + 1) / 2, p.na, part, pend, rows, xload, xat, aux, [] {}, [] {}, done);
 }
 
 template <int F, int T>
@@ -344,12 +354,13 @@ __global__ __launch_bounds__(T) void ln_matvec_kernel(LnMvArgs a) {
     row[1] = min(2 * u + 1, M.rows - 1);
   };
   auto xload = [&](int c, float *out) { x_chunk<VPC>(lds, cols, c, out); };
+  auto xat = [&](int c, int v) { return x_value<VPC>(lds, cols, c, v); };
   auto noaux = [](int) { return 0.f; };
   auto done = [&](int u, const float (&r)[2][2], const float (&)[2], const auto &out) {
     out.f32(a.out + 2 * (int64_t)u, r[0][0]);
     if (2 * u + 1 < M.rows) out.f32(a.out + 2 * (int64_t)u + 1, r[1][0]);
   };
-  stream_rows<F, T, cpl_for<F>(), 2, false, true, 1, false>(M, (M.rows + 1) / 2, M.chunks, part, pend, rows, xload,
+  stream_rows<F, T, cpl_for<F>(), 2, false, true, 1, false>(M, (M.rows + 1) / 2, M.chunks, part, pend, rows, xload, xat,
                                                             noaux, pre, prologue, done);
 }
 

@@ -156,7 +156,13 @@ __device__ __forceinline__ void rows_issue(RowBatch<CPL, R> &b, const LaneChunks
 // with fp32 x. With t = sum (q - c) x over a sub-block,
 //   sum (a q - b) x = a t + (c a - b) sum x,   sum (q - 32) a x = a t,
 // where sum x is formed once per chunk (load_x) and a = d scale, b = dmin min
-// are exact; the sums round as often as those over decoded values did.
+// are exact; the sums round as often as those over decoded values did, each
+// relative to the quants' range a |q - c| and to |c a - b| (a block's values
+// span its range, so that is their size). An infinity times q - c = 0 would be
+// a NaN, and an infinity in both terms too; and sums of quants times x leave
+// the range 2^5 / a before those of the values do. So x of kBigX and more is
+// left out here and multiplied with the decoded values (big_terms).
+constexpr float kBigX = 0x1p100f;
 typedef _Float16 kq_f16x2 __attribute__((ext_vector_type(2)));
 
 // q (bits 0-5 and 16-21) - C as two fp16 numbers; bits OR'd in from `high`.
@@ -266,6 +272,23 @@ __device__ __forceinline__ float reg_chunk_acc(const uint4 w, uint32_t s, uint2 
   }
 }
 
+// The sum of the lane's products with x of kBigX and more (x_at(c, v): value v
+// of chunk c), row `row` of M decoded value by value: hardly ever run.
+template <int F, int CPL, typename XAt>
+__device__ __forceinline__ float big_terms(const MatDesc &M, int row, const LaneChunks<CPL> &L, XAt x_at) {
+  float acc = 0.f;
+#pragma unroll
+  for (int j = 0; j < CPL; j++) {
+    if (!L.valid[j]) continue;
+#pragma unroll 1
+    for (int v = 0; v < Fmt<F>::VPC; v++) {
+      const float x = x_at(L.cc[j], v);
+      if (fabsf(x) >= kBigX) acc = fmaf(kquant_at<F>(M, row, (int64_t)L.cc[j] * Fmt<F>::VPC + v), x, acc);
+    }
+  }
+  return acc;
+}
+
 // Adds the batch's rows' products to acc[row].
 template <int F, int CPL, int R>
 __device__ __forceinline__ void rows_consume(const RowBatch<CPL, R> &b, const LaneChunks<CPL> &L,
@@ -305,7 +328,8 @@ __host__ __device__ inline void slice_range(const SliceShape &sh, int nch, int s
 // indices < M.rows) through the block; each row's sum comes in two parts,
 // chunks before `split` and from it on (split == M.chunks: one part).
 // Order of work: with XFIRST, `x_load(c, out)` fills the VPC x values of
-// each of the lane's chunks (zeros past the vector); `pre()` issues the
+// each of the lane's chunks (zeros past the vector; `x_at(c, v)` reads value
+// v of chunk c alone, where the 5/6-bit formats need it); `pre()` issues the
 // loads the prologue needs, and with PREWAIT the wave waits for them
 // before any weight load goes out (they are not queued behind the weight
 // stream); the first PRE batches (at most a group); `prologue()`
@@ -327,12 +351,13 @@ __host__ __device__ inline void slice_range(const SliceShape &sh, int nch, int s
 // stores after it waits for nothing else; with NOCARRY no group does (a
 // kernel held to fewer registers).
 template <int F, int T, int CPL, int R, bool XFIRST, bool PREWAIT, int PRE, bool AUX, bool COH = false,
-          bool DRAIN_FIRST = false, bool NOCARRY = false, typename Rows, typename XLoad, typename AuxLoad, typename Pre, typename Prologue, typename Done,
-          typename Hook = void (*)(int)>
+          bool DRAIN_FIRST = false, bool NOCARRY = false, typename Rows, typename XLoad, typename XAt,
+          typename AuxLoad, typename Pre, typename Prologue, typename Done, typename Hook = void (*)(int)>
 __device__ __forceinline__ void stream_rows(const MatDesc &M, int n_units, int split, float *red, PendingStore *pend,
-                                            Rows unit_rows, XLoad x_load, AuxLoad aux_load, Pre pre, Prologue prologue,
+                                            Rows unit_rows, XLoad x_load, XAt x_at, AuxLoad aux_load, Pre pre, Prologue prologue,
                                             Done done, Hook hook = [](int) {}, int blocks = 0) {
   constexpr int VPC = Fmt<F>::VPC, K = kRowGroup;
+  constexpr bool kQuant = F == FMT_Q5_1 || F == FMT_Q4_K || F == FMT_Q5_K || F == FMT_Q6_K;
   // The wave index in a scalar register: everything per wave below (slice,
   // row group, units, whether a batch is real) is then scalar, and so is
   // the choice of buffer descriptor (a per-lane choice would make the
@@ -373,6 +398,7 @@ __device__ __forceinline__ void stream_rows(const MatDesc &M, int n_units, int s
   const Planes P = make_planes(M);
   const LaneChunks<CPL> L = lane_chunks<F, CPL>(c0, width, lane);
   float x[CPL][VPC], xs[CPL] = {};  // xs (5/6-bit formats but Q6_K): each chunk's sum of x
+  bool big = false;  // (5/6-bit formats) some lane's x holds a value of kBigX or more: wave-uniform
   auto load_x = [&]() {
 #pragma unroll
     for (int j = 0; j < CPL; j++) {
@@ -382,10 +408,26 @@ __device__ __forceinline__ void stream_rows(const MatDesc &M, int n_units, int s
 #pragma unroll
         for (int v = 0; v < VPC; v++) x[j][v] = 0.f;
       }
-      if constexpr (F == FMT_Q4_K || F == FMT_Q5_K || F == FMT_Q5_1) {
+    }
+    if constexpr (kQuant) {
+      float most = 0.f;  // (a NaN leaves it as it is, and is one in every product)
+#pragma unroll
+      for (int j = 0; j < CPL; j++)
+#pragma unroll
+        for (int v = 0; v < VPC; v += 2) most = fmaxf(fmaxf(most, fabsf(x[j][v])), fabsf(x[j][v + 1]));
+      big = __any(most >= kBigX);
+      if (__builtin_expect(big, 0)) {
+#pragma unroll
+        for (int j = 0; j < CPL; j++)
+#pragma unroll
+          for (int v = 0; v < VPC; v++) x[j][v] = fabsf(x[j][v]) >= kBigX ? 0.f : x[j][v];
+      }
+    }
+    if constexpr (kQuant && F != FMT_Q6_K) {
+#pragma unroll
+      for (int j = 0; j < CPL; j++)
 #pragma unroll
         for (int v = 0; v < VPC; v++) xs[j] += x[j][v];
-      }
     }
   };
   // This wave's units: local indices rg, rg + RG, ... below nj (wave-uniform
@@ -432,6 +474,14 @@ __device__ __forceinline__ void stream_rows(const MatDesc &M, int n_units, int s
 #pragma unroll
       for (int i = 0; i < R; i++) acc[i] = 0.f;
       rows_consume<F, CPL, R>(b[k], L, x, xs, acc);
+      if constexpr (kQuant) {
+        if (__builtin_expect(big, 0)) {
+          int row[R];
+          unit_rows(unit_of(first_j + k * RG), row);
+#pragma unroll
+          for (int i = 0; i < R; i++) acc[i] += big_terms<F>(M, row[i], L, x_at);
+        }
+      }
 #pragma unroll
       for (int i = 0; i < R; i++) r[k][i] = __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, wave_total(acc[i])));
     }
