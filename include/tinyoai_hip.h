@@ -283,7 +283,13 @@ int tinyoai_weight_mul(tinyoai_weight *w, const float *x, int32_t n, float *out)
 /* The same product on device-resident buffers, enqueued on `stream`
  * (a hipStream_t; NULL = the weight's own stream) without synchronizing.
  * Operand planes and K-split partials live in a buffer per stream that the
- * weight keeps. */
+ * weight keeps (hipStreamPerThread: per thread; streams past eight share one
+ * buffer, their calls one after another), so calls in flight on several
+ * streams do not meet. A call on a capturing stream takes a buffer of its
+ * capture's own, allocated then, which the graph and the executable graphs
+ * made from it hold until they are destroyed; the replays of one executable
+ * graph run one after another, but two executable graphs of one capture share
+ * it. The arithmetic is that of the uncaptured call. */
 int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, float *out_dev, void *stream);
 /* tinyoai_weight_mul_device without any allocation, for callers that
  * cannot allocate (code under HIP graph capture, tight serving loops,

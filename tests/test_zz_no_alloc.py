@@ -166,3 +166,119 @@ def test_captured_products(dtype, n):
             rt.hipStreamDestroy(st)
         w.close()
         buf.close()
+
+
+def _captured(rt, w, st, calls, mode=0):
+    """An executable graph of the calls (x, n, y) captured on st."""
+    graph, ex = C.c_void_p(), C.c_void_p()
+    assert rt.hipStreamBeginCapture(st, mode) == 0
+    for x, n, y in calls:
+        w.mul_device(x, n, y, st.value)
+    assert rt.hipStreamEndCapture(st, C.byref(graph)) == 0
+    assert rt.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+    rt.hipGraphDestroy(graph)
+    return ex
+
+
+@pytest.mark.parametrize("dtype,n,warm", [(W.Q8_0, 48, 64), (W.Q8_0, 80, 0), (W.BF16, 7, 64), (W.F16, 90, 0),
+                                          (W.F32, 33, 0), (W.Q4_K, 9, 32), (W.Q5_K, 70, 0)])
+def test_captured_products_sum_as_eager_ones(dtype, n, warm):
+    """A captured product needs no eager call before it (a larger one may have
+    needed less scratch), in the mode that forbids every thread's allocations,
+    and gives an eager call's bits; two graphs and eager calls on a third
+    stream, all in flight together, do not disturb each other; and a graph
+    captured after others were destroyed."""
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    rows, cols = 700, 2048
+    v = rng.standard_normal((rows, cols), dtype=np.float32) * np.float32(0.02)
+    t = {W.F16: lambda: W.Tensor(W.F16, rows, cols, v.astype(np.float16).reshape(-1).view(np.uint8)),
+         W.F32: lambda: W.Tensor(W.F32, rows, cols, v.reshape(-1).view(np.uint8)),
+         W.BF16: lambda: W.synthetic_bf16(rows, cols, rng), W.Q8_0: lambda: W.synthetic_q8_0(rows, cols, rng)}
+    t = t[dtype]() if dtype in t else W.synthetic_kquant(dtype, rows, cols, rng)
+    buf = DeviceBuffers()
+    rt, w = buf.rt, hip.Weight(t)
+    streams, execs = [C.c_void_p() for _ in range(3)], []
+    try:
+        for st in streams:
+            assert rt.hipStreamCreateWithFlags(C.byref(st), 1) == 0
+        xs = [rng.standard_normal((max(n, warm), cols)).astype(np.float32) for _ in range(3)]
+        x = [buf.upload(a) for a in xs]
+        y = [buf.alloc(max(n, warm) * rows * 4) for _ in range(3)]
+        if warm:
+            w.mul_device(x[0], warm, y[0])
+        execs += [_captured(rt, w, streams[i], [(x[i], n, y[i])] * 2) for i in range(2)]
+        want = []
+        for i in range(3):
+            w.mul_device(x[i], n, y[2])
+            want.append(buf.download(y[2], (n, rows)))
+        mag = np.abs(xs[0][:n]).astype(np.float64) @ np.abs(w.read_values(0, rows * cols)).reshape(rows, cols).T
+        assert np.any(want[0]) and np.all(np.abs(want[0]) <= mag)
+        for round in range(3):
+            for _ in range(10):
+                for i in range(2):
+                    assert rt.hipGraphLaunch(execs[i], streams[i]) == 0
+                w.mul_device(x[2], n, y[2], streams[2].value)
+            for i in range(3):
+                assert np.array_equal(buf.download(y[i], (n, rows)), want[i]), (round, i)
+            rt.hipGraphExecDestroy(execs[round & 1])
+            execs[round & 1] = _captured(rt, w, streams[round & 1], [(x[round & 1], n, y[round & 1])])
+    finally:
+        for ex in execs:
+            rt.hipGraphExecDestroy(ex)
+        for st in streams:
+            rt.hipStreamDestroy(st)
+        w.close()
+        buf.close()
+
+
+@pytest.mark.parametrize("dtype,n", [(W.F16, 70), (W.Q8_0, 20)])
+def test_products_in_flight_on_many_streams(dtype, n):
+    """One weight's products in flight on twelve streams (four of them share a
+    buffer) and on two threads' hipStreamPerThread, sizes growing: every output
+    is that of a call alone."""
+    import threading
+
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    rows, cols = 900, 1536
+    v = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float16)
+    t = W.synthetic_q8_0(rows, cols, rng) if dtype == W.Q8_0 else W.Tensor(W.F16, rows, cols, v.reshape(-1).view(np.uint8))
+    buf = DeviceBuffers()
+    rt, w = buf.rt, hip.Weight(t)
+    streams = [C.c_void_p() for _ in range(12)]
+    try:
+        for st in streams:
+            assert rt.hipStreamCreateWithFlags(C.byref(st), 1) == 0
+        sizes = [n + 3 * i for i in range(4)]
+        x = [buf.upload(rng.standard_normal((sizes[-1], cols)).astype(np.float32)) for _ in range(14)]
+        y = [[buf.alloc(m * rows * 4) for m in sizes] for _ in range(14)]
+        ref = buf.alloc(sizes[-1] * rows * 4)
+        want = []
+        for i in range(14):
+            want.append([])
+            for m in sizes:
+                w.mul_device(x[i], m, ref)
+                want[i].append(buf.download(ref, (m, rows)))
+        for k, m in enumerate(sizes):
+            for i, st in enumerate(streams):
+                w.mul_device(x[i], m, y[i][k], st.value)
+
+        def on_thread(i):
+            rt.hipSetDevice(0)
+            for k, m in enumerate(sizes):
+                w.mul_device(x[i], m, y[i][k], 2)  # hipStreamPerThread
+
+        threads = [threading.Thread(target=on_thread, args=(i,)) for i in (12, 13)]
+        for th in threads:
+            th.start()
+        for th in threads:
+            th.join()
+        for i in range(14):
+            for k, m in enumerate(sizes):
+                assert np.array_equal(buf.download(y[i][k], (m, rows)), want[i][k]), (i, m)
+    finally:
+        for st in streams:
+            rt.hipStreamDestroy(st)
+        w.close()
+        buf.close()

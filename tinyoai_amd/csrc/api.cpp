@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -21,6 +22,7 @@
 
 #include "kernels.h"
 #include "model.h"
+#include "scratch.h"
 
 LaunchTiming &launch_timing() {
   thread_local LaunchTiming t;
@@ -1848,24 +1850,17 @@ struct tinyoai_weight {
   DevMatrix m;
   int device = 0;  // the device the weight lives on
   hipStream_t stream = nullptr;
-  // Operand planes and K-split partials of tinyoai_weight_mul_device, one
-  // buffer per stream it is called on (calls on one stream run in order;
-  // `mu` keeps one call's launches together). At most kStreams of them: with
-  // more, those no captured graph uses are given back. A buffer used under
-  // capture is kept until the weight is closed.
-  struct Scratch {
-    void *ptr = nullptr;
-    size_t bytes = 0;
-    bool captured = false;
-  };
-  static constexpr size_t kStreams = 8;
+  // Operand planes and K-split partials of tinyoai_weight_mul_device: a
+  // buffer per stream (calls on one stream run in order; `mu` keeps one
+  // call's launches together), one that further streams share in turn
+  // (`shared_done`: after its last call), and buffers that captured graphs
+  // own.
   std::mutex mu;
-  std::map<hipStream_t, Scratch> scratch;
-  std::vector<void *> kept;
+  ScratchPool scratch;
+  hipEvent_t shared_done = nullptr;
   ~tinyoai_weight() {
-    for (auto &s : scratch)
-      if (s.second.ptr) hipFree(s.second.ptr);
-    for (void *p : kept) hipFree(p);
+    scratch.clear([](void *p) { hipFree(p); });
+    if (shared_done) hipEventDestroy(shared_done);
     if (stream) hipStreamDestroy(stream);
   }
 };
@@ -2295,20 +2290,17 @@ int tinyoai_weight_read_values(tinyoai_weight *w, int64_t offset, int64_t n, flo
 
 }  // extern "C"
 
-// How a product of n rows runs, and the scratch it needs: partial outputs of
-// `ks` K splits (summed in order), then operand planes. A rule of the shape
-// alone (the partials within kProductPartialBytes), so the allocating and the
-// no-allocation entry points sum alike.
+// How a product of n rows runs, and the scratch it needs: operand planes, then
+// partial outputs of `ks` K splits (summed in order). A rule of the shape and
+// of x's alignment alone (the partials within kProductPartialBytes), so the
+// allocating and the no-allocation entry points sum alike, captured or not.
 //   one row: the row-streaming matvec;
 //   F16, BF16, Q8_0 up to 64 rows: the few-row kernel;
 //   Q8_0, BF16: the large tiles (bf16 planes);
 //   5/6-bit formats up to 32 rows: the few-row product (staged X);
 //   F16, F32, 5/6-bit formats: the fp32-accurate tiles (fp16 planes and the
 //   rows' factors);
-//   else (values that are not finite, very few columns) the vector-unit GEMM.
-// Under capture an F16 product of few rows runs in one range, and a product
-// of the fp32-accurate tiles on the vector-unit GEMM, both of which need no
-// scratch: a graph holds no buffer of theirs that other calls use.
+//   else (matrices that are marked, very few columns) the vector-unit GEMM.
 constexpr size_t kProductPartialBytes = (size_t)32 << 20, kProductScratchBytes = (size_t)48 << 20;
 enum class Route { row, few, mfma, exact, kq, simt };
 struct Product {
@@ -2318,7 +2310,7 @@ struct Product {
   size_t planes = 0, partials = 0;  // bytes
   size_t bytes() const { return planes + partials; }
 };
-static Product plan_product(const Matrix &m, const float *x_dev, int n, bool capturing) {
+static Product plan_product(const Matrix &m, const float *x_dev, int n) {
   Product p;
   auto round256 = [](size_t v) { return (v + 255) / 256 * 256; };
   auto split = [&](int ks, size_t limit = kProductPartialBytes) {
@@ -2330,7 +2322,7 @@ static Product plan_product(const Matrix &m, const float *x_dev, int n, bool cap
     p.route = Route::row;
   } else if (few_rows_supported(m, n, m.cols)) {
     p.route = Route::few;
-    split(capturing && m.fmt == FMT_F16 ? 1 : few_rows_splits(m, n, 64));
+    split(few_rows_splits(m, n, 64));
   } else if (gemm_mfma_supported(m)) {
     p.route = Route::mfma;
     p.planes = round256((size_t)n * m.cols * 2 * gemm_planes(m));
@@ -2338,12 +2330,12 @@ static Product plan_product(const Matrix &m, const float *x_dev, int n, bool cap
   } else if (kq_rows_supported(m, n) && (reinterpret_cast<uintptr_t>(x_dev) & 15) == 0 && m.cols % 4 == 0) {
     // (in splits since 27 blocks for 3475 x 1792 left the chip idle: 3 rows 25
     // us as one range, 10 so; below 1024 columns the splits' sum costs what
-    // they save; under capture one range, in the scratch it always took)
+    // they save)
     p.route = Route::kq;
     p.planes = round256(kq_rows_stage_bytes(m.cols, n));
-    split(capturing || m.cols < 1024 ? 1 : kq_rows_splits(m, 32),
+    split(m.cols < 1024 ? 1 : kq_rows_splits(m, 32),
           kProductScratchBytes - std::min(p.planes + 256, kProductScratchBytes));
-  } else if (!capturing && gemm_exact_supported(m, n, 32)) {
+  } else if (gemm_exact_supported(m, n, 32)) {
     p.route = Route::exact;
     p.planes = round256((size_t)n * gemm_exact_ld(m) * 4) + round256((size_t)n * 4);
     // planes and partials together within the no-allocation array
@@ -2393,6 +2385,23 @@ static hipError_t product_launch(const Product &p, const Matrix &m, const float 
   return e;
 }
 
+namespace {
+// Allowing this thread's allocations while a stream is captured.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  ~RelaxedCapture() {
+    if (set) hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
+// This thread's number, no other's before or after.
+uint64_t thread_number() {
+  static std::atomic<uint64_t> next{1};
+  thread_local const uint64_t number = next++;
+  return number;
+}
+}  // namespace
+
 extern "C" {
 
 int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, float *out_dev, void *stream) try {
@@ -2404,52 +2413,55 @@ int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, 
     e = product_launch(Product{Route::row}, m, x_dev, n, out_dev, nullptr, st);
     return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
   }
-  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if ((e = hipStreamIsCapturing(st, &cap)) != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
-  const bool capturing = cap != hipStreamCaptureStatusNone;
-  const Product p = plan_product(m, x_dev, n, capturing);
+  const Product p = plan_product(m, x_dev, n);
   if (!p.bytes()) {
     e = product_launch(p, m, x_dev, n, out_dev, nullptr, st);
     return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
   }
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  hipGraph_t graph = nullptr;
+  if ((e = hipStreamGetCaptureInfo_v2(st, &cap, &id, &graph, nullptr, nullptr)) != hipSuccess)
+    return hip_fail(e, "hipStreamGetCaptureInfo");
+  auto alloc = [](size_t bytes) {
+    RelaxedCapture relaxed;
+    void *ptr = nullptr;
+    return hipMalloc(&ptr, bytes) == hipSuccess ? ptr : nullptr;
+  };
   std::lock_guard<std::mutex> lock(w->mu);
-  if (!capturing && w->scratch.size() >= tinyoai_weight::kStreams && !w->scratch.count(st)) {
-    if ((e = hipDeviceSynchronize()) != hipSuccess) return hip_fail(e, "product scratch");
-    for (auto it = w->scratch.begin(); it != w->scratch.end();) {
-      if (it->second.captured) w->kept.push_back(it->second.ptr);
-      else hipFree(it->second.ptr);
-      it = w->scratch.erase(it);
-    }
-  }
-  // Capture cannot allocate: a call captured on a stream of its own takes the
-  // buffer that an eager call of its size left on another stream.
-  if (capturing && (!w->scratch.count(st) || w->scratch[st].bytes < p.bytes()))
-    for (auto &other : w->scratch)
-      if (other.second.bytes >= p.bytes()) {
-        other.second.captured = true;
-        e = product_launch(p, m, x_dev, n, out_dev, other.second.ptr, st);
-        return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
+  ScratchPool::Lease lease;
+  if (cap != hipStreamCaptureStatusNone) {
+    ScratchPool::Record *made = nullptr;
+    lease.ptr = w->scratch.captured(id, st, p.bytes(), alloc, &made);
+    hipUserObject_t owner = nullptr;
+    if (made) {  // the graph's, and that of every executable graph made from it
+      e = hipUserObjectCreate(&owner, made, ScratchPool::release, 1, hipUserObjectNoDestructorSync);
+      if (e != hipSuccess) {
+        ScratchPool::release(made);
+        return hip_fail(e, "product scratch");
       }
-  // A stream's scratch grows on demand (the stream is drained before an old
-  // buffer is released).
-  tinyoai_weight::Scratch &s = w->scratch[st];
-  if (p.bytes() > s.bytes) {
-    if (s.ptr && s.captured) {
-      w->kept.push_back(s.ptr);
-    } else if (s.ptr) {
-      hipStreamSynchronize(st);
-      hipFree(s.ptr);
+      if ((e = hipGraphRetainUserObject(graph, owner, 1, hipGraphUserObjectMove)) != hipSuccess) {
+        hipUserObjectRelease(owner, 1);
+        return hip_fail(e, "product scratch");
+      }
     }
-    s = {};
-    e = hipMalloc(&s.ptr, p.bytes());
-    if (e != hipSuccess) {
-      s.ptr = nullptr;
-      return fail(TINYOAI_ENOMEM, "hipMalloc(%zu): %s", p.bytes(), hipGetErrorString(e));
-    }
-    s.bytes = p.bytes();
+  } else {
+    lease = w->scratch.eager(st, st == hipStreamPerThread ? thread_number() : 0, p.bytes(), alloc);
   }
-  s.captured |= capturing;
-  e = product_launch(p, m, x_dev, n, out_dev, s.ptr, st);
+  if (!lease.ptr) return fail(TINYOAI_ENOMEM, "product scratch of %zu bytes", p.bytes());
+  if (lease.shared) {
+    RelaxedCapture relaxed;
+    if (!w->shared_done)
+      e = hipEventCreateWithFlags(&w->shared_done, hipEventDisableTiming);
+    else
+      e = hipStreamWaitEvent(st, w->shared_done, 0);
+    if (e != hipSuccess) return hip_fail(e, "product scratch");
+  }
+  e = product_launch(p, m, x_dev, n, out_dev, lease.ptr, st);
+  if (lease.shared) {  // also after a launch that failed: an earlier one of the call may run
+    const hipError_t r = hipEventRecord(w->shared_done, st);
+    if (e == hipSuccess) e = r;
+  }
   return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "product launch");
 } catch (const std::exception &e) {
   return fail(TINYOAI_ENOMEM, "product: %s", e.what());
@@ -2527,7 +2539,7 @@ int tinyoai_weight_mul_device_noalloc(tinyoai_weight *w, const float *x_dev, int
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if ((e = hipStreamIsCapturing(st, &cap)) != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
   const bool order = cap == hipStreamCaptureStatusNone;
-  const Product p = plan_product(m, x_dev, n, !order);
+  const Product p = plan_product(m, x_dev, n);
   if (p.bytes() > sizeof(scratch))
     return fail(TINYOAI_EINVAL, "product of %d x %d needs more than the no-allocation limit of %zu bytes", n, m.cols,
                 sizeof(scratch));
