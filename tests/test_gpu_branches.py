@@ -262,3 +262,46 @@ def test_sessions_after_other_sessions(hip, kv_bits):
     for got, w in zip(session(f, cases[2]), want[2]):
         assert np.array_equal(got, w)
     f.close()
+
+
+def test_closed_sessions_make_room(hip):
+    """The caches that a closed session leaves with its model go to whoever
+    finds the memory used up: another model's session, with less memory free
+    than it takes."""
+    import ctypes as C
+    config = W.validate_stablelm_config(dict(W.STABLELM_3B, num_hidden_layers=2, vocab_size=512,
+                                             max_position_embeddings=4096))
+    tensors = W.synthetic_stablelm(config, W.Q8_0, seed=3)
+    rng = np.random.default_rng(8)
+    suffixes = [rng.integers(0, 512, n).astype(np.int32) for n in [2000] + [3] * 15]
+    prefix = rng.integers(0, 512, 40).astype(np.int32)
+
+    def session(f):
+        f.forward(0, prefix, want_logits=False)
+        b = f.new_branches(len(prefix), len(suffixes))
+        rows = [b.append(suffixes).copy(), b.forward(np.arange(16, dtype=np.int32)).copy()]
+        b.close()
+        return rows
+
+    a, b = hip.StableLMForwarder(config, tensors), hip.StableLMForwarder(config, tensors)
+    rt, fill = C.CDLL("libamdhip64.so.7"), C.c_void_p()
+    free, total = C.c_size_t(), C.c_size_t()
+    want = session(b)  # (and every kernel of the session has run once)
+    b.reset()
+    assert rt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    before = free.value
+    session(a)
+    assert rt.hipDeviceSynchronize() == 0 and rt.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    kept = before - free.value
+    assert kept > 1 << 30  # 16 branches of 2048 positions: 1.3 GB, and a's own cache
+    try:
+        assert rt.hipMalloc(C.byref(fill), C.c_size_t(free.value - (768 << 20))) == 0
+        got = session(b)  # 1.3 GB of 0.75
+    finally:
+        rt.hipFree(fill)
+    for x, y in zip(got, want):
+        assert np.array_equal(x, y)
+    for x, y in zip(session(a), want):  # a's next one allocates again
+        assert np.array_equal(x, y)
+    a.close()
+    b.close()

@@ -114,6 +114,81 @@ static void kquant_repack_row(int fmt, const uint8_t *raw, int64_t cols, uint8_t
   }
 }
 
+// ---------------------------------------------------------------- device memory
+// Every model's kept buffers, and the lock of what they hold (neither is ever
+// destroyed: a model may be closed while the process ends).
+static std::mutex &kept_mutex() {
+  static std::mutex &m = *new std::mutex;
+  return m;
+}
+static std::vector<KeptBuffers *> &kept_list() {
+  static std::vector<KeptBuffers *> &l = *new std::vector<KeptBuffers *>;
+  return l;
+}
+KeptBuffers::KeptBuffers() {
+  std::lock_guard<std::mutex> lock(kept_mutex());
+  kept_list().push_back(this);
+}
+KeptBuffers::~KeptBuffers() {
+  std::lock_guard<std::mutex> lock(kept_mutex());
+  auto &l = kept_list();
+  l.erase(std::find(l.begin(), l.end(), this));
+  held.release();
+}
+void KeptBuffers::keep(BranchBuffers b) {
+  std::lock_guard<std::mutex> lock(kept_mutex());
+  held.release();
+  size_t total = b.cache_bytes();
+  for (const KeptBuffers *k : kept_list()) total += k->held.cache_bytes();
+  if (total > kMost) b.release_kv();
+  held = std::move(b);
+}
+std::vector<void *> KeptBuffers::take_kv(size_t count, size_t *bytes) {
+  std::lock_guard<std::mutex> lock(kept_mutex());
+  std::vector<void *> kv;
+  if (held.kv.size() == count && held.kv_bytes >= *bytes) {
+    *bytes = std::exchange(held.kv_bytes, 0);
+    kv.swap(held.kv);
+  } else {
+    held.release_kv();
+  }
+  return kv;
+}
+BranchBuffers KeptBuffers::take_scratch() {
+  std::lock_guard<std::mutex> lock(kept_mutex());
+  BranchBuffers b = std::exchange(held, BranchBuffers());
+  held.kv.swap(b.kv);
+  held.kv_bytes = std::exchange(b.kv_bytes, 0);
+  return b;
+}
+void KeptBuffers::release_kv() {
+  std::lock_guard<std::mutex> lock(kept_mutex());
+  held.release_kv();
+}
+void KeptBuffers::release() {
+  std::lock_guard<std::mutex> lock(kept_mutex());
+  held.release();
+}
+bool KeptBuffers::release_all() {
+  std::lock_guard<std::mutex> lock(kept_mutex());
+  bool any = false;
+  for (KeptBuffers *k : kept_list()) {
+    any |= k->held.cache_bytes() || k->held.partials || k->held.counters;
+    k->held.release();
+  }
+  return any;
+}
+
+hipError_t device_alloc_bytes(void **p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && KeptBuffers::release_all()) e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
+  }
+  return e;
+}
+
 DevMatrix::~DevMatrix() {
   if (mem) hipFree(mem);
 }
@@ -143,7 +218,7 @@ int DevMatrix::create(int32_t dtype, int64_t rows, int64_t cols, hipStream_t st)
   // first word: finish()'s flag)
   const size_t sbytes = dtype == FMT_F32 || is_kquant(dtype) ? round256((size_t)rows * 4) : 0;
   const size_t total = vbytes + mbytes + hbytes + sbytes + 256;
-  hipError_t e = hipMalloc(&mem, total);
+  hipError_t e = device_alloc(&mem, total);
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc(%zu): %s", total, hipGetErrorString(e));
   bytes = total;
   e = hipMemsetAsync(mem, 0, total, st);  // row padding reads as zeros
@@ -194,7 +269,7 @@ int DevMatrix::place(int32_t dtype, int64_t rows, int64_t cols, const void *data
     for (int64_t r = 0; r < rows; r++)
       kquant_repack_row(dtype, (const uint8_t *)data + r * raw_row, cols, hv + r * vb, hm + r * mb, hh + r * hb);
     void *dev = nullptr;
-    e = hipMalloc(&dev, host.size());
+    e = device_alloc(&dev, host.size());
     if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc(%zu): %s", host.size(), hipGetErrorString(e));
     const uint8_t *dv = (const uint8_t *)dev, *dm = dv + rows * vb, *dh = dm + rows * mb;
     e = hipMemcpyAsync(dev, host.data(), host.size(), hipMemcpyHostToDevice, st);
@@ -214,7 +289,7 @@ int DevMatrix::place(int32_t dtype, int64_t rows, int64_t cols, const void *data
     return e == hipSuccess ? TINYOAI_OK : hip_fail(e, "weight upload");
   }
   void *raw = nullptr;
-  e = hipMalloc(&raw, nbytes);
+  e = device_alloc(&raw, nbytes);
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc(%llu): %s", (unsigned long long)nbytes, hipGetErrorString(e));
   e = hipMemcpyAsync(raw, data, nbytes, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) e = launch_repack(dtype, (const uint8_t *)raw, rows, cols, m, map, col0, st);
@@ -338,7 +413,7 @@ StableModel::~StableModel() {
 }
 
 int StableModel::alloc(void **p, size_t bytes) {
-  hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 256));
+  hipError_t e = device_alloc(p, std::max<size_t>(bytes, 256));
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
   buffers.push_back(*p);
   return TINYOAI_OK;
@@ -607,11 +682,11 @@ int StableModel::ensure_kv(int needed) {
   const size_t esz = kv_half ? 2 : 4;
   const size_t per_head = (size_t)dims.hd * esz;
   std::vector<KVDev> grown(cfg.num_hidden_layers);
-  if (!open_branches) drop_spare_kv();
+  if (!open_branches) spare.release_kv();
   for (auto &l : grown) {
     const size_t bytes = (size_t)dims.kv_heads * want * per_head;
-    hipError_t e = hipMalloc(&l.k, bytes);
-    if (e == hipSuccess) e = hipMalloc(&l.v, bytes);
+    hipError_t e = device_alloc(&l.k, bytes);
+    if (e == hipSuccess) e = device_alloc(&l.v, bytes);
     if (e != hipSuccess) {
       for (auto &g : grown) { if (g.k) hipFree(g.k); if (g.v) hipFree(g.v); }
       return fail(TINYOAI_ENOMEM, "KV allocation of %d positions: %s", want, hipGetErrorString(e));
@@ -1306,12 +1381,6 @@ void Branches::drop_graphs() {
   graphs.clear();
 }
 
-void StableModel::drop_spare_kv() {
-  for (void *p : spare.kv) hipFree(p);
-  spare.kv.clear();
-  spare.kv_bytes = 0;
-}
-
 void Branches::free_kv() {
   for (auto &l : kv) {
     if (l.k) hipFree(l.k);
@@ -1348,8 +1417,14 @@ int StableModel::score_rows(int n, bool *last) {
   return TINYOAI_OK;
 }
 
-void BranchBuffers::release() {
+void BranchBuffers::release_kv() {
   for (void *p : kv) hipFree(p);
+  kv.clear();
+  kv_bytes = 0;
+}
+
+void BranchBuffers::release() {
+  release_kv();
   if (partials) hipFree(partials);
   if (counters) hipFree(counters);
   if (logits_host) hipHostFree(logits_host);
@@ -1359,26 +1434,13 @@ void BranchBuffers::release() {
 Branches::~Branches() {
   const bool drained = m && m->stream && hipStreamSynchronize(m->stream) == hipSuccess;
   drop_graphs();
-  if (drained && !failed && kv_bytes * 2 * kv.size() <= BranchBuffers::kMost) {
-    // the model keeps them for its next session (one session's at most)
-    m->spare.release();
-    for (auto &l : kv) {
-      m->spare.kv.push_back(l.k);
-      m->spare.kv.push_back(l.v);
-    }
-    m->spare.kv_bytes = kv_bytes;
-    m->spare.partials = partials;
-    m->spare.partial_floats = partial_floats;
-    m->spare.counters = counters;
-    m->spare.counter_words = counter_words;
-    m->spare.logits_host = logits_host;
-    m->spare.logits_bytes = logits_bytes;
-  } else {
-    free_kv();
-    if (partials) hipFree(partials);
-    if (counters) hipFree(counters);
-    if (logits_host) hipHostFree(logits_host);
+  BranchBuffers b{{}, kv_bytes, partials, partial_floats, counters, counter_words, logits_host, logits_bytes};
+  for (auto &l : kv) {
+    b.kv.push_back(l.k);
+    b.kv.push_back(l.v);
   }
+  if (drained && !failed) m->spare.keep(std::move(b));
+  else b.release();
   if (last) hipFree(last);
   if (segs) hipFree(segs);
   if (m) m->open_branches--;
@@ -1395,23 +1457,20 @@ int Branches::grow(int need) {
   const size_t per = (size_t)s.kv_heads * count * row;  // bytes of one position of every branch
   std::vector<KVDev> grown(m->cfg.num_hidden_layers);
   size_t bytes = per * want;
-  if (m->spare.kv.size() == 2 * grown.size() && m->spare.kv_bytes >= bytes) {
+  const std::vector<void *> kept = m->spare.take_kv(2 * grown.size(), &bytes);
+  if (!kept.empty()) {
     // the previous session's buffers; with room for up to four times the
     // positions, while the caches stay within 2 GiB (a small session after a
     // large one addresses no more than it would have grown to)
-    bytes = m->spare.kv_bytes;
     if (4 * per * want <= (size_t)INT32_MAX) want = (int)std::min<size_t>({(size_t)max_len, bytes / per, (size_t)want * 4});
     for (size_t l = 0; l < grown.size(); l++) {
-      grown[l].k = m->spare.kv[2 * l];
-      grown[l].v = m->spare.kv[2 * l + 1];
+      grown[l].k = kept[2 * l];
+      grown[l].v = kept[2 * l + 1];
     }
-    m->spare.kv.clear();
-    m->spare.kv_bytes = 0;
   } else {
-    m->drop_spare_kv();
     for (auto &l : grown) {
-      hipError_t e = hipMalloc(&l.k, bytes);
-      if (e == hipSuccess) e = hipMalloc(&l.v, bytes);
+      hipError_t e = device_alloc(&l.k, bytes);
+      if (e == hipSuccess) e = device_alloc(&l.v, bytes);
       if (e != hipSuccess) {
         for (auto &g : grown) { if (g.k) hipFree(g.k); if (g.v) hipFree(g.v); }
         return fail(TINYOAI_ENOMEM, "branch KV of %d positions: %s", want, hipGetErrorString(e));
@@ -1455,7 +1514,7 @@ int Branches::ensure_partials(int nq, int splits) {
     if (partials) hipFree(partials);
     partials = nullptr;
     partial_floats = 0;
-    hipError_t e = hipMalloc(&partials, need * 4);
+    hipError_t e = device_alloc(&partials, need * 4);
     if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "branch attention scratch (%zu floats): %s", need, hipGetErrorString(e));
     partial_floats = need;
   }
@@ -1465,7 +1524,7 @@ int Branches::ensure_partials(int nq, int splits) {
     if (counters) hipFree(counters);
     counters = nullptr;
     counter_words = 0;
-    hipError_t e = hipMalloc(&counters, words * 4);
+    hipError_t e = device_alloc(&counters, words * 4);
     if (e == hipSuccess) e = hipMemsetAsync(counters, 0, words * 4, m->stream);
     if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "branch attention counters: %s", hipGetErrorString(e));
     counter_words = words;
@@ -1536,7 +1595,7 @@ int StableModel::branch_rows(Branches &b, const int32_t *ids, const int32_t *br,
     int longest = 0;
     if (use_flash) {
       if (!b.segs) {  // at most one run per row of a chunk
-        hipError_t e = hipMalloc(&b.segs, (size_t)chunk * 3 * sizeof(int));
+        hipError_t e = device_alloc(&b.segs, (size_t)chunk * 3 * sizeof(int));
         if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "branch run table: %s", hipGetErrorString(e));
       }
       // the previous chunk's table may still be in flight from the host copy
@@ -1743,7 +1802,7 @@ int StableModel::forward_logprobs(int prefix, const int32_t *tokens, const int32
     if (score_mem) hipFree(score_mem);
     score_mem = nullptr;
     score_bytes = 0;
-    hipError_t e = hipMalloc(&score_mem, bt + bc + bi + bl + bs);
+    hipError_t e = device_alloc(&score_mem, bt + bc + bi + bl + bs);
     if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "probability scratch: %s", hipGetErrorString(e));
     score_bytes = bt + bc + bi + bl + bs;
   }
@@ -1905,7 +1964,7 @@ int tinyoai_summarize_logits(const float *logits, int32_t rows, int32_t vocab, c
   const size_t ni = (size_t)rows * count * 4, np = (size_t)rows * count * 8, ns = logprob_scratch_bytes(count);
   auto r256 = [](size_t b) { return (b + 255) / 256 * 256; };
   char *mem = nullptr;
-  hipError_t e = hipMalloc(&mem, r256(nl) + r256(nt) + r256(nc) + r256(ni) + r256(np) + r256(ns));
+  hipError_t e = device_alloc(&mem, r256(nl) + r256(nt) + r256(nc) + r256(ni) + r256(np) + r256(ns));
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc: %s", hipGetErrorString(e));
   float *dl = (float *)mem;
   int *dt = (int *)(mem + r256(nl));
@@ -2015,16 +2074,17 @@ int tinyoai_stablelm_branches_open(tinyoai_model *m, int32_t prefix, int32_t cou
   b.count = count;
   b.max_len = max_len > 0 ? std::min(max_len, room) : room;
   b.len.assign(count, 0);
-  hipError_t e = hipMalloc(&b.last, (size_t)count * s.dims.d * 4);
+  hipError_t e = device_alloc(&b.last, (size_t)count * s.dims.d * 4);
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "branch rows: %s", hipGetErrorString(e));
   // scratch the previous session left (the counters zero, as each launch
   // leaves them)
-  b.partials = std::exchange(s.spare.partials, nullptr);
-  b.partial_floats = std::exchange(s.spare.partial_floats, 0);
-  b.counters = std::exchange(s.spare.counters, nullptr);
-  b.counter_words = std::exchange(s.spare.counter_words, 0);
-  b.logits_host = std::exchange(s.spare.logits_host, nullptr);
-  b.logits_bytes = std::exchange(s.spare.logits_bytes, 0);
+  const BranchBuffers kept = s.spare.take_scratch();
+  b.partials = kept.partials;
+  b.partial_floats = kept.partial_floats;
+  b.counters = kept.counters;
+  b.counter_words = kept.counter_words;
+  b.logits_host = kept.logits_host;
+  b.logits_bytes = kept.logits_bytes;
   *out = h.release();
   return TINYOAI_OK;
 }
@@ -2279,7 +2339,7 @@ int tinyoai_weight_read_values(tinyoai_weight *w, int64_t offset, int64_t n, flo
     return fail(TINYOAI_EINVAL, "invalid readValues span");
   if (n == 0) return TINYOAI_OK;
   float *dev;
-  hipError_t e = hipMalloc(&dev, (size_t)n * 4);
+  hipError_t e = device_alloc(&dev, (size_t)n * 4);
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc: %s", hipGetErrorString(e));
   e = launch_read_values(w->m.desc, offset, n, dev, w->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(out, dev, (size_t)n * 4, hipMemcpyDeviceToHost, w->stream);
@@ -2423,14 +2483,18 @@ int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, 
   hipGraph_t graph = nullptr;
   if ((e = hipStreamGetCaptureInfo_v2(st, &cap, &id, &graph, nullptr, nullptr)) != hipSuccess)
     return hip_fail(e, "hipStreamGetCaptureInfo");
-  auto alloc = [](size_t bytes) {
+  // (under capture nothing is given back to make room: hipFree waits for the device)
+  const bool capturing = cap != hipStreamCaptureStatusNone;
+  auto alloc = [capturing](size_t bytes) {
     RelaxedCapture relaxed;
     void *ptr = nullptr;
-    return hipMalloc(&ptr, bytes) == hipSuccess ? ptr : nullptr;
+    if ((capturing ? hipMalloc(&ptr, bytes) : device_alloc(&ptr, bytes)) == hipSuccess) return ptr;
+    (void)hipGetLastError();
+    return static_cast<void *>(nullptr);
   };
   std::lock_guard<std::mutex> lock(w->mu);
   ScratchPool::Lease lease;
-  if (cap != hipStreamCaptureStatusNone) {
+  if (capturing) {
     ScratchPool::Record *made = nullptr;
     lease.ptr = w->scratch.captured(id, st, p.bytes(), alloc, &made);
     hipUserObject_t owner = nullptr;
@@ -2553,8 +2617,8 @@ int tinyoai_weight_mul(tinyoai_weight *w, const float *x, int32_t n, float *out)
   if (!w || !x || !out || n <= 0) return fail(TINYOAI_EINVAL, "invalid product arguments");
   const Matrix &m = w->m.desc;
   float *dx = nullptr, *dout = nullptr;
-  hipError_t e = hipMalloc(&dx, (size_t)n * m.cols * 4);
-  if (e == hipSuccess) e = hipMalloc(&dout, (size_t)n * m.rows * 4);
+  hipError_t e = device_alloc(&dx, (size_t)n * m.cols * 4);
+  if (e == hipSuccess) e = device_alloc(&dout, (size_t)n * m.rows * 4);
   if (e != hipSuccess) {
     hipFree(dx);
     return fail(TINYOAI_ENOMEM, "hipMalloc: %s", hipGetErrorString(e));

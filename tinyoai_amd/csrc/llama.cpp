@@ -35,7 +35,7 @@ LlamaModel::~LlamaModel() {
 }
 
 int LlamaModel::alloc(void **p, size_t bytes) {
-  hipError_t e = hipMalloc(p, std::max<size_t>(bytes, 256));
+  hipError_t e = device_alloc(p, std::max<size_t>(bytes, 256));
   if (e != hipSuccess) return fail(TINYOAI_ENOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
   buffers.push_back(*p);
   return TINYOAI_OK;
@@ -136,7 +136,7 @@ int LlamaModel::init(const tinyoai_llama_config &c, const float *w, uint64_t n_f
   kv.resize(L);
   {
     const size_t per = (size_t)kv_dim * seq * 4;
-    if (hipMalloc(&kv_base, 2 * L * per + kTinyPad) != hipSuccess) return fail(TINYOAI_ENOMEM, "KV allocation");
+    if (device_alloc(&kv_base, 2 * L * per + kTinyPad) != hipSuccess) return fail(TINYOAI_ENOMEM, "KV allocation");
     for (int64_t l = 0; l < L; l++) {
       kv[l].k = (uint8_t *)kv_base + 2 * l * per;
       kv[l].v = (uint8_t *)kv_base + (2 * l + 1) * per;

@@ -88,14 +88,17 @@ struct Layer {
   LayerDev dev() const { return LayerDev{win, wout, ln_w, ln_b, win2, wout2}; }
 };
 
-// What a closed branch session leaves for the model's next one: its caches'
-// buffers (hipMalloc and hipFree of the 16-branch session's 4096-token
-// caches took 5 of its 21 ms), attention scratch and pinned logits. One
-// session's at most and no more than kMost bytes of caches; given back with
-// the model, at a reset, when the model's own cache grows, or when a session
-// needs larger ones.
+// hipMalloc. Where memory runs out, every model's kept buffers (KeptBuffers) are
+// given back and it is tried again; a failure leaves no error for
+// hipGetLastError, which the next launch would report.
+hipError_t device_alloc_bytes(void **p, size_t bytes);
+template <typename T>
+hipError_t device_alloc(T **p, size_t bytes) {
+  return device_alloc_bytes(reinterpret_cast<void **>(p), bytes);
+}
+
+// A branch session's caches, attention scratch and pinned logits.
 struct BranchBuffers {
-  static constexpr size_t kMost = (size_t)8 << 30;
   std::vector<void *> kv;  // per layer K, V: kv_bytes each
   size_t kv_bytes = 0;
   float *partials = nullptr;
@@ -104,7 +107,35 @@ struct BranchBuffers {
   size_t counter_words = 0;
   float *logits_host = nullptr;
   size_t logits_bytes = 0;
+  size_t cache_bytes() const { return kv_bytes * kv.size(); }
+  void release_kv();
   void release();
+};
+
+// What a closed branch session leaves for the model's next one (hipMalloc and
+// hipFree of the 16-branch session's 4096-token caches took 5 of its 21 ms):
+// one session's at most, and no more than kMost bytes of caches over all
+// models of the process. Given back with the model, at a reset, when the
+// model's own cache grows, when a session needs larger ones, and when any
+// allocation here finds the memory used up (on any thread: hence the lock).
+class KeptBuffers {
+ public:
+  static constexpr size_t kMost = (size_t)8 << 30;
+  KeptBuffers();
+  ~KeptBuffers();
+  KeptBuffers(const KeptBuffers &) = delete;
+  KeptBuffers &operator=(const KeptBuffers &) = delete;
+  void keep(BranchBuffers b);  // in the place of what is there
+  // `count` caches of at least `bytes`, their size in *bytes; or none, and
+  // what is there is given back.
+  std::vector<void *> take_kv(size_t count, size_t *bytes);
+  BranchBuffers take_scratch();  // all but the caches
+  void release_kv();
+  void release();
+  static bool release_all();  // whether there was anything
+
+ private:
+  BranchBuffers held;
 };
 
 // A StableLM resident on one GPU with its KV cache (stableState,
@@ -130,8 +161,7 @@ struct StableModel {
   // the model gate (branches.go:16-22).
   int open_branches = 0;
   int busy_with_branches() const;
-  BranchBuffers spare;
-  void drop_spare_kv();
+  KeptBuffers spare;
 
   // decode workspaces
   float *x = nullptr, *qbuf = nullptr, *mbuf = nullptr, *abuf = nullptr, *logits_dev = nullptr;
