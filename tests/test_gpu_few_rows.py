@@ -101,3 +101,36 @@ def test_f16_infinities_and_nan(n):
         assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
         assert np.array_equal(np.sign(got[np.isinf(want)]), np.sign(want[np.isinf(want)]))
         assert np.allclose(got[fin], want[fin], rtol=0, atol=1e-4)
+
+
+@pytest.mark.parametrize("mlp,attn,d,inter,hd,n", [
+    (W.F16, W.F16, 264, 172, 8, 65), (W.F16, W.F16, 264, 172, 8, 300), (W.F16, W.F16, 320, 1000, 80, 129),
+    (W.F32, W.F32, 264, 172, 8, 70), (W.F32, W.F32, 4104, 120, 8, 35), (W.Q4_K, W.Q6_K, 256, 768, 64, 33),
+    (W.Q4_K, W.Q6_K, 512, 256, 128, 300), (W.Q6_K, W.Q4_K, 256, 768, 64, 129), (W.Q5_K, W.Q5_K, 512, 768, 8, 257),
+    (W.Q6_K, W.Q6_K, 256, 512, 64, 70), (W.Q5_1, W.Q5_1, 320, 352, 80, 130), (W.Q4_K, W.F16, 512, 256, 64, 100)])
+def test_layers_of_odd_sizes(oracle, mlp, attn, d, inter, hd, n):
+    """Whole layers on the fp32-accurate tiles, alone and as pairs of products,
+    with LayerNorm rows as planes (and past 4096 columns without): widths that
+    are no multiple of a tile or a K step, against the oracle. Its fp32 sums
+    and these differ by at most 1e-6 of a layer's range (four times that here)."""
+    from tinyoai_amd import hip
+    heads = d // hd
+    config = W.validate_stablelm_config(dict(W.STABLELM_3B, hidden_size=d, intermediate_size=inter,
+                                             num_attention_heads=heads, num_key_value_heads=heads, num_hidden_layers=2,
+                                             vocab_size=300, max_position_embeddings=512))
+    if mlp == W.Q5_1:
+        rng = np.random.default_rng(n)
+        tensors = {name: t if t.rows == 1 else _weight(W.Q5_1, t.rows, t.cols, rng, oracle)[0]
+                   for name, t in W.synthetic_stablelm(config, W.F32, seed=d + n).items()}
+    else:
+        tensors = W.synthetic_stablelm(config, mlp, seed=d + n, attn_dtype=attn)
+    ids = np.random.default_rng(n).integers(0, 300, n).astype(np.int32)
+    oracle.set_threads(8)
+    ref = oracle.StableLM(config, tensors, capacity=512)
+    ref.trace(True)
+    f = hip.StableLMForwarder(config, tensors)
+    f.trace(True)
+    want, got = ref.prefill(ids, 0), f.forward(0, ids)
+    for a, b in zip(list(ref.trace_data()) + [want], list(f.trace_read()) + [got]):
+        assert np.max(np.abs(a - b)) <= 4e-6 * float(np.ptp(a)), (np.max(np.abs(a - b)), np.ptp(a))
+    f.close()

@@ -888,7 +888,7 @@ int StableModel::project(const Matrix &w, const float *x, int ldx, int n, float 
     const FewProduct p{w, x, ldx, y, ldy, ks, (int64_t)n * ldy};
     STAGE(ST_PREFILL_GEMM, launch_few_rows(&p, 1, n, stream), "projection");
   } else if (use_exact(w, n, room) ||
-             (!rowstream && w.fmt == FMT_F32 && use_wide && gemm_exact_supported(w, n, room))) {
+             (!rowstream && w.fmt == FMT_F32 && use_wide && gemm_exact_supported(w, n, room) && gemm_exact_faster(w, n))) {
     const ExactPlan plan = gemm_exact_plan(n, w, nullptr, room);
     if (splits) *splits = plan.ks;
     const int ld = gemm_exact_ld(w);
@@ -1025,7 +1025,7 @@ bool StableModel::use_few(const Matrix &w, int n) const {
 // rows than the few-row kernels (F16: 64, 5/6-bit formats: 32), in up to
 // max_splits K splits.
 bool StableModel::use_exact(const Matrix &w, int n, int max_splits) const {
-  return use_wide && n > 32 && !use_few(w, n) && gemm_exact_supported(w, n, max_splits);
+  return use_wide && n > 32 && !use_few(w, n) && gemm_exact_supported(w, n, max_splits) && gemm_exact_faster(w, n);
 }
 
 // Whether layer l's LayerNorm of n rows leaves as the fp16 planes of its
@@ -2395,7 +2395,7 @@ static Product plan_product(const Matrix &m, const float *x_dev, int n) {
     p.planes = round256(kq_rows_stage_bytes(m.cols, n));
     split(m.cols < 1024 ? 1 : kq_rows_splits(m, 32),
           kProductScratchBytes - std::min(p.planes + 256, kProductScratchBytes));
-  } else if (gemm_exact_supported(m, n, 32)) {
+  } else if (gemm_exact_supported(m, n, 32) && gemm_exact_faster(m, n)) {
     p.route = Route::exact;
     p.planes = round256((size_t)n * gemm_exact_ld(m) * 4) + round256((size_t)n * 4);
     // planes and partials together within the no-allocation array

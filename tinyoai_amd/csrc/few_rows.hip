@@ -360,8 +360,7 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
       }
     }
     __syncthreads();
-    // The segment's batches in rounds of kStages (past the range both
-    // operands are zeros). Batch kb + 1 goes to LDS, and its registers to
+    // The segment's batches in rounds of kStages. Batch kb + 1 goes to LDS, and its registers to
     // batch kb + 1 + kStages, while batch kb is computed.
     if (first) {
       put(ring[0], 0);
@@ -375,6 +374,10 @@ __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(2, 2))) void
     for (int kb = 0; kb < nb; kb += kStages) {
 #pragma unroll
       for (int j = 0; j < kStages; j++) {
+        // past the range: the rest of the round would multiply zeros (512 x 64
+        // Q8_0 of 2 rows 11.0 us with it, 7.9 without; 6912 x 2560 of 16 18.1,
+        // 17.2)
+        if (j > 0 && kb + j >= nb) break;
         put(ring[(j + 1) % kStages], (j + 1) & 1);
         issue(ring[(j + 1) % kStages], kb0 + kb + j + 1 + kStages);
 #pragma unroll

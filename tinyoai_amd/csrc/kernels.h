@@ -389,6 +389,15 @@ struct ExactProduct {
 constexpr int kExactRun = 16384;
 inline int gemm_exact_min_splits(const MatDesc &w) { return (w.cols + kExactRun - 1) / kExactRun; }
 bool gemm_exact_supported(const Matrix &w, int M, int max_splits = 1);
+// Whether they are faster than the vector-unit GEMM, whose time is about that
+// of its columns while the device takes all its tiles at once: from 96 columns
+// on (40 rows of 512 x 96 with Q5_1 18.1 us there, 16.5 here; x 64 12.9, 14.6;
+// F32, which that kernel reads as it is, from 128: x 96 14.2, 15.6; x 128
+// 18.1, 17.1), and with fewer from 2^21 outputs on (8192 x 64 F32: 256 rows
+// 14.2, 16.1; 512 rows 26.0, 17.8).
+inline bool gemm_exact_faster(const MatDesc &w, int M) {
+  return w.cols >= (w.fmt == FMT_F32 ? 128 : 96) || (int64_t)M * w.rows > 1 << 21;
+}
 bool gemm_exact_pair_supported(int a, int b);
 inline int gemm_exact_ld(const MatDesc &w) { return (w.cols + 31) / 32 * 32; }
 // The tiles of 256 rows (tall) or 128 and the K splits of one product or of
