@@ -1,6 +1,6 @@
 // Products of many rows with F16, F32 and 5/6-bit weights on the gfx950
-// matrix cores, as accurate as fp32 products: Y[M][N] = X[M][K] * W^T with
-// v_mfma_f32_32x32x16_f16.
+// matrix cores, no further from float64 than fp32 products with float64 totals
+// of 512 columns: Y[M][N] = X[M][K] * W^T with v_mfma_f32_32x32x16_f16.
 //
 // What bounds it: the matrix cores, at two (F16) or three products per
 // multiply-add. The vector-unit GEMM runs at about 2 TFLOP/s here, and the
@@ -10,12 +10,14 @@
 // Operands: X comes as fp16 hi + lo planes of rows scaled by a power of two
 // (Fp16Planes: 22 bits of a value down to 2^-16 of its row's largest; a row
 // that the planes do not serve is marked, and its outputs come from its fp32
-// values). F16 weights are used as stored. Other formats are decoded once per block to the fp32 values of
-// mat_value, scaled by the row's power of two (Matrix::rscale, from the
-// row's largest value) and split into fp16 hi + lo planes; the products are
-// hi hi + lo hi + hi lo. A K step of 32 columns is summed on the matrix
-// cores from zero and added to the fp32 totals, so a total rounds once per
-// step.
+// values). F16 weights are used as stored. Other formats are decoded once per
+// block to the fp32 values of mat_value, scaled by the row's power of two
+// (Matrix::rscale, from the row's largest value) and split into fp16 hi + lo
+// planes, which hold them as X's do (a matrix that they do not serve is marked
+// at its upload and does not come here); the products are hi hi + lo hi + hi
+// lo. A K step of 32 columns is summed on the matrix cores from zero and added
+// to the fp32 totals, so a total rounds once per step (kExactRun columns at
+// most).
 //
 // Tile: 128 * WM rows x 256 columns per block of eight waves (two per SIMD:
 // one's decoding runs beside the other's matrix products), a wave 32 * WM x
@@ -57,6 +59,7 @@ __global__ __launch_bounds__(256) void split_f16_kernel(const float *x, int64_t 
   };
   __shared__ int wave_most[4], wave_vote[4];
   int most = 0, vote = 0;
+  bool suspect = false;
   for (int i0 = 0; i0 < k; i0 += U * 1024) {
     load(i0);
 #pragma unroll
@@ -79,17 +82,30 @@ __global__ __launch_bounds__(256) void split_f16_kernel(const float *x, int64_t 
       if (i >= ldo) break;
       uint2 a, b;
       fp16_split4(v[u], s, a, b);
-      vote += (fp16_vote(v[u].x, most) + fp16_vote(v[u].y, most)) + (fp16_vote(v[u].z, most) + fp16_vote(v[u].w, most));
+      suspect |= fp16_suspect(v[u], most);
       *reinterpret_cast<uint2 *>(h + i) = a;
       *reinterpret_cast<uint2 *>(l + i) = b;
     }
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) vote += __shfl_xor(vote, o);
-  if ((threadIdx.x & 63) == 0) wave_vote[threadIdx.x >> 6] = vote;
+  const bool wave_suspect = __any(suspect);
+  if ((threadIdx.x & 63) == 0) wave_vote[threadIdx.x >> 6] = wave_suspect;
   __syncthreads();
-  if (threadIdx.x == 0)
-    unscale[row] = (wave_vote[0] + wave_vote[1]) + (wave_vote[2] + wave_vote[3]) > 0 ? -inverse : inverse;
+  bool marked = false;
+  if (wave_vote[0] | wave_vote[1] | wave_vote[2] | wave_vote[3]) {
+    for (int i0 = 0; i0 < k; i0 += U * 1024) {
+      load(i0);
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        vote += (fp16_vote(v[u].x, most) + fp16_vote(v[u].y, most)) + (fp16_vote(v[u].z, most) + fp16_vote(v[u].w, most));
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) vote += __shfl_xor(vote, o);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) wave_vote[threadIdx.x >> 6] = vote;
+    __syncthreads();
+    marked = (wave_vote[0] + wave_vote[1]) + (wave_vote[2] + wave_vote[3]) > 0;
+  }
+  if (threadIdx.x == 0) unscale[row] = marked ? -inverse : inverse;
 }
 
 template <int WF>
@@ -382,7 +398,7 @@ int tiles_of(const ExactArgs &g, int i) {
 // XCD x takes tiles [x * per, (x + 1) * per) of both products together, so one
 // XCD's blocks share weight tiles and none holds more than its share. (A run
 // per product gave seven XCDs 33 blocks for 32 CUs where the whole launch had
-// 252: 472 us instead of 258 for 700 rows of 21504 x 2560.)
+// 252: 472 us instead of 280 for 700 rows of 21504 x 2560.)
 __device__ __forceinline__ int tile_of(int per) { return ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3); }
 
 template <int WF, int WM>
@@ -454,6 +470,8 @@ hipError_t launch_split_f16(const float *x, int64_t ldx, int k, int rows, uint16
   return hipGetLastError();
 }
 
+// Planes of less than 1 GiB: the kernel's offsets are 32 bits, with kPast
+// (2^30) added to those past a range, and must stay past every plane.
 bool gemm_exact_supported(const Matrix &w, int M, int max_splits) {
   constexpr int64_t kGiB = int64_t(1) << 30;
   const bool fmt = w.fmt == FMT_F16 || ((w.fmt == FMT_F32 || is_kquant(w.fmt)) && w.rscale);
@@ -462,6 +480,9 @@ bool gemm_exact_supported(const Matrix &w, int M, int max_splits) {
          (int64_t)w.rows * w.mstride < kGiB && (int64_t)M * gemm_exact_ld(w) * 2 < kGiB;
 }
 
+// (each pair is two more kernels to compile: there are those that the K-quant
+// mix, F16 and Q5_K models form; others, a whole model of Q4_K or Q6_K among
+// them, run as two launches, and what a pair would give there is not measured)
 bool gemm_exact_pair_supported(int a, int b) {
   return (a == FMT_Q6_K && b == FMT_Q4_K) || (a == FMT_Q4_K && b == FMT_Q6_K) || (a == b && (a == FMT_Q5_K || a == FMT_F16));
 }

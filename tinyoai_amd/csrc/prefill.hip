@@ -340,20 +340,31 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(float *x, const float *p
   mag = max(max(most[0], most[1]), max(most[2], most[3]));
   float down;
   const float up = fp16_scale(mag, down);
-  int vote = 0;
+  bool suspect = false;
 #pragma unroll
   for (int g = 0; g < kNormG; g++) {
     if (at(g) >= fp.ld) continue;
     uint2 hi, lo;
     fp16_split4(v[g], up, hi, lo);
-    vote += (fp16_vote(v[g].x, mag) + fp16_vote(v[g].y, mag)) + (fp16_vote(v[g].z, mag) + fp16_vote(v[g].w, mag));
+    suspect |= fp16_suspect(v[g], mag);
     *reinterpret_cast<uint2 *>(fp.hi + row * fp.ld + at(g)) = hi;
     *reinterpret_cast<uint2 *>(fp.lo + row * fp.ld + at(g)) = lo;
   }
-  for (int o = 32; o > 0; o >>= 1) vote += __shfl_xor(vote, o);
-  if ((tid & 63) == 0) votes[tid >> 6] = vote;
+  const bool wave_suspect = __any(suspect);
+  if ((tid & 63) == 0) votes[tid >> 6] = wave_suspect;
   __syncthreads();
-  const bool marked = (votes[0] + votes[1]) + (votes[2] + votes[3]) > 0;
+  bool marked = false;
+  if (votes[0] | votes[1] | votes[2] | votes[3]) {  // uniform
+    int vote = 0;
+#pragma unroll
+    for (int g = 0; g < kNormG; g++)  // (zeros past the row)
+      vote += (fp16_vote(v[g].x, mag) + fp16_vote(v[g].y, mag)) + (fp16_vote(v[g].z, mag) + fp16_vote(v[g].w, mag));
+    for (int o = 32; o > 0; o >>= 1) vote += __shfl_xor(vote, o);
+    __syncthreads();
+    if ((tid & 63) == 0) votes[tid >> 6] = vote;
+    __syncthreads();
+    marked = (votes[0] + votes[1]) + (votes[2] + votes[3]) > 0;
+  }
   if (tid == 0) fp.unscale[row] = marked ? -down : down;
   if (!marked) return;
 #pragma unroll
