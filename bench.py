@@ -384,7 +384,7 @@ def main():
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU; --gpus {args.gpus} is not supported (the path would shard by "
-              f"attention head / MLP column with one all-reduce per layer; see DESIGN.md).", file=sys.stderr)
+              f"attention head / MLP column with one all-reduce per layer).", file=sys.stderr)
         sys.exit(2)
 
     if args.workload in ("branches", "long_context"):

@@ -8,7 +8,7 @@ into the decode_in launch (up to 1800 positions) and the separate 4-step
 launch beyond, the matrix-core prefill, and the branch passes (the shared
 prefix on the matrix cores, each branch's suffix split-K).
 
-Tolerances are north_star's: 1e-3 of the range for fp32-KV paths, 2e-2
+Tolerances: 1e-3 of the range for fp32-KV paths, 2e-2
 where the KV cache is fp16. The GPU is fed the oracle's greedy tokens, so
 every step compares the same positions; the argmax must agree at each.
 """

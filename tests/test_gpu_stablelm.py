@@ -463,7 +463,7 @@ def test_mixed_format_layers_against_oracle(hip, oracle, mlp, attn):
     keeps its sections as matrices of their own. StableLM-3B layer shapes,
     two layers, fp16 KV, a 300-token prompt (prefill in one chunk) and 8
     decode tokens: logits within 1e-3 of their range of the oracle's (2e-2
-    where a section is BF16: north_star's bound for the bf16 paths, which
+    where a section is BF16: the bound of the bf16 paths, which
     the two-plane products meet by far), identical greedy ids."""
     config = W.validate_stablelm_config(dict(W.STABLELM_3B, num_hidden_layers=2, max_position_embeddings=512))
     tensors = W.synthetic_stablelm(config, mlp, seed=23, attn_dtype=attn, head_dtype=attn)

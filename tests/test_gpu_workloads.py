@@ -17,7 +17,7 @@ The oracle needs minutes for these, so its results are committed fixtures
 the weights and prompts are rebuilt here from those seeds. A logits vector
 is compared through its summary: the values at a fixed sample of 253 ids
 and the 16 largest entries, against the oracle's range (max - min).
-Tolerances are north_star's: 1e-3 of the range for fp32 paths, 2e-2 where
+Tolerances: 1e-3 of the range for fp32 paths, 2e-2 where
 the KV cache is fp16. Greedy ids must be identical; the GPU is fed the
 oracle's tokens (teacher forcing), so every step is compared at the same
 positions even if an id ever differed.

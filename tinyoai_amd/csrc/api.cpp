@@ -872,10 +872,13 @@ static void wide_shape(int n, int N, int *mf, int *nf) {
 }
 
 // y[n][ldy] = x[n][ldx] * W^T: on the matrix cores when the format allows
-// (activations split into bf16 hi/lo planes first), else the vector-unit
-// GEMM. Without rowstream every output row depends only on its own input
-// row, whatever the chunk size (a prefix reused from the cache gives the
-// same results).
+// (activations split into 16-bit planes first), else the vector-unit GEMM.
+// Which kernel runs, and in how many K splits, depends on n: a prompt taken in
+// other chunks (a prefix reused from the cache among them) has the same values
+// to the kernels' accuracy, not to the bit. Without splits, an output row
+// depends on its own input row alone within the sizes of one kernel: few rows
+// (a few-row F16 or Q8_0 row's scales follow the segment that n gives), and
+// more.
 int StableModel::project(const Matrix &w, const float *x, int ldx, int n, float *y, int ldy, int *splits,
                          bool rowstream, int max_splits, bool *staged) {
   if (splits) *splits = 1;
@@ -2352,7 +2355,7 @@ int tinyoai_weight_read_values(tinyoai_weight *w, int64_t offset, int64_t n, flo
 
 // How a product of n rows runs, and the scratch it needs: operand planes, then
 // partial outputs of `ks` K splits (summed in order). A rule of the shape and
-// of x's alignment alone (the partials within kProductPartialBytes), so the
+// of x's alignment (the partials within kProductPartialBytes), so the
 // allocating and the no-allocation entry points sum alike, captured or not.
 //   one row: the row-streaming matvec;
 //   F16, BF16, Q8_0 up to 64 rows: the few-row kernel;
@@ -2540,7 +2543,9 @@ int tinyoai_weight_mul_device(tinyoai_weight *w, const float *x_dev, int32_t n, 
 // device address of each GPU's copy comes from hipGetSymbolAddress (once
 // per device, with that device current) and only that address is used.
 constexpr size_t kScratchValues = (size_t)4 << 20;  // activation values per call (n * cols)
-// bf16 hi and lo planes (16 MiB), then the K-split partials (32 MiB)
+// operand planes (two of 16 bits: 16 MiB; fp16 planes of rows that are no
+// multiple of 32 columns up to 24), then the K-split partials in what is left,
+// at most 32 MiB
 static __device__ __align__(256) uint16_t scratch[kProductScratchBytes / 2];
 static_assert(2 * kScratchValues * 2 + kProductPartialBytes <= kProductScratchBytes, "planes, then partials");
 

@@ -22,11 +22,11 @@
 // this does not serve is marked, and its outputs come from its fp32 values
 // (plain_rows): where most of the groups of four values that are not all zero
 // lie below 2^-16 of the segment's largest (Q8_0: 2^-22, since two bf16 planes
-// would carry 16 bits of every value). Q8_0
-// quants are exact in fp16, each quant block's product is formed unscaled
-// and added as acc += d * block. BF16 weights take bf16 hi + lo planes (16
-// bits, as the wide tiles). Each segment's sums (F16: every 1024 columns') are
-// unscaled and added to fp32 totals.
+// would carry 16 bits of every value). Q8_0 quants are exact in fp16, each
+// quant block's product is formed unscaled and added as acc += d * block. BF16
+// weights take bf16 hi + lo planes (16 bits, as the wide tiles). Each
+// segment's sums (F16: every 1024 columns') are unscaled and added to fp32
+// totals.
 //
 // K ranges (splits) write partial outputs, split s at y + s * split_stride,
 // which the consumer sums in order.
@@ -447,7 +447,7 @@ double value_bytes(int fmt) { return fmt == FMT_Q8_0 ? 34.0 / 32 : 2.0; }
 int row_blocks(const MatDesc &w) { return (w.rows + kBlockRows - 1) / kBlockRows; }
 
 // Microseconds of a launch of `blocks` blocks whose longest covers `kb`
-// batches, and of the partial outputs (written and read): about 20 GB/s of
+// batches, and of the partial outputs (written and read): about 20 KB of
 // matrix per CU and microsecond, 3 us before a block's stream is going.
 double launch_cost(int blocks, int kb, int fmt, double partial_bytes) {
   const double batch = kBlockRows * batch_cols(fmt) * value_bytes(fmt) / 20e3;

@@ -198,8 +198,9 @@ __global__ __launch_bounds__(kT) void logprob_kernel(const float *logits, int64_
 // The count-th largest of the maxima of 64 groups of threads is a lower bound
 // of the count-th largest value (count groups hold one at least as large), so
 // the values from it on are the candidates: few more than count unless many
-// are equal (about 300 for count 64). Past kCand of them, the threshold and then the highest id taken
-// among its equals are found by bisection over the registers.
+// are equal (about 300 for count 64). Past kCand of them, the threshold and
+// then the highest id taken among its equals are found by bisection over the
+// registers.
 constexpr int kFew = kT / 16, kCand = 1024;  // at most as many entries as groups
 
 template <int J>
@@ -351,6 +352,8 @@ hipError_t launch_logprobs(const float *logits, int64_t ld, int rows, int vocab,
                            double *chosen, int *top_ids, double *top_lp, void *scratch, hipStream_t st) {
   if (rows < 1 || vocab < 1 || count < 1 || count > vocab || ld < vocab || !scratch) return hipErrorInvalidValue;
   int *bad = reinterpret_cast<int *>(scratch);
+  // Rows in registers up to 65536 values: 64 of the 128 registers that a thread
+  // of 1024 may have (twice that would spill); longer rows are read again.
   if (count <= kFew && vocab <= 4096 * 4) {
     hipLaunchKernelGGL(logprob_few_kernel<4>, dim3(rows), dim3(kT), 0, st, logits, ld, vocab, targets, count, chosen,
                        top_ids, top_lp, bad);

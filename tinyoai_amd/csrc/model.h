@@ -234,8 +234,8 @@ struct StableModel {
   // rowstream (branch steps), a product of at most 32 rows with a 5/6-bit
   // matrix runs on the matrix cores as one few-row product, and of at most
   // kRowStreamMax rows in another format without a matrix-core path as one
-  // row-streaming matvec per row; otherwise every chunk size takes the
-  // same arithmetic.
+  // row-streaming matvec per row. Which kernel a product takes, and so the
+  // order of its sums, depends on n.
   // A null x (fp32-accurate products only): its fp16 planes are in XH, XL, XU
   // and its marked rows in H.
   // staged (few-row 5/6-bit products): in, the workspace already holds
