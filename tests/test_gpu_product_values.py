@@ -287,3 +287,42 @@ def test_large_values_in_one_row(fmt, cols):
         want, mag = y64 @ dense.T, np.abs(y64) @ np.abs(dense).T
         assert np.all(np.abs(got - want) <= (cols / 64 + 64) * 2.0 ** -24 * mag)
     w.close()
+
+
+@pytest.mark.parametrize("fmt,n", [(W.F16, 20), (W.F16, 50), (W.F16, 100), (W.Q8_0, 9), (W.Q8_0, 40), (W.Q6_K, 100)])
+def test_down_product_with_an_outlier(fmt, n):
+    """A SiLU-gate output of up to 1e8 beside ordinary ones, where the down
+    matrix is zero: the down product, the second of its launch with the o
+    product, takes the marked rows from their fp32 values, and the logits are
+    those of the same model with an ordinary value there (to about the error
+    of its fp32 sums, 1e-6 of their range)."""
+    from tinyoai_amd import hip
+    d, inter = 512, 768
+    config = W.validate_stablelm_config(dict(W.STABLELM_3B, hidden_size=d, intermediate_size=inter, num_attention_heads=8,
+                                             num_key_value_heads=8, num_hidden_layers=2, vocab_size=256,
+                                             max_position_embeddings=512))
+    ids = np.random.default_rng(n).integers(0, 256, n).astype(np.int32)
+    got = []
+    for huge in (False, True):
+        tensors = W.synthetic_stablelm(config, fmt, seed=6)
+        for name, t in tensors.items():
+            if name.endswith("down_proj.weight"):  # column 9 of every row
+                if fmt == W.F16:
+                    t.data.view(np.float16).reshape(d, inter)[:, 9] = 0
+                elif fmt == W.Q8_0:
+                    t.data.reshape(d, inter // 32, 34)[:, 0, 2 + 9] = 0
+                else:
+                    b = t.data.reshape(d, inter // 256, 210)
+                    b[:, 0, 9] &= 0xF0
+                    b[:, 0, 137] = (b[:, 0, 137] & 0xFC) | 2
+            elif huge and name.endswith("up_proj.weight"):  # row 9
+                if fmt == W.F16:
+                    t.data.view(np.float16).reshape(inter, d)[9] *= np.float16(30000)
+                else:
+                    size, at = (34, 0) if fmt == W.Q8_0 else (210, 208)
+                    t.data.reshape(inter, -1, size)[9, :, at:at + 2] = np.float16(30000).reshape(1).view(np.uint8)
+        f = hip.StableLMForwarder(config, tensors)
+        got.append(f.forward(0, ids))
+        f.close()
+    assert np.all(np.isfinite(got[0])) and np.std(got[0]) > 0
+    assert np.max(np.abs(got[0] - got[1])) <= 4e-6 * np.ptp(got[0]), np.max(np.abs(got[0] - got[1])) / np.ptp(got[0])

@@ -282,3 +282,40 @@ def test_products_in_flight_on_many_streams(dtype, n):
             rt.hipStreamDestroy(st)
         w.close()
         buf.close()
+
+
+@pytest.mark.parametrize("dtype,n", [(W.F16, 80), (W.F32, 40), (W.Q4_K, 9), (W.Q8_0, 20)])
+def test_captured_no_alloc_product_matches_the_eager_one(dtype, n):
+    from tinyoai_amd import hip
+    rng = np.random.default_rng(n)
+    rows, cols = 300, 1280
+    t = {W.F32: W.synthetic_f32, W.Q8_0: W.synthetic_q8_0}.get(dtype)
+    if dtype == W.F16:
+        v = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float16)
+        t = W.Tensor(W.F16, rows, cols, v.reshape(-1).view(np.uint8))
+    else:
+        t = t(rows, cols, rng) if t else W.synthetic_kquant(dtype, rows, cols, rng)
+    buf = DeviceBuffers()
+    rt, w = buf.rt, hip.Weight(t)
+    st, graph, ex = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    try:
+        x = buf.upload(rng.standard_normal((n, cols)).astype(np.float32))
+        y, y2 = buf.upload(np.zeros((n, rows), np.float32)), buf.alloc(n * rows * 4)
+        assert rt.hipStreamCreateWithFlags(C.byref(st), 1) == 0
+        w.mul_device_noalloc(x, n, y2, st.value)
+        want = buf.download(y2, (n, rows))
+        assert rt.hipStreamBeginCapture(st, 0) == 0
+        w.mul_device_noalloc(x, n, y, st.value)
+        assert rt.hipStreamEndCapture(st, C.byref(graph)) == 0
+        assert rt.hipGraphInstantiate(C.byref(ex), graph, None, None, C.c_size_t(0)) == 0
+        for _ in range(3):
+            assert rt.hipGraphLaunch(ex, st) == 0 and rt.hipStreamSynchronize(st) == 0
+            assert np.array_equal(buf.download(y, (n, rows)), want)
+            w.mul_device(x, n, y2)
+            assert np.array_equal(buf.download(y2, (n, rows)), want)
+    finally:
+        for handle, destroy in ((ex, rt.hipGraphExecDestroy), (graph, rt.hipGraphDestroy), (st, rt.hipStreamDestroy)):
+            if handle.value:
+                destroy(handle)
+        w.close()
+        buf.close()
